@@ -161,18 +161,29 @@ __device__ void setup_point(const SetupArgs& a, const DrawDesc& d, uint32_t di, 
 }
 
 // Pixel box that holds every pixel whose centre can pass the four edge
-// tests of a line quad with corners c[4] (NDC), or false when the quad is
-// too degenerate for the bound below (the caller then scans the viewport,
-// as the reference does for every line).
+// tests of a line quad with corners c[4] (NDC; the edges go c0 -> c1 -> c3 ->
+// c2 -> c0), or false when the quad is too degenerate for the bound below
+// (the caller then scans the viewport, as the reference does for every line).
 //
-// The bound: in pixel space (x + 0.5 = (ndc + 1) * extent / 2) let the quad
-// have sides of at least 0.5 px and an angle with sine >= 0.1, corners
-// within 4 of the origin in NDC and viewport extents <= 32768.  A pixel
-// centre 3.5 px or more outside the corners' box is then at least
-// 3.5 * sin(angle / 2) >= 0.16 px outside some edge, i.e. >= 9.6e-6 NDC.
-// The float evaluation (x - ax) * dy - (y - ay) * dx of that edge errs by
-// at most 8 * 2^-24 * (|x - ax| + |y - ay|) * |d| <= 4.8e-6 * |d|, so the
-// edge value stays negative and the pixel fails.
+// The bound: in pixel space (x + 0.5 = (ndc + 1) * extent / 2) let the quad be
+// convex with the orientation that makes all edge functions positive inside,
+// every corner's sine at least 0.1, every side at least 2^-10 px, corners
+// within 4 of the origin in NDC and viewport extents <= 32768.  The nearest
+// point of the quad to a pixel centre 3.5 px or more outside the corners' box
+// lies on a side, or at a corner of angle t between whose two side lines the
+// centre is at least 3.5 * sin(t / 2) >= 3.5 * 0.05 = 0.175 px outside one.
+// The float evaluation (x - ax) * dy - (y - ay) * dx of that side's edge errs
+// by at most 8u (|x - ax||dy| + |y - ay||dx|), u = 2^-24, which in pixels is
+// at most 8u * |p - a| <= 8u * 1.2e5 = 0.06 px of distance from the side's
+// line, whatever the side's length (sides of 2^-10 px keep the products
+// normal), and the rounded pixel centre is within 0.01 px: the edge value
+// stays negative and the pixel fails.
+//
+// The sides' lengths do not enter, so the thin quads of lines whose clip w
+// varies (normalize(p1 - p0) runs over all four components) get their box:
+// 6,001 lines of about 40 px over 1920x1080 with w in [0.5, 2], half of whose
+// quads are below half a pixel wide, took 20 ms of raster time while only
+// quads with sides of half a pixel had one.
 __device__ bool line_box(const DrawDesc& d, const float* c[4], int32_t* x0, int32_t* y0, int32_t* x1, int32_t* y1)
 {
     if (!(d.vp_w <= 32768.0f) || !(d.vp_h <= 32768.0f)) return false;
@@ -180,18 +191,22 @@ __device__ bool line_box(const DrawDesc& d, const float* c[4], int32_t* x0, int3
     for (int k = 0; k < 4; k++)
         if (!(fabsf(c[k][0]) <= 4.0f) || !(fabsf(c[k][1]) <= 4.0f)) return false;
     const double sx = 0.5 * (double)d.vp_w, sy = 0.5 * (double)d.vp_h;
-    // c = {p00, p01, p10, p11}: long side p00 -> p10, short side p00 -> p01
-    const double ux = ((double)c[2][0] - (double)c[0][0]) * sx, uy = ((double)c[2][1] - (double)c[0][1]) * sy;
-    const double vx = ((double)c[1][0] - (double)c[0][0]) * sx, vy = ((double)c[1][1] - (double)c[0][1]) * sy;
-    const double lu = sqrt(ux * ux + uy * uy), lv = sqrt(vx * vx + vy * vy);
-    if (!(lu >= 0.5) || !(lv >= 0.5) || !(fabs(ux * vy - uy * vx) >= 0.1 * lu * lv)) return false;
+    const int loop[4] = {0, 1, 3, 2};
     double mnx = 1e30, mxx = -1e30, mny = 1e30, mxy = -1e30;
+    bool fits = true;
 #pragma unroll
     for (int k = 0; k < 4; k++) {
-        const double px = ((double)c[k][0] + 1.0) * sx, py = ((double)c[k][1] + 1.0) * sy;
+        const float *a = c[loop[k]], *b = c[loop[(k + 1) & 3]], *n = c[loop[(k + 2) & 3]];
+        const double ux = ((double)b[0] - (double)a[0]) * sx, uy = ((double)b[1] - (double)a[1]) * sy;
+        const double vx = ((double)n[0] - (double)b[0]) * sx, vy = ((double)n[1] - (double)b[1]) * sy;
+        const double lu2 = ux * ux + uy * uy, lv2 = vx * vx + vy * vy;
+        const double e = vx * uy - vy * ux;   // the edge function of a -> b at n: positive for the drawn orientation
+        fits = fits && lu2 >= 0x1p-20 && e > 0.0 && e * e >= 0.01 * lu2 * lv2;
+        const double px = ((double)a[0] + 1.0) * sx, py = ((double)a[1] + 1.0) * sy;
         mnx = fmin(mnx, px); mxx = fmax(mxx, px);
         mny = fmin(mny, py); mxy = fmax(mxy, py);
     }
+    if (!fits) return false;
     *x0 = max(*x0, (int32_t)floor(mnx) - 4);
     *y0 = max(*y0, (int32_t)floor(mny) - 4);
     *x1 = min(*x1, (int32_t)floor(mxx) + 5);
@@ -460,6 +475,7 @@ __global__ __launch_bounds__(kScanThreads) void scan_down_kernel(const uint32_t*
 
 struct EmitArgs {
     const TriSetup* recs;
+    const LineExt* ext;           // per-primitive line extension (launches with lines)
     const uint32_t* counts;
     const uint32_t* offsets;
     const DrawDesc* draws;
@@ -521,11 +537,11 @@ __device__ __forceinline__ void centre_range(int p0, int p1, float half, float& 
     hi = fmaxf(a + ea, b + eb);
 }
 
-// pair_blocks less, for a triangle, the quarters where it covers no pixel
-// (points and lines keep their box's quarters).  box is relative to the
+// pair_blocks less, for a triangle or a line, the quarters where it covers
+// no pixel (points keep their box's quarters).  box is relative to the
 // primitive's first tile, whose pixel origin is (ox, oy); e holds the
-// record's edges (bytes 0-47: ax[3], ay[3], dy[3], dx[3]) and vp the draw's
-// (vp_w, vp_h, half_x, half_y).
+// record's edges (bytes 0-47: ax[3], ay[3], dy[3], dx[3]), l a line's fourth
+// edge (ax, ay, dy, dx) and vp the draw's (vp_w, vp_h, half_x, half_y).
 //
 // The raster kernel's edge value at a pixel centre (x, y) is
 // fl(A(x) - B(y)), A(x) = fl(fl(x - a.x) * dy), B(y) = fl(fl(y - a.y) * dx),
@@ -537,15 +553,17 @@ __device__ __forceinline__ void centre_range(int p0, int p1, float half, float& 
 // pixel's value exceeds A(dy > 0 ? xhi : xlo) - B(dx < 0 ? yhi : ylo); when
 // that is negative every pixel's is (a pixel's NaN needs A = B = +-inf,
 // which makes the bound +inf or NaN) and the quarter is dropped.  NaN is
-// not < 0, and non-finite terms keep every quarter.  Each edge's bound is
+// not < 0, and non-finite terms keep every quarter.  A line's pixel needs all
+// four edge values >= 0, so the same bound drops its quarters: without it the
+// raster kernel visits every block of a line's box for the few it crosses.  Each edge's bound is
 // computed once per quarter column and row, from an interval holding the
 // column's (row's) centres: centre_range's, or for viewport extents below
 // 0.5 in magnitude the exact centres of its two ends.
-__device__ __forceinline__ uint32_t pair_blocks_covered(int tile_shift, int4 box, uint32_t col, uint32_t row, bool triangle,
-                                                        const float4 e[3], float4 vp, int ox, int oy)
+__device__ __forceinline__ uint32_t pair_blocks_covered(int tile_shift, int4 box, uint32_t col, uint32_t row, uint32_t kind,
+                                                        const float4 e[3], float4 l, float4 vp, int ox, int oy)
 {
     const uint32_t m = pair_blocks(tile_shift, box, col, row);
-    if (m == 0u || !triangle) return m;
+    if (m == 0u || (kind & kPrimPoint)) return m;
     const int half = 1 << (tile_shift - 1);
     const int X = (int)col << tile_shift, Y = (int)row << tile_shift;
     const uint32_t bits = m >> kPairBlockShift;
@@ -581,6 +599,16 @@ __device__ __forceinline__ uint32_t pair_blocks_covered(int tile_shift, int4 box
             range(oy + max(Y + half * h, box.y), oy + min(Y + half * h + half, box.w) - 1, vp.y, vp.w, ylo[h], yhi[h]);
     }
     if (!finite) return m;
+    uint32_t keep = bits;
+    if (kind & kPrimLine) {
+        if (!(__builtin_isfinite(l.x) && __builtin_isfinite(l.y) && __builtin_isfinite(l.z) && __builtin_isfinite(l.w))) return m;
+#pragma unroll
+        for (int b = 0; b < 4; b++) {
+            const float a = ((l.z > 0.0f ? xhi[b & 1] : xlo[b & 1]) - l.x) * l.z;
+            const float c = ((l.w < 0.0f ? yhi[b >> 1] : ylo[b >> 1]) - l.y) * l.w;
+            if (a - c < 0.0f) keep &= ~(1u << b);
+        }
+    }
     float amax[3][2], bmin[3][2];
 #pragma unroll
     for (int i = 0; i < 3; i++)
@@ -589,15 +617,14 @@ __device__ __forceinline__ uint32_t pair_blocks_covered(int tile_shift, int4 box
             amax[i][h] = ((dy[i] > 0.0f ? xhi[h] : xlo[h]) - ax[i]) * dy[i];
             bmin[i][h] = ((dx[i] < 0.0f ? yhi[h] : ylo[h]) - ay[i]) * dx[i];
         }
-    uint32_t keep = 0u;
 #pragma unroll
     for (int b = 0; b < 4; b++) {
-        bool cover = ((bits >> b) & 1u) != 0u;
+        bool cover = true;
 #pragma unroll
         for (int i = 0; i < 3; i++) cover = cover & !(amax[i][b & 1] - bmin[i][b >> 1] < 0.0f);
-        if (cover) keep |= 1u << (kPairBlockShift + b);
+        if (!cover) keep &= ~(1u << b);
     }
-    return keep;
+    return keep << kPairBlockShift;
 }
 
 // Writes the (tile, primitive) pairs of every primitive at its scanned
@@ -612,12 +639,12 @@ __device__ __forceinline__ uint32_t pair_blocks_covered(int tile_shift, int4 box
 // primitive go in row-major order of its tile rectangle.
 __global__ __launch_bounds__(256) void emit_kernel(EmitArgs a)
 {
-    constexpr uint32_t kNoEdgeTest = 0x80000000u;   // s_w flag: a point or line keeps its box's quarters
+    constexpr int kKindShift = 29;    // s_w: the primitive's kind (kPrimPoint, kPrimLine) above the columns
     __shared__ uint32_t s_tmp[4];
     __shared__ uint32_t s_off[257];   // exclusive scan of the kept pair counts
     __shared__ uint32_t s_dst[256];   // output offset of each primitive's first pair
     __shared__ uint32_t s_key[256];   // global tile index of each primitive's first tile
-    __shared__ uint32_t s_w[256];     // tile columns of each primitive's rectangle, | kNoEdgeTest
+    __shared__ uint32_t s_w[256];     // tile columns of each primitive's rectangle, | kind << kKindShift
     __shared__ uint32_t s_tx[256];    // tile columns of each primitive's target
     __shared__ int4 s_box[256];       // pixel box of each primitive, relative to its first tile
     __shared__ int2 s_org[256];       // pixel origin of each primitive's first tile
@@ -642,7 +669,7 @@ __global__ __launch_bounds__(256) void emit_kernel(EmitArgs a)
             const uint32_t ty0 = (uint32_t)r.y0 >> sh;
             s_dst[threadIdx.x] = a.offsets[gp];
             s_key[threadIdx.x] = t.tile_base + ty0 * t.tiles_x + tx0;
-            s_w[threadIdx.x] = (tx1 - tx0 + 1) | ((r.flags & (kPrimPoint | kPrimLine)) ? kNoEdgeTest : 0u);
+            s_w[threadIdx.x] = (tx1 - tx0 + 1) | ((r.flags & (kPrimPoint | kPrimLine)) << kKindShift);
             s_tx[threadIdx.x] = t.tiles_x;
             const int ox = (int)(tx0 << sh), oy = (int)(ty0 << sh);
             s_box[threadIdx.x] = make_int4(r.x0 - ox, r.y0 - oy, r.x1 - ox, r.y1 - oy);
@@ -665,7 +692,7 @@ __global__ __launch_bounds__(256) void emit_kernel(EmitArgs a)
                 if (s_off[lo + step] <= j) lo += step;
             const uint32_t k = j - s_off[lo];
             const uint32_t wl = s_w[lo];
-            const uint32_t w = wl & ~kNoEdgeTest;
+            const uint32_t w = wl & ((1u << kKindShift) - 1u), kind = wl >> kKindShift;
             // row = k / w: k < kEmitBig = 2048 and w <= 2048, so (k + 1/2) / w
             // is at least 1/(2w) from an integer while the product with
             // v_rcp_f32's reciprocal (1 ulp) errs by under 1.5 * 2^-23 * 2049 / w
@@ -676,8 +703,10 @@ __global__ __launch_bounds__(256) void emit_kernel(EmitArgs a)
                 a.keys[out] = s_key[lo] + row * s_tx[lo] + col;
                 const int2 org = s_org[lo];
                 const float4 e[3] = {s_edge[lo][0], s_edge[lo][1], s_edge[lo][2]};
+                float4 l = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                if (kind & kPrimLine) l = *(const float4*)&a.ext[blk * 256u + lo];
                 a.vals[out] = (blk * 256u + lo) |
-                              pair_blocks_covered(a.tile_shift, s_box[lo], col, row, (wl & kNoEdgeTest) == 0u, e, s_vp[lo], org.x, org.y);
+                              pair_blocks_covered(a.tile_shift, s_box[lo], col, row, kind, e, l, s_vp[lo], org.x, org.y);
             }
         }
         __syncthreads();
@@ -705,11 +734,12 @@ __global__ __launch_bounds__(256) void emit_big_kernel(EmitArgs a)
         const float4* e4 = (const float4*)&r;
         const float4 e[3] = {e4[0], e4[1], e4[2]};
         const float4 vp = make_float4(dd.vp_w, dd.vp_h, dd.half_x, dd.half_y);
-        const bool triangle = (r.flags & (kPrimPoint | kPrimLine)) == 0u;
+        const uint32_t kind = r.flags & (kPrimPoint | kPrimLine);
+        const float4 l = (kind & kPrimLine) ? *(const float4*)&a.ext[gp] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         for (uint32_t k = threadIdx.x; k < c && off + k < a.cap; k += 256u) {
             const uint32_t row = k / w, col = k % w;
             a.keys[off + k] = t.tile_base + (ty0 + row) * t.tiles_x + tx0 + col;
-            a.vals[off + k] = gp | pair_blocks_covered(sh, box, col, row, triangle, e, vp, (int)(tx0 << sh), (int)(ty0 << sh));
+            a.vals[off + k] = gp | pair_blocks_covered(sh, box, col, row, kind, e, l, vp, (int)(tx0 << sh), (int)(ty0 << sh));
         }
     }
 }

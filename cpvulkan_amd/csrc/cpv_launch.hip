@@ -412,7 +412,7 @@ int enqueue_bin(Exec& x, const LaunchPlan& P, uint8_t* arena, uint32_t pair_cap,
     // emit pairs in primitive order
     if (P.prim_total) {
         fill_u32(x.s, b.big.p, 0u, 1);
-        EmitArgs ea{b.recs.as<TriSetup>(), b.counts.as<uint32_t>(), b.offsets.as<uint32_t>(), d_dd, d_tp, b.keys[0].as<uint32_t>(),
+        EmitArgs ea{b.recs.as<TriSetup>(), P.lines ? b.line_ext.as<LineExt>() : nullptr, b.counts.as<uint32_t>(), b.offsets.as<uint32_t>(), d_dd, d_tp, b.keys[0].as<uint32_t>(),
                     b.vals[0].as<uint32_t>(), b.big.as<uint32_t>(), P.prim_total, P.tile_shift, cap};
         const uint32_t blocks = std::min<uint32_t>((P.prim_total + 255) / 256, 8192);
         hipLaunchKernelGGL(emit_kernel, dim3(blocks), dim3(256), 0, x.s, ea);

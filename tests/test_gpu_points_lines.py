@@ -46,6 +46,18 @@ def test_line_list(gpu_ctx, width):
     _check(gpu_ctx, W.lines_scene(400, 256, 160, seed=23, line_width=width), f"line list w={width}")
 
 
+@pytest.mark.parametrize("Wd,Ht", [(640, 360), (97, 401)])
+@pytest.mark.parametrize("spread", [0.05, 20.0])
+def test_thin_lines(gpu_ctx, Wd, Ht, spread):
+    """Quads far thinner than a pixel: clip w (and with it the length that normalize divides by) varies by `spread`."""
+    s = W.lines_scene(500, Wd, Ht, seed=37, line_width=1.25)
+    v = s.draws[0].vertices[0].view(np.float32).reshape(-1, 8)
+    w = 0.5 + spread * np.random.default_rng(5).random((v.shape[0], 1), dtype=np.float32)
+    v[:, :3] *= w / v[:, 3:4]
+    v[:, 3:4] = w
+    _check(gpu_ctx, s, f"thin lines {Wd}x{Ht} spread {spread}")
+
+
 @pytest.mark.parametrize("width", [1.0, 3.0])
 @pytest.mark.parametrize("perspective", [True, False])
 def test_line_strip(gpu_ctx, width, perspective):

@@ -149,11 +149,11 @@ __device__ void setup_point(const SetupArgs& a, const DrawDesc& d, uint32_t di, 
     r.dt_lo = -__builtin_inff();
     r.dt_hi = __builtin_inff();
     r.area = 1.0f;
-    r.draw = di;
+    r.draw_flags = di | ((kPrimFront | kPrimPoint) << kPrimFlagShift);   // DrawPixel(..., front = true, ...)
+    r.rinv = 1.0f;
     r.z[0] = P[2]; r.z[1] = 0.0f; r.z[2] = 0.0f;
     r.w[0] = r.w[1] = r.w[2] = P[3];
     r.v[0] = r.v[1] = r.v[2] = slot;
-    r.flags = kPrimFront | kPrimPoint;   // DrawPixel(..., front = true, ...)
     r.provoking = slot;
     r.pad = 0;
     store_record(&a.recs[gp], r);
@@ -260,11 +260,11 @@ __device__ void setup_line(const SetupArgs& a, const DrawDesc& d, uint32_t di, u
     r.x0 = x0; r.y0 = y0; r.x1 = x1; r.y1 = y1;
     r.dt_lo = -__builtin_inff();
     r.dt_hi = __builtin_inff();
-    r.draw = di;
+    r.draw_flags = di | ((kPrimFront | kPrimLine) << kPrimFlagShift);
+    r.rinv = 0.0f;
     r.z[0] = P0[2]; r.z[1] = P1[2]; r.z[2] = 0.0f;
     r.w[0] = P0[3]; r.w[1] = P1[3]; r.w[2] = P1[3];
     r.v[0] = s0; r.v[1] = s1; r.v[2] = s1;
-    r.flags = kPrimFront | kPrimLine;
     r.provoking = s0;
     r.pad = 0;
     store_record(&a.recs[gp], r);
@@ -356,9 +356,14 @@ __global__ __launch_bounds__(256) void setup_kernel(SetupArgs a)
     r.w[0] = P[0][3]; r.w[1] = P[1][3]; r.w[2] = P[2][3];
     r.x0 = x0; r.y0 = y0; r.x1 = x1; r.y1 = y1;
     r.v[0] = i0; r.v[1] = i1; r.v[2] = i2;
-    r.flags = front ? 1u : 0u;
     r.provoking = slot[3];
-    r.draw = di;
+    r.pad = 0;
+    r.rinv = 1.0f / area;
+    bool fast = area >= 0x1p-60f && area <= 0x1p60f;   // false for NaN, as each of these
+#pragma unroll
+    for (int k = 0; k < 3; k++)
+        fast = fast && fabsf(P[k][0]) <= 0x1p20f && fabsf(P[k][1]) <= 0x1p20f && P[k][2] >= 0.0f && P[k][2] <= 0x1p20f;
+    r.draw_flags = di | ((front ? kPrimFront : 0u) | (fast ? kPrimFast : 0u)) << kPrimFlagShift;
     depth_bounds(r, P, d);
     uint4* dst = (uint4*)&a.recs[gp];
     const uint4* src = (const uint4*)&r;
@@ -662,14 +667,14 @@ __global__ __launch_bounds__(256) void emit_kernel(EmitArgs a)
             const TriSetup& r = a.recs[gp];
             const float4* e4 = (const float4*)&r;
             const float4 e0 = e4[0], e1 = e4[1], e2 = e4[2];
-            const DrawDesc& dd = a.draws[r.draw];
+            const DrawDesc& dd = a.draws[r.draw_flags & kPrimDraw];
             const TargetParams& t = a.targets[dd.target];
             const int sh = a.tile_shift;
             const uint32_t tx0 = (uint32_t)r.x0 >> sh, tx1 = (uint32_t)(r.x1 - 1) >> sh;
             const uint32_t ty0 = (uint32_t)r.y0 >> sh;
             s_dst[threadIdx.x] = a.offsets[gp];
             s_key[threadIdx.x] = t.tile_base + ty0 * t.tiles_x + tx0;
-            s_w[threadIdx.x] = (tx1 - tx0 + 1) | ((r.flags & (kPrimPoint | kPrimLine)) << kKindShift);
+            s_w[threadIdx.x] = (tx1 - tx0 + 1) | (((r.draw_flags >> kPrimFlagShift) & (kPrimPoint | kPrimLine)) << kKindShift);
             s_tx[threadIdx.x] = t.tiles_x;
             const int ox = (int)(tx0 << sh), oy = (int)(ty0 << sh);
             s_box[threadIdx.x] = make_int4(r.x0 - ox, r.y0 - oy, r.x1 - ox, r.y1 - oy);
@@ -722,7 +727,7 @@ __global__ __launch_bounds__(256) void emit_big_kernel(EmitArgs a)
     for (uint32_t b = blockIdx.x; b < n; b += gridDim.x) {
         const uint32_t gp = a.big[1 + b];
         const TriSetup& r = a.recs[gp];
-        const TargetParams& t = a.targets[a.draws[r.draw].target];
+        const TargetParams& t = a.targets[a.draws[r.draw_flags & kPrimDraw].target];
         const int sh = a.tile_shift;
         const uint32_t tx0 = (uint32_t)r.x0 >> sh, tx1 = (uint32_t)(r.x1 - 1) >> sh;
         const uint32_t ty0 = (uint32_t)r.y0 >> sh;
@@ -730,11 +735,11 @@ __global__ __launch_bounds__(256) void emit_big_kernel(EmitArgs a)
         const uint32_t c = a.counts[gp], off = a.offsets[gp];
         const int4 box = make_int4(r.x0 - (int)(tx0 << sh), r.y0 - (int)(ty0 << sh), r.x1 - (int)(tx0 << sh),
                                    r.y1 - (int)(ty0 << sh));
-        const DrawDesc& dd = a.draws[r.draw];
+        const DrawDesc& dd = a.draws[r.draw_flags & kPrimDraw];
         const float4* e4 = (const float4*)&r;
         const float4 e[3] = {e4[0], e4[1], e4[2]};
         const float4 vp = make_float4(dd.vp_w, dd.vp_h, dd.half_x, dd.half_y);
-        const uint32_t kind = r.flags & (kPrimPoint | kPrimLine);
+        const uint32_t kind = (r.draw_flags >> kPrimFlagShift) & (kPrimPoint | kPrimLine);
         const float4 l = (kind & kPrimLine) ? *(const float4*)&a.ext[gp] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         for (uint32_t k = threadIdx.x; k < c && off + k < a.cap; k += 256u) {
             const uint32_t row = k / w, col = k % w;

@@ -70,6 +70,7 @@ struct LaunchPlan {
     int raster_variant = 3;          // index into Program::raster
     bool lines = false;              // some draw rasterises lines (LineExt records)
     int32_t hiz_op = -1, hiz_kind = 32;
+    int32_t less_depth = 0;          // RasterArgs::less_depth
     int32_t uniform_fstate = -1;     // every draw's fragment state is fstates[0] (0), or not (-1)
     size_t o_env = 0, o_dd = 0, o_fs = 0, o_tp = 0, o_vb = 0, o_sb = 0;   // offsets in the arena
 };
@@ -169,6 +170,7 @@ int plan_launch(const cpv_config& cfg, const Program& prog, const std::vector<Ta
         vout_total += nverts;
         prim_total += o.prim_count;
     }
+    if (lds.size() > kPrimDraw) return fail(CPV_ERROR_UNSUPPORTED, "more than 2^28 draws in one launch");
     if (prim_total >= (1u << 28)) return fail(CPV_ERROR_UNSUPPORTED, "more than 2^28 primitives in one launch");
     P->vout_total = vout_total;
     P->prim_total = prim_total;
@@ -196,10 +198,13 @@ int plan_launch(const cpv_config& cfg, const Program& prog, const std::vector<Ta
     P->tiles = tiles;
     // Hierarchical depth culling is exact when only the depth test observes
     // a fragment (no stencil, no depth bounds), every draw uses the same
-    // compare op and depth format, and nobody counts covered fragments.
+    // compare op and depth format, and nobody counts covered fragments.  The
+    // raster kernel's short depth path takes launches whose every draw so
+    // observes LESS or LESS_OR_EQUAL, counted or not.
     P->hiz_op = -1;
     P->hiz_kind = 32;
-    if (!cfg.count_fragments && !P->fstates.empty()) {
+    P->less_depth = 0;
+    if (!P->fstates.empty()) {
         const std::vector<FragmentState>& fs = P->fstates;
         bool ok = true;
         for (const FragmentState& f : fs) {
@@ -209,8 +214,9 @@ int plan_launch(const cpv_config& cfg, const Program& prog, const std::vector<Ta
         }
         for (const TargetParams& t : targets) ok = ok && t.has_ds && t.ds_fmt.depth_kind == fs[0].ds.depth_kind;
         if (ok) {
-            P->hiz_op = fs[0].depth_compare;
+            if (!cfg.count_fragments) P->hiz_op = fs[0].depth_compare;
             P->hiz_kind = fs[0].ds.depth_kind;
+            P->less_depth = fs[0].depth_compare == CPV_COMPARE_LESS || fs[0].depth_compare == CPV_COMPARE_LESS_OR_EQUAL;
         }
     }
     P->uniform_fstate = P->fstates.empty() ? -1 : 0;
@@ -507,7 +513,9 @@ int enqueue_raster(Exec& x, const LaunchPlan& P, uint8_t* arena, const Binned& b
     ra.persistent = sched == CPV_SCHED_COUNTER ? 1u : 0u;
     ra.hiz_op = P.hiz_op;
     ra.hiz_depth_kind = P.hiz_kind;
+    ra.less_depth = P.less_depth;
     ra.uniform_fstate = P.uniform_fstate;
+    ra.count = x.cfg.count_fragments ? 1u : 0u;
     uint32_t grid = P.tiles;
     if (ra.persistent) {
         const int resident = resident_workgroups(x, rk, block);

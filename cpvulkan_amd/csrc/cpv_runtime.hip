@@ -600,7 +600,11 @@ int build_target(const cpv_pass_desc& pass, bool first_segment, int tile, uint32
         t->color_bytes = f.total;
         // DONT_CARE keeps memory as is in the reference, which is LOAD here.
         t->color_load = (first_segment && pass.color[0].load_op == CPV_LOAD_OP_CLEAR) ? 1 : 0;
-        for (int i = 0; i < 4; i++) t->clear_color[i] = pass.color[0].clear.u32[i];
+        // the clear value packed once, as ClearImage -> SetPixel does
+        // (CommandBuffer.Draw.cpp:117-149, ImageSampler.cpp:723-774)
+        if (f.base == kBaseUInt) pack_color_u32(f, pass.color[0].clear.u32, t->clear_color);
+        else if (f.base == kBaseSInt) pack_color_i32(f, pass.color[0].clear.i32, t->clear_color);
+        else pack_color_f32(f, pass.color[0].clear.f32, t->clear_color);
     }
     if (t->has_ds) {
         if (!format_desc(pass.depth_stencil.format, &f)) return fail(CPV_ERROR_UNSUPPORTED, "depth format %u", pass.depth_stencil.format);
@@ -608,8 +612,7 @@ int build_target(const cpv_pass_desc& pass, bool first_segment, int tile, uint32
         t->ds_addr = pass.depth_stencil.address;
         t->ds_bytes = f.total;
         t->ds_load = (first_segment && pass.depth_stencil.load_op == CPV_LOAD_OP_CLEAR) ? 1 : 0;
-        std::memcpy(&t->clear_ds[0], &pass.depth_stencil.clear.ds.depth, 4);
-        t->clear_ds[1] = pass.depth_stencil.clear.ds.stencil;
+        pack_depth_stencil(f, pass.depth_stencil.clear.ds.depth, pass.depth_stencil.clear.ds.stencil, t->clear_ds[0], t->clear_ds[1]);
     }
     return CPV_OK;
 }

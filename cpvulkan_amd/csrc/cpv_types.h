@@ -73,9 +73,9 @@ struct TriSetup {
     int32_t x0, y0, x1, y1;   // 48-63: pixel bounding box, [x0, x1) x [y0, y1)
     float dt_lo, dt_hi;       // 64-71: bounds of the viewport-transformed depth of every covered pixel
     float area;               // 72: |EdgeFunction(p0, p1, p2)|
-    uint32_t draw;            // 76: draw index within the launch
+    uint32_t draw_flags;      // 76: draw index within the launch (28 bits), the kPrim flags above it
     float z[3];               // 80-91: p_k.z / p_k.w
-    uint32_t flags;           // 92: bit 0 front facing, the primitive kind
+    float rinv;               // 92: 1 / area, correctly rounded
     // Bytes 0-95 are everything a primitive's visit of a pixel block reads
     // (kVisitParts 16-byte parts); the rest only the colour work reads.
     float w[3];               // 96-107: clip-space w of p_k
@@ -85,15 +85,20 @@ struct TriSetup {
 };
 static_assert(sizeof(TriSetup) == 128, "TriSetup must be 128 bytes");
 constexpr int kVisitParts = 6;
-static_assert(__builtin_offsetof(TriSetup, flags) == 92 && __builtin_offsetof(TriSetup, w) == 16 * kVisitParts,
+static_assert(__builtin_offsetof(TriSetup, rinv) == 92 && __builtin_offsetof(TriSetup, w) == 16 * kVisitParts,
               "the visit fields fill the first kVisitParts parts");
 
-// TriSetup.flags: bit 0 front facing; the primitive kind.  A point record
-// holds its screen centre (int bits of ax[0], ay[0]), its size (dx[0]), its
-// clamped square [x0, x1) x [y0, y1) and its vertex in v[0]; a line record
-// holds three edges of its quad (the fourth in LineExt), |p1.xy - p0.xy|^2
-// in area, z = (p0.z, p1.z), w = (p0.w, p1.w) and v = (p0, p1).
-enum : uint32_t { kPrimFront = 1u, kPrimPoint = 2u, kPrimLine = 4u };
+// The primitive's flags: front facing; its kind; kPrimFast, set for
+// triangles whose coordinates lie within 2^20, whose area is in [2^-60, 2^60]
+// and whose depths are in [0, 2^20], for which the raster kernel's cheap
+// depth rejection and divisions are proven.  A point record holds its screen
+// centre (int bits of ax[0], ay[0]), its size (dx[0]), its clamped square
+// [x0, x1) x [y0, y1) and its vertex in v[0]; a line record holds three edges
+// of its quad (the fourth in LineExt), |p1.xy - p0.xy|^2 in area,
+// z = (p0.z, p1.z), w = (p0.w, p1.w) and v = (p0, p1).
+enum : uint32_t { kPrimFront = 1u, kPrimPoint = 2u, kPrimLine = 4u, kPrimFast = 8u };
+constexpr int kPrimFlagShift = 28;
+constexpr uint32_t kPrimDraw = (1u << kPrimFlagShift) - 1u;   // launches hold at most this many draws
 
 // A (tile, primitive) pair's value: the primitive index in the low 28 bits
 // (launches hold fewer than 2^28 primitives) and, for 16x16 and 32x32
@@ -151,8 +156,8 @@ struct TargetParams {
     int32_t color_load, ds_load;   // CPV_LOAD_OP_*
     int32_t has_color, has_ds;
     int32_t color_bytes, ds_bytes; // bytes per pixel
-    uint32_t clear_color[4];       // VkClearColorValue bits (float32 / uint32 / int32 by format)
-    uint32_t clear_ds[2];          // VkClearDepthStencilValue: depth bits, stencil
+    uint32_t clear_color[4];       // the clear value as a packed colour pixel
+    uint32_t clear_ds[2];          // the clear value as a packed depth/stencil pixel
     FormatDesc color_fmt, ds_fmt;
 };
 

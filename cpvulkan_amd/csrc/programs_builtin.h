@@ -64,6 +64,7 @@ struct VsMvpLambert {
 // Samples/15-draw_cube/15-draw_cube.cpp:53-61: outColor = color.
 struct FsColor {
     static constexpr int kInputs = 4;
+    static constexpr bool kReadsEnv = false;
     static constexpr bool kMayDiscard = false;
     static constexpr int kWavesPerEU = 6;
     __device__ static int interp(int) { return 0; }
@@ -78,6 +79,7 @@ struct FsColor {
 template <int MODE>
 struct FsColorInterp {
     static constexpr int kInputs = 4;
+    static constexpr bool kReadsEnv = false;
     static constexpr bool kMayDiscard = false;
     static constexpr int kWavesPerEU = 6;
     __device__ static int interp(int) { return MODE; }
@@ -93,6 +95,7 @@ using FsColorNoPerspective = FsColorInterp<1>;
 // if (color.r < 0.25) discard; out = color.
 struct FsColorDiscard {
     static constexpr int kInputs = 4;
+    static constexpr bool kReadsEnv = false;
     static constexpr bool kMayDiscard = true;
     static constexpr int kWavesPerEU = 6;
     __device__ static int interp(int) { return 0; }

@@ -14,6 +14,7 @@
 namespace cpv {
 
 #define CPV_DEV __device__ __forceinline__
+#define CPV_HOST_DEV __host__ __device__ __forceinline__
 
 // ---------------------------------------------------------------- helpers
 
@@ -25,8 +26,28 @@ CPV_DEV int32_t trunc_to_i32(float v)
 }
 
 // llvm.maxnum / llvm.minnum: a NaN operand yields the other operand.
-CPV_DEV float maxnum(float a, float b) { return fmaxf(a, b); }
-CPV_DEV float minnum(float a, float b) { return fminf(a, b); }
+CPV_HOST_DEV float maxnum(float a, float b) { return fmaxf(a, b); }
+CPV_HOST_DEV float minnum(float a, float b) { return fminf(a, b); }
+
+// A wave-uniform address as a pointer through the constant address space:
+// what is read through it (launch descriptors, which no kernel writes) comes
+// by scalar loads, and branches on it are scalar.  With the per-lane address
+// a texture's descriptor cost a vector load for every field and a divergent
+// branch for every format and mode.
+template <class T>
+CPV_DEV const T* uniform_ptr(uint64_t address)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    typedef const __attribute__((address_space(4))) T* ScalarPtr;
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)address);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(address >> 32));
+    return (const T*)(ScalarPtr)(((uint64_t)hi << 32) | lo);
+#else
+    return (const T*)address;
+#endif
+}
+template <class T>
+CPV_DEV const T* uniform_ptr(const T* p) { return uniform_ptr<T>((uint64_t)p); }
 
 // Byte extraction/insertion in a pixel held as 4 dwords (up to 16 bytes).
 CPV_DEV uint32_t pick_word(const uint32_t px[4], int w)
@@ -40,7 +61,7 @@ CPV_DEV uint32_t get_field(const uint32_t px[4], int byte_off, int nbytes)
     const uint32_t v = word >> shift;
     return nbytes >= 4 ? v : (v & ((1u << (nbytes * 8)) - 1u));
 }
-CPV_DEV void set_field(uint32_t px[4], int byte_off, int nbytes, uint32_t v)
+CPV_HOST_DEV void set_field(uint32_t px[4], int byte_off, int nbytes, uint32_t v)
 {
     const int w = byte_off >> 2;
     const int shift = (byte_off & 3) * 8;
@@ -53,6 +74,23 @@ CPV_DEV void set_field(uint32_t px[4], int byte_off, int nbytes, uint32_t v)
 }
 
 // ------------------------------------------------------ format conversion
+
+// The UNORM conversions (float)u / (float)(2^n - 1), n = 8, 16 and 24, as the
+// reference's fdiv rounds them, in two operations: 1 / (2^n - 1) is split
+// into a head whose product with every code is exact and a tail, and the fma
+// rounds once.  Equal to the correctly rounded quotient for every code
+// (tests/test_unorm_forms.py, exhaustive).  One double multiply rounded to
+// float, the form before, took three 64-bit instructions per channel, and a
+// bilinear sample unpacks sixteen channels.
+CPV_DEV float unorm8_to_float(uint32_t u) { return fmaf((float)u, 0x1.010102p-24f, (float)u * 0x1.01p-8f); }
+CPV_DEV float unorm16_to_float(uint32_t u) { return fmaf((float)u, 0x1.0001p-32f, (float)u * 0x1p-16f); }
+CPV_DEV float unorm24_to_float(uint32_t u) { return fmaf((float)u, 0x1.000002p-48f, (float)u * 0x1p-24f); }
+
+// (uint32_t)roundf(x) (half away from zero) for 0 <= x <= 2^24: truncating
+// x + pred(0.5) gives the same integer for every float in that range (checked
+// for all 1.27e9 of them; tests/test_unorm_forms.py checks the floats around
+// every half) in two instructions instead of seven.
+CPV_HOST_DEV uint32_t round_to_u32(float x) { return (uint32_t)(x + 0x1.fffffep-2f); }
 
 // GetPixelF32 of a normal format (LLVMRuntime/ImageCompiler.cpp:161-230,
 // 303-347): channels absent from the format read as (0, 0, 0, 1); integer
@@ -68,12 +106,8 @@ CPV_DEV void unpack_color(const FormatDesc& f, const uint32_t px[4], float out[4
         if (f.base == kBaseSFloat) {
             v = __uint_as_float(raw);
         } else if (f.base == kBaseUNorm || f.base == kBaseUScaled || f.base == kBaseUInt) {
-            // (float)u / 255.0f and (float)u / 65535.0f, computed as one double
-            // multiply rounded to float: identical for every 8- and 16-bit code
-            // (checked exhaustively), a quarter of the instructions of a
-            // correctly rounded fp32 division.
-            if (f.element == 1) v = (float)((double)raw * (1.0 / 255.0));
-            else if (f.element == 2) v = (float)((double)raw * (1.0 / 65535.0));
+            if (f.element == 1) v = unorm8_to_float(raw);
+            else if (f.element == 2) v = unorm16_to_float(raw);
             else v = (float)raw / 4294967296.0f;
         } else {
             const int32_t s = f.element == 1 ? (int32_t)(int8_t)raw : f.element == 2 ? (int32_t)(int16_t)raw : (int32_t)raw;
@@ -87,7 +121,7 @@ CPV_DEV void unpack_color(const FormatDesc& f, const uint32_t px[4], float out[4
 // SetPixelF32 of a normal format (ImageCompiler.cpp:1077-1114, 1179-1197):
 // UNORM clamps with maxnum/minnum, scales by the type maximum, rounds half
 // away from zero (llvm.round) and converts.
-CPV_DEV void pack_color_f32(const FormatDesc& f, const float in[4], uint32_t px[4])
+CPV_HOST_DEV void pack_color_f32(const FormatDesc& f, const float in[4], uint32_t px[4])
 {
 #pragma unroll
     for (int i = 0; i < 4; i++) {
@@ -96,19 +130,19 @@ CPV_DEV void pack_color_f32(const FormatDesc& f, const float in[4], uint32_t px[
         uint32_t raw;
         if (f.base == kBaseUNorm) {
             v = minnum(maxnum(v, 0.0f), 1.0f);
-            raw = (uint32_t)roundf(v * (f.element == 1 ? 255.0f : 65535.0f));
+            raw = round_to_u32(v * (f.element == 1 ? 255.0f : 65535.0f));
         } else if (f.base == kBaseSNorm) {
             v = minnum(maxnum(v, -1.0f), 1.0f);
             raw = (uint32_t)(int32_t)roundf(v * (f.element == 1 ? 127.0f : 32767.0f));
         } else {
-            raw = __float_as_uint(v);
+            raw = __builtin_bit_cast(uint32_t, v);
         }
         set_field(px, f.off[i], f.element, raw);
     }
 }
 
 // SetPixelU32 / SetPixelI32 (ImageCompiler.cpp:1121-1175).
-CPV_DEV void pack_color_u32(const FormatDesc& f, const uint32_t in[4], uint32_t px[4])
+CPV_HOST_DEV void pack_color_u32(const FormatDesc& f, const uint32_t in[4], uint32_t px[4])
 {
 #pragma unroll
     for (int i = 0; i < 4; i++) {
@@ -119,7 +153,7 @@ CPV_DEV void pack_color_u32(const FormatDesc& f, const uint32_t in[4], uint32_t 
         set_field(px, f.off[i], f.element, v);
     }
 }
-CPV_DEV void pack_color_i32(const FormatDesc& f, const int32_t in[4], uint32_t px[4])
+CPV_HOST_DEV void pack_color_i32(const FormatDesc& f, const int32_t in[4], uint32_t px[4])
 {
 #pragma unroll
     for (int i = 0; i < 4; i++) {
@@ -135,10 +169,8 @@ CPV_DEV void pack_color_i32(const FormatDesc& f, const int32_t in[4], uint32_t p
 // as two dwords: dword 0 = bytes 0-3, dword 1 = bytes 4-7.
 CPV_DEV float unpack_depth(const FormatDesc& f, uint32_t d0)
 {
-    // same double-multiply form as unpack_color, exhaustively equal to the
-    // fp32 divisions u / 65535.0f and u / 16777215.0f
-    if (f.depth_kind == 16) return (float)((double)(d0 & 0xFFFFu) * (1.0 / 65535.0));
-    if (f.depth_kind == 24) return (float)((double)(d0 & 0x00FFFFFFu) * (1.0 / 16777215.0));
+    if (f.depth_kind == 16) return unorm16_to_float(d0 & 0xFFFFu);
+    if (f.depth_kind == 24) return unorm24_to_float(d0 & 0x00FFFFFFu);
     if (f.depth_kind == 32) return __uint_as_float(d0);
     return 0.0f;
 }
@@ -150,18 +182,18 @@ CPV_DEV uint32_t unpack_stencil(const FormatDesc& f, uint32_t d0, uint32_t d1)
 }
 
 // SetDSPixel (ImageCompiler.cpp:869-947).
-CPV_DEV void pack_depth_stencil(const FormatDesc& f, float depth, uint32_t stencil, uint32_t& d0, uint32_t& d1)
+CPV_HOST_DEV void pack_depth_stencil(const FormatDesc& f, float depth, uint32_t stencil, uint32_t& d0, uint32_t& d1)
 {
     if (f.depth_kind == 16) {
         const float v = minnum(maxnum(depth, 0.0f), 1.0f);
-        d0 = (d0 & 0xFFFF0000u) | ((uint32_t)roundf(v * 65535.0f) & 0xFFFFu);
+        d0 = (d0 & 0xFFFF0000u) | (round_to_u32(v * 65535.0f) & 0xFFFFu);
     } else if (f.depth_kind == 24) {
         const float v = minnum(maxnum(depth, 0.0f), 1.0f) * 16777215.0f;
-        uint32_t u = (uint32_t)roundf(v);
+        uint32_t u = round_to_u32(v);
         if (f.stencil_off == 3) u |= (stencil & 0xFFu) << 24;   // D24_UNORM_S8_UINT
         d0 = u;
     } else if (f.depth_kind == 32) {
-        d0 = __float_as_uint(depth);                              // raw store, no clamp
+        d0 = __builtin_bit_cast(uint32_t, depth);                 // raw store, no clamp
     }
     if (f.stencil_off >= 0 && !(f.depth_kind == 24 && f.stencil_off == 3)) {
         if (f.stencil_off >= 4) {
@@ -198,7 +230,11 @@ struct TextureDesc {
 // wrap (CPVulkan/ImageSampler.cpp:12-38)
 CPV_DEV int32_t wrap_coord(int32_t v, int32_t size, int32_t mode)
 {
-    if (mode == 0) return (v % size + size) % size;                       // REPEAT
+    if (mode == 0) {                                                       // REPEAT: (v % size + size) % size
+        if ((size & (size - 1)) == 0) return v & (size - 1);               // no division for sizes 2^k
+        const int32_t m = v % size;
+        return m < 0 ? m + size : m;
+    }
     if (mode == 1) {                                                       // MIRRORED_REPEAT
         const int32_t two = 2 * size;
         const int32_t n = (v % two + two) % two - size;
@@ -240,12 +276,14 @@ CPV_DEV void texel(const TextureDesc& t, uint32_t level, int32_t x, int32_t y, f
 }
 
 // lerp (ImageSampler.cpp:51-55): the difference in float, the rest in double.
+// t holds a float, so the product of two 24-bit significands is exact in
+// double and the fma rounds where the multiply and add round.
 CPV_DEV void lerp4(const float a[4], const float b[4], double t, float out[4])
 {
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         const float d = b[i] - a[i];
-        out[i] = (float)((double)a[i] + (double)d * t);
+        out[i] = (float)fma((double)d, t, (double)a[i]);
     }
 }
 
@@ -569,12 +607,11 @@ CPV_DEV bool depth_surely_fails_unit(int32_t op, float cur, float e0, float e1, 
 // the corners, so every pixel's depth lies in [min da - B, max da + B] with
 // B = 2 (3.0001u + 12.2u (1 + 8u)) K + 2^-105 sum |z_i| + 2^-119, which
 // 2^-18 K + 2^-100 sum |z_i| + 2^-118 exceeds by more than the rounding of
-// K, B, lo and hi.
-CPV_DEV bool block_depth_range(const float ax[3], const float ay[3], const float dy[3], const float dx[3], float area,
+// K, B, lo and hi.  r is 1 / area (within an ulp).
+CPV_DEV bool block_depth_range(const float ax[3], const float ay[3], const float dy[3], const float dx[3], float area, float r,
                                const float z[3], float xlo, float xhi, float ylo, float yhi, float& lo, float& hi)
 {
     if (!(area >= 0x1p-40f)) return false;
-    const float r = __builtin_amdgcn_rcpf(area);
     // corners (xlo, ylo), (xhi, ylo), (xlo, yhi), (xhi, yhi)
     float d0 = 0.0f, d1 = 0.0f, d2 = 0.0f, d3 = 0.0f, K = 0.0f, Z = 0.0f;
 #pragma unroll

@@ -79,7 +79,10 @@ struct RasterArgs {
     uint32_t persistent;            // 0: one workgroup per tile; 1: work queue
     int32_t hiz_op;                 // depth compare op shared by every draw when depth culling is exact, else -1
     int32_t hiz_depth_kind;         // 16, 24 or 32
+    int32_t less_depth;             // 1: every draw has the depth test with LESS or LESS_OR_EQUAL (all the same
+                                    // op) and no stencil or depth-bounds test, and all share one depth format
     int32_t uniform_fstate;         // the fragment state every draw of the launch has, -1 when they differ
+    uint32_t count;                 // covered fragments are counted
 };
 
 // True when a depth in [lo, hi] fails `op` against every stored depth in
@@ -92,8 +95,9 @@ __device__ __forceinline__ bool hiz_rejects(int32_t op, float lo, float hi, floa
 __device__ __forceinline__ float stored_depth(int32_t kind, uint32_t d0)
 {
     if (kind == 32) return __uint_as_float(d0);
-    if (kind == 16) return (float)((double)(d0 & 0xFFFFu) * (1.0 / 65535.0));
-    return (float)((double)(d0 & 0x00FFFFFFu) * (1.0 / 16777215.0));
+    if (kind == 0) return 0.0f;
+    if (kind == 16) return unorm16_to_float(d0 & 0xFFFFu);
+    return unorm24_to_float(d0 & 0x00FFFFFFu);
 }
 
 // SetDatum (CommandBuffer.Draw.cpp:816-837) for the three interpolation modes.
@@ -191,12 +195,12 @@ __device__ __forceinline__ void fragment_inputs(const Rec& g, const float* vout,
     const float* q1 = vout + (uint64_t)g.v[1] * stride + 4;
     const float* q2 = vout + (uint64_t)g.v[2] * stride + 4;
     const float* qp = vout + (uint64_t)g.provoking * stride + 4;
-    if (ANYPRIM && (g.flags & kPrimPoint)) {
+    if (ANYPRIM && ((g.draw_flags >> kPrimFlagShift) & kPrimPoint)) {
 #pragma unroll
         for (int c = 0; c < FS::kInputs; c++) in[c] = q0[c];
         return;
     }
-    if (ANYPRIM && (g.flags & kPrimLine)) {
+    if (ANYPRIM && ((g.draw_flags >> kPrimFlagShift) & kPrimLine)) {
 #pragma unroll
         for (int c = 0; c < FS::kInputs; c++) in[c] = interpolate_line(FS::interp(c), w, pw, q0[c], q1[c], qp[c]);
         return;
@@ -218,33 +222,55 @@ __device__ __forceinline__ void fragment_inputs(const Rec& g, const float* vout,
     }
 }
 
+// Whether a fragment shader reads its draw's resources (uniforms, textures);
+// shaders that say nothing are taken to.
+template <class FS, class = void>
+struct ShaderReadsEnv {
+    static constexpr bool value = true;
+};
+template <class FS>
+struct ShaderReadsEnv<FS, decltype((void)FS::kReadsEnv)> {
+    static constexpr bool value = FS::kReadsEnv;
+};
+
 // The shader and the colour write of one queued fragment (lanes hold
-// fragments of different primitives).  When every draw of the launch has
-// the same fragment state (uniform_fstate >= 0) it is read once for the
-// wave, so the blend and format state are scalar and its branches uniform.
+// fragments of different primitives).  The resources and the fragment state
+// are read through scalar pointers: the lanes are taken in groups that share
+// them -- one draw, for a shader that reads its resources, else one fragment
+// state -- and a launch whose draws all have the same state, or a wave whose
+// fragments are of one draw, is one group.  Per-lane descriptor reads made
+// the textured 4K grid's raster kernel wait for a vector load at nearly every
+// format and sampler branch (1,355 us; see raster_tile.h for the kernel now).
 template <class FS, bool ANYPRIM = false, bool FIXED = false>
 __device__ __forceinline__ PixelState shade_fragment(const TriSetup* recs, const DrawDesc* draws, const FragmentState* fstates,
                                                   int32_t uniform_fstate, const float* vout, uint32_t stride, uint32_t gprim,
                                                   float w0, float w1, float w2, int x, int y, PixelState ps)
 {
+    constexpr bool ENV = ShaderReadsEnv<FS>::value;
     const TriSetup& g = recs[gprim];
-    const DrawDesc& d = draws[g.draw];
-    const DrawEnv& de = *(const DrawEnv*)d.env;
+    const uint32_t draw = g.draw_flags & kPrimDraw, flags = g.draw_flags >> kPrimFlagShift;
     float in[FS::kInputs > 0 ? FS::kInputs : 1];
     fragment_inputs<FS, ANYPRIM>(g, vout, stride, w0, w1, w2, in);
     // a point's depth is its vertex's; a line's is p0.z * t + p1.z * (1 - t)
     // with t = w1 (ProcessLines :1494)
-    const float depth = (ANYPRIM && (g.flags & kPrimPoint)) ? g.z[0]
-                        : (ANYPRIM && (g.flags & kPrimLine)) ? g.z[0] * w1 + g.z[1] * (1.0f - w1)
-                                                               : g.z[0] * w0 + g.z[1] * w1 + g.z[2] * w2;
-    float colour[4];
-    // one copy of the shader body (it reads no fragment state); only the
-    // colour write is taken twice
-    const int32_t upper_left = uniform_fstate >= 0 ? fstates[uniform_fstate].origin_upper_left : fstates[d.fstate].origin_upper_left;
-    const float fc[4] = {upper_left ? (float)x : d.vp_w - (float)x - 1.0f, (float)y, depth, 1.0f};
-    FS::run(de, in, fc, (g.flags & 1u) != 0, colour);
-    if (uniform_fstate >= 0) color_write_state<FIXED>(fstates[uniform_fstate], ps, colour);
-    else color_write_state<FIXED>(fstates[d.fstate], ps, colour);
+    const float depth = (ANYPRIM && (flags & kPrimPoint)) ? g.z[0]
+                        : (ANYPRIM && (flags & kPrimLine)) ? g.z[0] * w1 + g.z[1] * (1.0f - w1)
+                                                             : g.z[0] * w0 + g.z[1] * w1 + g.z[2] * w2;
+    uint32_t key = draw;
+    if (!ENV) key = uniform_fstate >= 0 ? (uint32_t)uniform_fstate : draws[draw].fstate;
+    bool todo = true;
+    while (todo) {
+        const uint32_t k = __builtin_amdgcn_readfirstlane(key);
+        if (k != key) continue;
+        todo = false;
+        const DrawDesc& d = *uniform_ptr(&draws[ENV ? k : __builtin_amdgcn_readfirstlane(draw)]);
+        const FragmentState& st = *uniform_ptr(&fstates[ENV ? (uniform_fstate >= 0 ? (uint32_t)uniform_fstate : d.fstate) : k]);
+        const float vw = ENV ? d.vp_w : draws[draw].vp_w;   // lanes of one fragment state may be of different draws
+        const float fc[4] = {st.origin_upper_left ? (float)x : vw - (float)x - 1.0f, (float)y, depth, 1.0f};
+        float colour[4];
+        FS::run(*uniform_ptr<DrawEnv>(d.env), in, fc, (flags & kPrimFront) != 0, colour);
+        color_write_state<FIXED>(st, ps, colour);
+    }
     return ps;
 }
 
@@ -254,30 +280,21 @@ struct DepthStencilResult {
 };
 
 // depth_stencil_ops with the pixel state passed and returned by value (one
-// call site per raster kernel instantiation, inlined).  OP >= 0: the draw
-// has the depth test with compare op OP and no stencil or depth-bounds
-// test, folded into the state as constants.
-template <bool FIXED = false, int OP = -1>
-__device__ __forceinline__ DepthStencilResult depth_stencil_call(const FragmentState* st, PixelState px, float depth, uint32_t front)
+// call site per raster kernel instantiation, inlined).
+template <bool FIXED = false>
+__device__ __forceinline__ DepthStencilResult depth_stencil_call(const FragmentState& st, PixelState px, float depth, uint32_t front)
 {
     DepthStencilResult r;
     r.px = px;
     if constexpr (FIXED) {
-        FragmentState s = *st;
+        FragmentState s = st;
         fold_fixed_formats(s);
-        if constexpr (OP >= 0) {
-            s.depth_test = 1;
-            s.depth_compare = OP;
-            s.stencil_test = 0;
-            s.depth_bounds_test = 0;
-        }
         r.write = depth_stencil_ops(s, r.px, depth, front != 0) ? 1u : 0u;
     } else {
-        r.write = depth_stencil_ops(*st, r.px, depth, front != 0) ? 1u : 0u;
+        r.write = depth_stencil_ops(st, r.px, depth, front != 0) ? 1u : 0u;
     }
     return r;
 }
-
 
 __device__ __forceinline__ uint32_t find_target(const TargetParams* t, uint32_t n, uint32_t tile)
 {

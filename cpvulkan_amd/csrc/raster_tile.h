@@ -103,22 +103,104 @@ __device__ __forceinline__ void wave_lds_fence()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Staging area of a workgroup: the visit fields of a chunk's candidates,
-// one region per wave, used with several blocks per lane (see GATHER).
+// The lanes (all of the wave active) that hold a true predicate, as a scalar
+// mask, and back.  The primitive walk keeps its lane tests in such masks:
+// a comparison writes one directly, they combine by scalar instructions, and
+// an empty one is a scalar branch.
+__device__ __forceinline__ uint64_t lanes(bool p)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_ballot_w64(p);
+#else
+    return p ? 1u : 0u;
+#endif
+}
+__device__ __forceinline__ bool in_lanes(uint64_t m)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_inverse_ballot_w64(m);
+#else
+    return m != 0;
+#endif
+}
+
+// An upper bound of the values of a wave's 64 lanes (all active) from row
+// shifts and row broadcasts by DPP on the floats' ordered integer images:
+// their largest, or a NaN (which no comparison below takes for a rejection)
+// when a lane holds a positive one.  Six vector instructions, where a tree
+// of __shfl_xor is six dependent trips through the LDS pipe for every chunk
+// of the primitive walk, and fmaxf adds a canonicalising instruction to each.
+__device__ __forceinline__ float wave_max(float f)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    int32_t v = __builtin_bit_cast(int32_t, f);
+    v ^= (v >> 31) & 0x7FFFFFFF;
+#define CPV_DPP_MAX(ctrl) v = max(v, __builtin_amdgcn_update_dpp((int32_t)0x80000000, v, ctrl, 0xF, 0xF, false))
+    CPV_DPP_MAX(0x111);   // row_shr:1
+    CPV_DPP_MAX(0x112);   // row_shr:2
+    CPV_DPP_MAX(0x114);   // row_shr:4
+    CPV_DPP_MAX(0x118);   // row_shr:8
+    CPV_DPP_MAX(0x142);   // row_bcast:15
+    CPV_DPP_MAX(0x143);   // row_bcast:31
+#undef CPV_DPP_MAX
+    v = __builtin_amdgcn_readlane(v, 63);
+    v ^= (v >> 31) & 0x7FFFFFFF;
+    return __builtin_bit_cast(float, v);
+#else
+    return f;
+#endif
+}
+
+// LDS of a workgroup: the visit fields of a chunk's candidates, one region
+// per wave, used with several blocks per lane (see GATHER), and the lanes'
+// queues of shading work.
 template <class FS, int TILE, int WAVES>
 struct RasterStage {
     static constexpr int kBlocksPerLane = (TILE / 8) * (TILE / 8) / WAVES;
     static constexpr bool kOn = !FS::kMayDiscard && kBlocksPerLane > 1;
-    uint4 v[kOn ? WAVES : 1][kOn ? kVisitParts : 1][64];
+    static constexpr int kQueue = FS::kMayDiscard ? 1 : 4;   // a power of two
+    uint4 v[kOn ? WAVES : 1][kOn ? kVisitParts : 1][kOn ? 64 : 1];
+    float4 q[FS::kMayDiscard ? 1 : WAVES][kQueue][64];
 };
 
-// The kernel body (raster_kernel below).  OP >= 0 is the launch's depth
-// compare op as a compile-time constant, for launches whose every draw has
-// the depth test with that op and no stencil or depth-bounds test (the
-// launches with hierarchical culling): the depth interval tests and the
-// depth compare then fold to single comparisons.  OP = -1 reads the ops at
-// run time.
-template <class FS, int TILE, int WAVES, bool ANYPRIM, bool FIXED, int OP>
+// True when a triangle's depth (weights q_i = e_i / area to within 2 ulps,
+// z_i >= 0, kPrimFast) surely fails LESS and LESS_OR_EQUAL against `cur`.
+// The reference's depth is the rounded sum of z_i * w_i, w_i = e_i / area
+// correctly rounded; it lies within 4.1u S of the real sum D of z_i e_i / area,
+// S = sum |z_i e_i / area| (e_i >= 0 on covered pixels, so S = D), u = 2^-24,
+// and the fused sum below, whose weights err by 2u and which rounds three
+// times, within 5.1u S, both to 2^-122 where products are subnormal (z_i <=
+// 2^20).  So the depth is at least da (1 - 2^-19) - 2^-120, with a factor of
+// three to spare for the roundings of that expression.  With kPrimFast's
+// ranges nothing overflows; a NaN edge makes the comparison false.
+__device__ __forceinline__ bool depth_surely_not_less(float cur, float q0, float q1, float q2, const TriSetup& r)
+{
+    const float da = fmaf(r.z[2], q2, fmaf(r.z[1], q1, r.z[0] * q0));
+    return fmaf(da, 1.0f - 0x1p-19f, -0x1p-120f) > cur;
+}
+
+// e / area correctly rounded, from q = fl(e * rinv), rinv = fl(1 / area):
+// two Newton steps with exact fma residuals (Markstein, "Computation of
+// elementary functions on the IBM RISC System/6000 processor", 1990: when q
+// is within an ulp of the quotient and rinv is the rounded reciprocal, the
+// fma q + rinv * (e - area q) rounds correctly; q = fl(e rinv) is within 1.5
+// ulps, one step brings it within an ulp).  For area in [2^-60, 2^60] and e
+// in [2^-60, 2^43] no step leaves the normal range and the residual is exact.
+// Four instructions beside the product that the depth test shares, where a
+// division takes ten, one of them a quarter-rate reciprocal.
+__device__ __forceinline__ float divide_exact(float e, float area, float rinv, float q)
+{
+    q = fmaf(fmaf(-area, q, e), rinv, q);
+    return fmaf(fmaf(-area, q, e), rinv, q);
+}
+
+// The kernel body.  Launches whose every draw tests depth with LESS or
+// LESS_OR_EQUAL alone (less_depth) take short depth tests: one comparison
+// each for the intervals and the estimate, two for the fragment.  The branch
+// is wave-uniform, and one body serves every launch: a second copy for the
+// op as a template constant raised the register demand past the budget
+// (24 bytes per lane spilled) and doubled the code.
+template <class FS, int TILE, int WAVES, bool ANYPRIM, bool FIXED>
 __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS, TILE, WAVES>& stage_area)
 {
     constexpr int BW = TILE / 8;               // 8x8 blocks per tile row
@@ -126,7 +208,7 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
     constexpr int BPW = BLOCKS / WAVES;        // blocks (pixels) per lane
     static_assert(BLOCKS % WAVES == 0, "tile blocks must divide among the waves");
 
-    const int wave = threadIdx.x >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     const uint32_t home = blockIdx.x % kRasterQueues;
     // Pairs that outgrew their arrays were dropped: the launch draws nothing
@@ -154,7 +236,8 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
     constexpr bool BLOCK_DEPTH = !ANYPRIM && !GATHER && BPW == 1;
     auto& stage = stage_area.v;
     // the hierarchical depth op (-1: no hierarchical culling)
-    const int32_t hiz_op = OP >= 0 ? OP : a.hiz_op;
+    const int32_t hiz_op = a.hiz_op;
+    const bool less = a.less_depth != 0;
     uint32_t tried = 0;   // queues found empty, starting at home
 
     for (;;) {
@@ -179,40 +262,26 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
             if (tried == kRasterQueues) break;
         }
         if (item >= a.tiles) break;
-        const uint32_t tile = a.order ? a.order[item] : item;
+        const uint32_t tile = __builtin_amdgcn_readfirstlane(a.order ? a.order[item] : item);
         const uint64_t t_begin = clock64();
 
-        const uint32_t ti = find_target(a.targets, a.target_count, tile);
-        const TargetParams& tp = a.targets[ti];
+        const uint32_t ti = find_target(uniform_ptr(a.targets), a.target_count, tile);
+        const TargetParams& tp = *uniform_ptr(&a.targets[ti]);
         const uint32_t local = tile - tp.tile_base;
-        const int tile_x0 = (int)(local % tp.tiles_x) * TILE;
-        const int tile_y0 = (int)(local / tp.tiles_x) * TILE;
+        const int tile_x0 = __builtin_amdgcn_readfirstlane((int)(local % tp.tiles_x) * TILE);
+        const int tile_y0 = __builtin_amdgcn_readfirstlane((int)(local / tp.tiles_x) * TILE);
+        const bool has_color = FIXED || tp.has_color, has_ds = FIXED || tp.has_ds;
+        const int color_bytes = FIXED ? 4 : tp.color_bytes, ds_bytes = FIXED ? 4 : tp.ds_bytes;
 
-        // ---- pixel state: loadOp CLEAR packs the clear value as ClearImage ->
-        // SetPixel does (CommandBuffer.Draw.cpp:117-149, ImageSampler.cpp:723-774);
+        // ---- pixel state: loadOp CLEAR sets the packed clear value;
         // LOAD / DONT_CARE read the attachment.
-        PixelState clear;
-        clear.color[0] = clear.color[1] = clear.color[2] = clear.color[3] = 0u;
-        clear.ds0 = clear.ds1 = 0u;
-        if (tp.has_color && tp.color_load == 1) {
-            if (tp.color_fmt.base == kBaseUInt) {
-                pack_color_u32(tp.color_fmt, tp.clear_color, clear.color);
-            } else if (tp.color_fmt.base == kBaseSInt) {
-                const int32_t ci[4] = {(int32_t)tp.clear_color[0], (int32_t)tp.clear_color[1], (int32_t)tp.clear_color[2],
-                                       (int32_t)tp.clear_color[3]};
-                pack_color_i32(tp.color_fmt, ci, clear.color);
-            } else {
-                const float cf[4] = {__uint_as_float(tp.clear_color[0]), __uint_as_float(tp.clear_color[1]),
-                                     __uint_as_float(tp.clear_color[2]), __uint_as_float(tp.clear_color[3])};
-                pack_color_f32(tp.color_fmt, cf, clear.color);
-            }
-        }
-        if (tp.has_ds && tp.ds_load == 1)
-            pack_depth_stencil(tp.ds_fmt, __uint_as_float(tp.clear_ds[0]), tp.clear_ds[1], clear.ds0, clear.ds1);
-
         PixelState px[BPW];
+        // the stored depth as a float, beside its packed code (a D32 code is
+        // its bits)
+        float zc[BPW];
         int pxx[BPW], pxy[BPW];
         bool inside[BPW];
+        const int32_t tile_depth = FIXED ? 32 : has_ds ? tp.ds_fmt.depth_kind : 0;
 #pragma unroll
         for (int k = 0; k < BPW; k++) {
             const int blk = slot + k * WAVES;
@@ -220,39 +289,42 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
             pxx[k] = bx0 + (lane & 7);
             pxy[k] = by0 + (lane >> 3);
             inside[k] = pxx[k] < (int)tp.width && pxy[k] < (int)tp.height;
-            px[k] = clear;
+#pragma unroll
+            for (int w = 0; w < 4; w++) px[k].color[w] = tp.clear_color[w];
+            px[k].ds0 = tp.clear_ds[0];
+            px[k].ds1 = tp.clear_ds[1];
             const uint64_t pix = (uint64_t)pxy[k] * tp.width + (uint64_t)pxx[k];
-            if (inside[k] && tp.has_color && tp.color_load != 1)
-                load_pixel((const uint8_t*)tp.color_addr + pix * tp.color_bytes, tp.color_bytes, px[k].color);
-            if (inside[k] && tp.has_ds && tp.ds_load != 1) {
+            if (inside[k] && has_color && tp.color_load != 1)
+                load_pixel((const uint8_t*)tp.color_addr + pix * color_bytes, color_bytes, px[k].color);
+            if (inside[k] && has_ds && tp.ds_load != 1) {
                 uint32_t w4[4];
-                load_pixel((const uint8_t*)tp.ds_addr + pix * tp.ds_bytes, tp.ds_bytes, w4);
+                load_pixel((const uint8_t*)tp.ds_addr + pix * ds_bytes, ds_bytes, w4);
                 px[k].ds0 = w4[0];
                 px[k].ds1 = w4[1];
-            } else if (inside[k] && tp.has_ds && tp.ds_bytes == 8) {
+            } else if (inside[k] && has_ds && ds_bytes == 8) {
                 // D32_SFLOAT_S8_UINT cleared: SetPixelDepthStencil writes the
                 // depth and the stencil byte and keeps the three padding bytes
                 // (ImageCompiler.cpp:895-945)
                 uint32_t w4[4];
-                load_pixel((const uint8_t*)tp.ds_addr + pix * tp.ds_bytes, tp.ds_bytes, w4);
-                px[k].ds1 = (w4[1] & 0xFFFFFF00u) | (clear.ds1 & 0xFFu);
+                load_pixel((const uint8_t*)tp.ds_addr + pix * ds_bytes, ds_bytes, w4);
+                px[k].ds1 = (w4[1] & 0xFFFFFF00u) | (tp.clear_ds[1] & 0xFFu);
             }
+            zc[k] = stored_depth(tile_depth, px[k].ds0);
         }
+        auto cur_depth = [&](int k) { return FIXED ? __uint_as_float(px[k].ds0) : zc[k]; };
 
         // ---- per-draw state, refreshed when the draw changes
         uint32_t cur_draw = 0xFFFFFFFFu;
         float xf[BPW], yf[BPW];
         float vp_min = 0.0f, vp_max = 1.0f;
-        bool vp_identity = true;
+        bool vp_identity = true, depth_write = false;
+        uint64_t or_equal = 0;   // every lane for LESS_OR_EQUAL, none for LESS
         const FragmentState* fst = nullptr;
         const DrawEnv* env = nullptr;
-        // Conservative depth rejection allowed for this draw, and its op.
-        // With the op a constant (OP >= 0: every draw has the depth test
-        // with op OP and no stencil or depth-bounds test) both are constants
-        // from the start, so the rejection test folds to one compare.
-        bool early = OP >= 0;
-        int32_t depth_op = OP >= 0 ? OP : 7;
-        int32_t depth_kind = 0;
+        // conservative depth rejection allowed for this draw, and its op
+        // (launches without less_depth)
+        bool early = false;
+        int32_t depth_op = 7;
         unsigned long long nfrag = 0;
 
         // Deferred colour work: a fragment that passed the depth/stencil
@@ -260,11 +332,13 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
         // (interpolation, fragment shader, blend, pack) queued.  Queues drain
         // in order, so every pixel still sees its colour writes in primitive
         // order; draining for all lanes at once keeps the shading path from
-        // running once per primitive whenever any lane passes.
-        constexpr int Q = FS::kMayDiscard ? 1 : 4;
-        uint32_t q_prim[Q];
-        float q_w0[Q], q_w1[Q], q_w2[Q];
-        int qn = 0;
+        // running once per primitive whenever any lane passes.  A lane's
+        // queue is a ring of Q 16-byte entries in LDS (primitive and block,
+        // three weights): a push is one store, where entries in registers
+        // took 20 vector selects per push, a shift per drain and 16 registers.
+        constexpr int Q = RasterStage<FS, TILE, WAVES>::kQueue;
+        int qn = 0, qhead = 0;
+        auto& queue = stage_area.q[FS::kMayDiscard ? 0 : wave];
 
         auto shade = [&](uint32_t gprim, int k, float w0, float w1, float w2) {
             PixelState ps = px[0];
@@ -278,24 +352,21 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
             for (int kk = 0; kk < BPW; kk++)
                 if (kk == k) px[kk] = ps;
         };
-        // Shades the oldest queued entry of every lane that has one and
-        // shifts the queues: called when some lane's queue is full, this
-        // keeps the other lanes' queues filled, so each shading pass runs
-        // with as many lanes as possible.
+        // Shades the oldest queued entry of every lane that has one: called
+        // when some lane's queue is full, this keeps the other lanes' queues
+        // filled, so each shading pass runs with as many lanes as possible.
         auto drain_one = [&]() {
-            if (qn > 0) shade(q_prim[0] & 0x0FFFFFFFu, (int)(q_prim[0] >> 28), q_w0[0], q_w1[0], q_w2[0]);
-#pragma unroll
-            for (int e = 0; e + 1 < Q; e++) {
-                q_prim[e] = q_prim[e + 1];
-                q_w0[e] = q_w0[e + 1];
-                q_w1[e] = q_w1[e + 1];
-                q_w2[e] = q_w2[e + 1];
+            if (qn > 0) {
+                const float4 e = queue[qhead & (Q - 1)][lane];
+                const uint32_t tag = __float_as_uint(e.x);
+                shade(tag & kPairPrim, (int)(tag >> 28), e.y, e.z, e.w);
+                qhead++;
+                qn--;
             }
-            qn = qn > 0 ? qn - 1 : 0;
         };
 
         // ---- walk the tile's primitives in submission order
-        const uint32_t lbeg = a.tile_start[tile], lend = a.tile_start[tile + 1];
+        const uint32_t lbeg = uniform_ptr(a.tile_start)[tile], lend = uniform_ptr(a.tile_start)[tile + 1];
         uint32_t e_next = lbeg + (uint32_t)lane < lend ? a.tile_prims[lbeg + lane] : 0u;
         for (uint32_t base = lbeg; base < lend; base += 64) {
             const int n = (int)min(64u, lend - base);
@@ -305,17 +376,14 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
             float bmin = __builtin_inff(), bmax = -__builtin_inff();
             if (hiz_op >= 0) {
 #pragma unroll
-                for (int k = 0; k < BPW; k++) {
-                    if (inside[k]) {
-                        const float cd = stored_depth(FIXED ? 32 : a.hiz_depth_kind, px[k].ds0);
-                        bmin = fminf(bmin, cd);
-                        bmax = fmaxf(bmax, cd);
-                    }
-                }
+                for (int k = 0; k < BPW; k++)
+                    if (inside[k]) bmax = fmaxf(bmax, cur_depth(k));
+                bmax = wave_max(bmax);
+                if (!less) {
 #pragma unroll
-                for (int off = 32; off > 0; off >>= 1) {
-                    bmin = fminf(bmin, __shfl_xor(bmin, off, 64));
-                    bmax = fmaxf(bmax, __shfl_xor(bmax, off, 64));
+                    for (int k = 0; k < BPW; k++)
+                        if (inside[k]) bmin = fminf(bmin, cur_depth(k));
+                    bmin = -wave_max(-bmin);
                 }
             }
             // each lane tests one primitive of the chunk against the wave's area
@@ -386,7 +454,7 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
                             p5 = src[5];
                         }
                         dz = *(const float4*)(src + 4);
-                        ov = !hiz_rejects(hiz_op, dz.x, dz.y, bmin, bmax);
+                        ov = less ? !(dz.x > bmax) : !hiz_rejects(hiz_op, dz.x, dz.y, bmin, bmax);
                     }
                     if (near) {
                         // lane c holds column bx0 + c, lane 8 r row by0 + r
@@ -395,24 +463,24 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
                         const int rl = min(max((int)p3.y - by0, 0), 7), rh = min(max((int)p3.w - 1 - by0, 0), 7);
                         const float xa = __shfl(xf[0], cl, 64), xb = __shfl(xf[0], ch, 64);
                         const float ya = __shfl(yf[0], rl * 8, 64), yb = __shfl(yf[0], rh * 8, 64);
-                        if (ov && __float_as_uint(dz.w) == cur_draw) {
+                        if (ov && (__float_as_uint(dz.w) & kPrimDraw) == cur_draw) {
                             const float ax[3] = {__uint_as_float(p0.x), __uint_as_float(p0.y), __uint_as_float(p0.z)};
                             const float ay[3] = {__uint_as_float(p0.w), __uint_as_float(p1.x), __uint_as_float(p1.y)};
                             const float dy[3] = {__uint_as_float(p1.z), __uint_as_float(p1.w), __uint_as_float(p2.x)};
                             const float dx[3] = {__uint_as_float(p2.y), __uint_as_float(p2.z), __uint_as_float(p2.w)};
                             const float z[3] = {__uint_as_float(p5.x), __uint_as_float(p5.y), __uint_as_float(p5.z)};
                             float lo, hi;
-                            if (block_depth_range(ax, ay, dy, dx, dz.z, z, fminf(xa, xb), fmaxf(xa, xb), fminf(ya, yb), fmaxf(ya, yb),
-                                                  lo, hi))
-                                ov = !hiz_rejects(hiz_op, lo, hi, bmin, bmax);
+                            if (block_depth_range(ax, ay, dy, dx, dz.z, __uint_as_float(p5.w), z, fminf(xa, xb), fmaxf(xa, xb),
+                                                  fminf(ya, yb), fmaxf(ya, yb), lo, hi))
+                                ov = less ? !(lo > bmax) : !hiz_rejects(hiz_op, lo, hi, bmin, bmax);
                         }
                     }
                 } else if (ov) {
                     if constexpr (!GATHER) dz = *(const float4*)&a.recs[gp_l].dt_lo;
-                    ov = !hiz_rejects(hiz_op, dz.x, dz.y, bmin, bmax);
+                    ov = less ? !(dz.x > bmax) : !hiz_rejects(hiz_op, dz.x, dz.y, bmin, bmax);
                 }
             }
-            uint64_t mask = __ballot(ov);
+            uint64_t mask = lanes(ov);
             if constexpr (STAGE) {
                 __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): the LDS loads have landed
                 wave_lds_fence();
@@ -439,11 +507,12 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
                     // the loads of all visit fields issued before the first of
                     // them is used: one memory latency per survivor, not one
                     // for the draw index and another for the rest
-                    __asm__ volatile("" ::"s"(r.ax[0]), "s"(r.y1), "s"(r.dt_lo), "s"(r.draw), "s"(r.z[0]), "s"(r.flags));
+                    __asm__ volatile("" ::"s"(r.ax[0]), "s"(r.y1), "s"(r.dt_lo), "s"(r.draw_flags), "s"(r.z[0]), "s"(r.rinv));
                 }
-                if (r.draw != cur_draw) {
-                    cur_draw = r.draw;
-                    const DrawDesc& d = a.draws[cur_draw];
+                const uint32_t flags = r.draw_flags >> kPrimFlagShift;
+                if ((r.draw_flags & kPrimDraw) != cur_draw) {
+                    cur_draw = r.draw_flags & kPrimDraw;
+                    const DrawDesc& d = *uniform_ptr(&a.draws[cur_draw]);
                     // pixel centres (ProcessTriangles :1571-1580)
 #pragma unroll
                     for (int k = 0; k < BPW; k++) {
@@ -453,28 +522,20 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
                     vp_min = d.vp_min_depth;
                     vp_max = d.vp_max_depth;
                     vp_identity = vp_min == 0.0f && vp_max == 1.0f;
-                    fst = &a.fstates[d.fstate];
-                    env = (const DrawEnv*)d.env;
+                    fst = uniform_ptr(&a.fstates[d.fstate]);
+                    env = uniform_ptr<DrawEnv>(d.env);
+                    or_equal = fst->depth_compare == 3 ? ~0ull : 0ull;   // LESS_OR_EQUAL
+                    depth_write = fst->depth_write != 0;
                     // Rejecting on the depth test alone is exact when nothing
                     // else observes the fragment: no depth-bounds or stencil
                     // test (and so no stencil write).
-                    if constexpr (OP >= 0) {
-                        depth_kind = 32;
-                    } else if constexpr (FIXED) {
-                        early = fst->depth_test && !fst->depth_bounds_test;
-                        depth_kind = 32;
-                    } else {
-                        early = fst->depth_test && fst->has_ds && fst->ds.depth_off >= 0 && fst->ds.vk_format != 127u &&
-                                !fst->depth_bounds_test && !fst->stencil_test;
-                        depth_kind = fst->ds.depth_kind;
-                    }
-                    depth_op = OP >= 0 ? OP : fst->depth_compare;
+                    early = !less && fst->depth_test && (FIXED || (fst->has_ds && fst->ds.depth_off >= 0 && fst->ds.vk_format != 127u)) &&
+                            !fst->depth_bounds_test && !fst->stencil_test;
+                    depth_op = fst->depth_compare;
                 }
+                const bool has_fcolor = FIXED || fst->has_color;
 #pragma unroll
                 for (int k = 0; k < BPW; k++) {
-                    // every lane is active here; a lane queues at most one
-                    // entry per iteration, so a free slot always exists
-                    if (!FS::kMayDiscard && __any(qn == Q)) drain_one();
                     const int blk = slot + k * WAVES;
                     const int bx0 = tile_x0 + (blk % BW) * 8, by0 = tile_y0 + (blk / BW) * 8;
                     if (TILE == 16 && BPW > 1) {
@@ -485,24 +546,29 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
                         if (TILE == 32 && !((blocks >> ((blk / BW) / 2 * 2 + (blk % BW) / 2)) & 1u)) continue;
                         if (r.x1 <= bx0 || r.x0 >= bx0 + 8 || r.y1 <= by0 || r.y0 >= by0 + 8) continue;
                     }
+                    // The tests narrow `m`, the lanes still in, with every lane
+                    // evaluating them; the visit ends when it is empty, and no
+                    // lane branches until the fragments that are left.
                     const int x = pxx[k], y = pxy[k];
-                    if (x < r.x0 || x >= r.x1 || y < r.y0 || y >= r.y1) continue;
+                    uint64_t m = lanes(x >= r.x0) & lanes(x < r.x1) & lanes(y >= r.y0) & lanes(y < r.y1);
                     if (hiz_op >= 0) {
-                        const float cd = stored_depth(FIXED ? 32 : a.hiz_depth_kind, px[k].ds0);
-                        if (hiz_rejects(hiz_op, r.dt_lo, r.dt_hi, cd, cd)) continue;
+                        const float cd = cur_depth(k);
+                        if (less) m &= ~lanes(r.dt_lo > cd);
+                        else m &= ~lanes(hiz_rejects(hiz_op, r.dt_lo, r.dt_hi, cd, cd));
                     }
+                    if (!m) continue;
                     float w0, w1, w2, depth;
-                    if (ANYPRIM && (r.flags & kPrimPoint)) {
+                    if (ANYPRIM && (flags & kPrimPoint)) {
                         // ProcessPoints (:1358-1378): s, t of the pixel in the
                         // point's square, the vertex's outputs and depth as they are
                         const float size = r.dx[0];
                         const float s = 0.5f + (float)(int32_t)((uint32_t)x - (uint32_t)__float_as_int(r.ax[0])) / size;
                         const float t = 0.5f + (float)(int32_t)((uint32_t)y - (uint32_t)__float_as_int(r.ay[0])) / size;
-                        if (!(s >= 0.0f && t >= 0.0f && s <= 1.0f && t <= 1.0f)) continue;
-                        nfrag++;
+                        m &= lanes(s >= 0.0f) & lanes(t >= 0.0f) & lanes(s <= 1.0f) & lanes(t <= 1.0f);
+                        nfrag += (uint32_t)__popcll(m);
                         w0 = 1.0f; w1 = 0.0f; w2 = 0.0f;
                         depth = r.z[0];
-                    } else if (ANYPRIM && (r.flags & kPrimLine)) {
+                    } else if (ANYPRIM && (flags & kPrimLine)) {
                         // ProcessLines (:1420-1497): all four quad edges >= 0
                         // (NaN fails), t = dot(p - p0, p1 - p0) / |p1 - p0|^2
                         const LineExt L = load_line_ext(a.line_ext, gprim);
@@ -510,57 +576,97 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
                         const float e1 = (xf[k] - r.ax[1]) * r.dy[1] - (yf[k] - r.ay[1]) * r.dx[1];
                         const float e2 = (xf[k] - r.ax[2]) * r.dy[2] - (yf[k] - r.ay[2]) * r.dx[2];
                         const float e3 = (xf[k] - L.ax3) * L.dy3 - (yf[k] - L.ay3) * L.dx3;
-                        if (!(e0 >= 0.0f && e1 >= 0.0f && e2 >= 0.0f && e3 >= 0.0f)) continue;
-                        nfrag++;
+                        m &= lanes(e0 >= 0.0f) & lanes(e1 >= 0.0f) & lanes(e2 >= 0.0f) & lanes(e3 >= 0.0f);
+                        nfrag += (uint32_t)__popcll(m);
+                        if (!m) continue;
                         const float t = ((xf[k] - L.p0x) * L.ddx + (yf[k] - L.p0y) * L.ddy) / r.area;
                         w0 = 1.0f - t; w1 = t; w2 = 0.0f;
                         depth = r.z[0] * t + r.z[1] * (1.0f - t);
                     } else {
-                        // GetFragmentInput (:874-903); NaN edge values are not < 0 and pass
+                        // GetFragmentInput (:874-903); NaN edge values are not
+                        // < 0 and pass, and fminf passes over them
                         const float e0 = (xf[k] - r.ax[0]) * r.dy[0] - (yf[k] - r.ay[0]) * r.dx[0];
                         const float e1 = (xf[k] - r.ax[1]) * r.dy[1] - (yf[k] - r.ay[1]) * r.dx[1];
                         const float e2 = (xf[k] - r.ax[2]) * r.dy[2] - (yf[k] - r.ay[2]) * r.dx[2];
-                        if (e0 < 0 || e1 < 0 || e2 < 0) continue;
-                        nfrag++;
-                        if (early) {
-                            const float cur = (FIXED || depth_kind == 32) ? __uint_as_float(px[k].ds0) : unpack_depth(fst->ds, px[k].ds0);
-                            if (vp_identity ? depth_surely_fails_unit(depth_op, cur, e0, e1, e2, r.area, r.z[0], r.z[1], r.z[2])
-                                            : depth_surely_fails(depth_op, cur, e0, e1, e2, r.area, r.z[0], r.z[1], r.z[2], vp_min, vp_max))
-                                continue;
+                        const float emin = fminf(fminf(e0, e1), e2);
+                        m &= ~lanes(emin < 0.0f);
+                        nfrag += (uint32_t)__popcll(m);
+                        const bool fast = (flags & kPrimFast) != 0;   // wave-uniform
+                        const float q0 = e0 * r.rinv, q1 = e1 * r.rinv, q2 = e2 * r.rinv;
+                        if (less) {
+                            if (fast && vp_identity) m &= ~lanes(depth_surely_not_less(cur_depth(k), q0, q1, q2, r));
+                        } else if (early) {
+                            if (vp_identity)
+                                m &= ~lanes(depth_surely_fails_unit(depth_op, cur_depth(k), e0, e1, e2, r.area, r.z[0], r.z[1], r.z[2]));
+                            else
+                                m &= ~lanes(depth_surely_fails(depth_op, cur_depth(k), e0, e1, e2, r.area, r.z[0], r.z[1], r.z[2],
+                                                               vp_min, vp_max));
                         }
-                        w0 = e0 / r.area; w1 = e1 / r.area; w2 = e2 / r.area;
+                        if (!m) continue;
+                        // a tiny edge value (or an exact zero, whose sign the
+                        // quotient keeps) takes the divisions
+                        if (fast && !(m & ~lanes(emin >= 0x1p-60f))) {
+                            w0 = divide_exact(e0, r.area, r.rinv, q0);
+                            w1 = divide_exact(e1, r.area, r.rinv, q1);
+                            w2 = divide_exact(e2, r.area, r.rinv, q2);
+                        } else {
+                            w0 = e0 / r.area; w1 = e1 / r.area; w2 = e2 / r.area;
+                        }
                         depth = r.z[0] * w0 + r.z[1] * w1 + r.z[2] * w2;
                     }
                     // DrawPixel (:1300-1313)
                     const float dt = (vp_max - vp_min) * depth + vp_min;
-                    const bool front = (r.flags & 1u) != 0;
+                    const bool front = (flags & kPrimFront) != 0;
                     if (FS::kMayDiscard) {
+                        if (!in_lanes(m)) continue;
                         // the shader decides first whether anything is written
-                        float in[FS::kInputs > 0 ? FS::kInputs : 1];
-                        fragment_inputs<FS, ANYPRIM>(r, a.vout, a.vout_stride, w0, w1, w2, in);
-                        const float fc[4] = {fst->origin_upper_left ? (float)x : a.draws[cur_draw].vp_w - (float)x - 1.0f, (float)y,
-                                             depth, 1.0f};
+                        float in_v[FS::kInputs > 0 ? FS::kInputs : 1];
+                        fragment_inputs<FS, ANYPRIM>(r, a.vout, a.vout_stride, w0, w1, w2, in_v);
+                        const float fc[4] = {fst->origin_upper_left ? (float)x : uniform_ptr(&a.draws[cur_draw])->vp_w - (float)x - 1.0f,
+                                             (float)y, depth, 1.0f};
                         float colour[4];
-                        if (FS::run(*env, in, fc, front, colour)) continue;
-                        const DepthStencilResult dr = depth_stencil_call<FIXED, OP>(fst, px[k], dt, front ? 1u : 0u);
+                        if (FS::run(*env, in_v, fc, front, colour)) continue;
+                        const DepthStencilResult dr = depth_stencil_call<FIXED>(*fst, px[k], dt, front ? 1u : 0u);
                         px[k] = dr.px;
-                        if (dr.write && (FIXED || fst->has_color)) color_write_state<FIXED>(*fst, px[k], colour);
+                        if (!FIXED) zc[k] = stored_depth(tile_depth, px[k].ds0);
+                        if (dr.write && has_fcolor) color_write_state<FIXED>(*fst, px[k], colour);
                     } else {
-                        const DepthStencilResult dr = depth_stencil_call<FIXED, OP>(fst, px[k], dt, front ? 1u : 0u);
-                        px[k] = dr.px;
-                        if (!(dr.write && (FIXED || fst->has_color))) continue;
-                        const uint32_t tag = gprim | ((uint32_t)k << 28);
-#pragma unroll
-                        for (int e = 0; e < Q; e++) {
-                            if (e == qn) { q_prim[e] = tag; q_w0[e] = w0; q_w1[e] = w1; q_w2[e] = w2; }
+                        if (less) {
+                            const float cd = cur_depth(k);
+                            m &= lanes(dt < cd) | (lanes(dt == cd) & or_equal);
+                            if (!m) continue;
+                            if (depth_write && in_lanes(m)) {
+                                if (FIXED) {
+                                    px[k].ds0 = __float_as_uint(dt);
+                                } else {
+                                    pack_depth_stencil(fst->ds, dt, unpack_stencil(fst->ds, px[k].ds0, px[k].ds1), px[k].ds0, px[k].ds1);
+                                    zc[k] = stored_depth(tile_depth, px[k].ds0);
+                                }
+                            }
+                        } else {
+                            bool write = false;
+                            if (in_lanes(m)) {
+                                const DepthStencilResult dr = depth_stencil_call<FIXED>(*fst, px[k], dt, front ? 1u : 0u);
+                                px[k] = dr.px;
+                                if (!FIXED) zc[k] = stored_depth(tile_depth, px[k].ds0);
+                                write = dr.write != 0;
+                            }
+                            m = lanes(write);
                         }
-                        qn++;
+                        if (!m || !has_fcolor) continue;
+                        // every lane is active here; a lane queues at most one
+                        // entry per visit, so a free slot always exists
+                        if (lanes(qn == Q)) drain_one();
+                        if (in_lanes(m)) {
+                            queue[(qhead + qn) & (Q - 1)][lane] = make_float4(__uint_as_float(gprim | ((uint32_t)k << 28)), w0, w1, w2);
+                            qn++;
+                        }
                     }
                 }
             }
         }
         if (!FS::kMayDiscard) {
-            while (__any(qn > 0)) drain_one();
+            while (lanes(qn > 0)) drain_one();
         }
         (void)env;
 
@@ -569,16 +675,15 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
         for (int k = 0; k < BPW; k++) {
             if (!inside[k]) continue;
             const uint64_t pix = (uint64_t)pxy[k] * tp.width + (uint64_t)pxx[k];
-            if (tp.has_color) store_pixel((uint8_t*)tp.color_addr + pix * tp.color_bytes, FIXED ? 4 : tp.color_bytes, px[k].color);
-            if (tp.has_ds) {
+            if (has_color) store_pixel((uint8_t*)tp.color_addr + pix * color_bytes, color_bytes, px[k].color);
+            if (has_ds) {
                 const uint32_t w4[4] = {px[k].ds0, px[k].ds1, 0u, 0u};
-                store_pixel((uint8_t*)tp.ds_addr + pix * tp.ds_bytes, FIXED ? 4 : tp.ds_bytes, w4);
+                store_pixel((uint8_t*)tp.ds_addr + pix * ds_bytes, ds_bytes, w4);
             }
         }
 
-        // ---- statistics
-        for (int off = 32; off > 0; off >>= 1) nfrag += __shfl_down(nfrag, off, 64);
-        if (lane == 0 && nfrag) atomicAdd(a.fragments, nfrag);
+        // ---- statistics (nfrag is wave-uniform)
+        if (a.count && lane == 0 && nfrag) atomicAdd(a.fragments, nfrag);
         if (a.trace_cycles && lane == 0) a.trace_cycles[(uint64_t)tile * WAVES + slot] = (float)(clock64() - t_begin);
 
         if (!a.persistent) break;
@@ -588,20 +693,13 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
 // ANYPRIM: the launch may hold point and line records besides triangles
 // (one 16x16 / four-wave instantiation per fragment shader carries it).
 // FIXED: every pipeline and target of the launch has the fixed formats
-// (fold_fixed_formats).  The fixed-format kernels carry a second copy of
-// the body for depth op LESS, the common one.
+// (fold_fixed_formats).
 template <class FS, int TILE, int WAVES, bool ANYPRIM = false, bool FIXED = false>
 __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(raster_waves_per_eu<FS, TILE, WAVES>()))) void
 raster_kernel(RasterArgs a)
 {
     __shared__ RasterStage<FS, TILE, WAVES> stage;
-    if constexpr (FIXED) {
-        if (a.hiz_op == 1) {
-            raster_body<FS, TILE, WAVES, ANYPRIM, FIXED, 1>(a, stage);
-            return;
-        }
-    }
-    raster_body<FS, TILE, WAVES, ANYPRIM, FIXED, -1>(a, stage);
+    raster_body<FS, TILE, WAVES, ANYPRIM, FIXED>(a, stage);
 }
 
 }  // namespace cpv

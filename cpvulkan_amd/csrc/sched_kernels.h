@@ -72,7 +72,7 @@ __global__ __launch_bounds__(256) void tile_features_kernel(FeatureArgs a)
         const float box = (float)(max(cx1 - cx0, 0) * max(cy1 - cy0, 0));
         s_box += box;
         s_full += (r.x0 <= x0 && r.y0 <= y0 && r.x1 >= x1 && r.y1 >= y1) ? 1.0f : 0.0f;
-        const DrawDesc& d = a.draws[r.draw];
+        const DrawDesc& d = a.draws[r.draw_flags & kPrimDraw];
         const float tri = fabsf(r.area) * d.vp_w * d.vp_h * 0.125f;   // edge function = twice the NDC area
         s_tri += fminf(tri, tile_px);
         s_blend += a.fstates[d.fstate].blend_enable ? 1.0f : 0.0f;

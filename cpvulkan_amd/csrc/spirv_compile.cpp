@@ -1590,6 +1590,8 @@ Translation translate(const uint32_t* vs, size_t vs_n, const char* vs_entry, con
     const int fin = (int)gf.interp.size();
     s << "struct SpvFs {\n    static constexpr int kInputs = " << fin << ";\n" << gf.types.str()
       << "    static constexpr bool kMayDiscard = " << (gf.discard ? "true" : "false") << ";\n"
+      << "    static constexpr bool kReadsEnv = "
+      << ((gf.decl.str() + gf.fns.str() + gf.pro.str() + gf.code.str() + gf.epi.str()).find("env") != std::string::npos ? "true" : "false") << ";\n"
       << "    __device__ static int interp(int c)\n    {\n";
     for (int c = 0; c < fin; c++)
         if (gf.interp[c]) s << "        if (c == " << c << ") return " << gf.interp[c] << ";\n";

@@ -1,5 +1,6 @@
-// Shader-independent kernels: triangle setup, prefix scans and the
-// order-preserving tile binning (emit + stable LSD radix sort by tile).
+// Shader-independent kernels: triangle setup and the order-preserving tile
+// binning: emit + stable LSD radix sort by tile, or for small launches one
+// kernel that writes the tiles' lists directly.
 //
 // Binning must keep submission order inside every tile: blending and the
 // LESS depth test are order dependent, and the reference draws primitives
@@ -23,6 +24,7 @@ struct SetupArgs {
     TriSetup* recs;
     LineExt* ext;                 // per-primitive line extension (launches with lines)
     uint32_t* counts;             // tiles overlapped per primitive (0 = dropped)
+    uint64_t* sums;               // tiles overlapped by the primitives of each workgroup
     uint32_t stride;
     int32_t tile_shift;
 };
@@ -126,10 +128,10 @@ __device__ __forceinline__ int32_t wrap_sub(int32_t a, int32_t b) { return (int3
 // ProcessPoints (CommandBuffer.Draw.cpp:1315-1383): centre
 // (int)((p.x + 1) * 0.5f * (viewport.width - 1)), half extent
 // (int)ceil(pointSize / 2), square [max(0, c - h), min(width, c + h + 1)).
-__device__ void setup_point(const SetupArgs& a, const DrawDesc& d, uint32_t di, uint32_t p, uint32_t gp)
+__device__ uint32_t setup_point(const SetupArgs& a, const DrawDesc& d, uint32_t di, uint32_t p, uint32_t gp)
 {
     uint32_t slot;
-    if (!vertex_slot(d, p, &slot)) { a.counts[gp] = 0; return; }
+    if (!vertex_slot(d, p, &slot)) return 0u;
     float P[4];
     clip_to_ndc(a.vout, a.stride, slot, P);
     const float size = d.psize >= 0 ? a.vout[(uint64_t)slot * a.stride + 4 + (uint32_t)d.psize] : 0.0f;
@@ -138,7 +140,7 @@ __device__ void setup_point(const SetupArgs& a, const DrawDesc& d, uint32_t di, 
     const int32_t h = trunc_to_i32(ceilf(size / 2.0f));
     const int32_t x0 = max(0, wrap_sub(cx, h)), y0 = max(0, wrap_sub(cy, h));
     const int32_t x1 = min(d.limit_x, wrap_add(wrap_add(cx, h), 1)), y1 = min(d.limit_y, wrap_add(wrap_add(cy, h), 1));
-    if (x0 >= x1 || y0 >= y1) { a.counts[gp] = 0; return; }
+    if (x0 >= x1 || y0 >= y1) return 0u;
     TriSetup r;
     r.ax[0] = __int_as_float(cx);
     r.ay[0] = __int_as_float(cy);
@@ -157,7 +159,7 @@ __device__ void setup_point(const SetupArgs& a, const DrawDesc& d, uint32_t di, 
     r.provoking = slot;
     r.pad = 0;
     store_record(&a.recs[gp], r);
-    a.counts[gp] = tiles_of(x0, y0, x1, y1, a.tile_shift);
+    return tiles_of(x0, y0, x1, y1, a.tile_shift);
 }
 
 // Pixel box that holds every pixel whose centre can pass the four edge
@@ -220,11 +222,11 @@ __device__ bool line_box(const DrawDesc& d, const float* c[4], int32_t* x0, int3
 // its centre has E(p00, p01) >= 0, E(p11, p10) >= 0, E(p10, p00) >= 0 and
 // E(p01, p11) >= 0.  The reference scans the whole viewport; the record's
 // box is line_box's when it applies.
-__device__ void setup_line(const SetupArgs& a, const DrawDesc& d, uint32_t di, uint32_t p, uint32_t gp)
+__device__ uint32_t setup_line(const SetupArgs& a, const DrawDesc& d, uint32_t di, uint32_t p, uint32_t gp)
 {
     const uint32_t r0 = d.topology == 1 ? 2 * p : p;   // LINE_LIST or LINE_STRIP (CalculatePrimitives :584-611)
     uint32_t s0, s1;
-    if (!vertex_slot(d, r0, &s0) || !vertex_slot(d, r0 + 1, &s1)) { a.counts[gp] = 0; return; }
+    if (!vertex_slot(d, r0, &s0) || !vertex_slot(d, r0 + 1, &s1)) return 0u;
     float P0[4], P1[4];
     clip_to_ndc(a.vout, a.stride, s0, P0);
     clip_to_ndc(a.vout, a.stride, s1, P1);
@@ -256,7 +258,7 @@ __device__ void setup_line(const SetupArgs& a, const DrawDesc& d, uint32_t di, u
     int32_t y1 = d.vp_h >= (float)t.height ? (int32_t)t.height : (int32_t)ceilf(d.vp_h);
     const float* cs[4] = {p00, p01, p10, p11};
     line_box(d, cs, &x0, &y0, &x1, &y1);
-    if (x0 >= x1 || y0 >= y1) { a.counts[gp] = 0; return; }
+    if (x0 >= x1 || y0 >= y1) return 0u;
     r.x0 = x0; r.y0 = y0; r.x1 = x1; r.y1 = y1;
     r.dt_lo = -__builtin_inff();
     r.dt_hi = __builtin_inff();
@@ -269,21 +271,14 @@ __device__ void setup_line(const SetupArgs& a, const DrawDesc& d, uint32_t di, u
     r.pad = 0;
     store_record(&a.recs[gp], r);
     a.ext[gp] = L;
-    a.counts[gp] = tiles_of(x0, y0, x1, y1, a.tile_shift);
+    return tiles_of(x0, y0, x1, y1, a.tile_shift);
 }
 
 // Per-primitive part of ProcessTriangles (CommandBuffer.Draw.cpp:1526-1569)
 // and the per-triangle constants of GetFragmentInput (:879-898, :900 cull).
-__global__ __launch_bounds__(256) void setup_kernel(SetupArgs a)
+// Returns the tiles the triangle's box overlaps, 0 when it is dropped.
+__device__ uint32_t setup_triangle(const SetupArgs& a, const DrawDesc& d, uint32_t di, uint32_t p, uint32_t gp)
 {
-    const uint32_t di = a.block_draw[blockIdx.x];
-    const DrawDesc& d = a.draws[di];
-    const uint32_t p = (blockIdx.x - d.sblock_base) * 256u + threadIdx.x;
-    if (p >= d.prim_count) return;
-    const uint32_t gp = d.prim_base + p;
-    if (d.topology == 0) { setup_point(a, d, di, p, gp); return; }
-    if (d.topology <= 2) { setup_line(a, d, di, p, gp); return; }
-
     // CalculatePrimitives (:567-673)
     uint32_t raw[3], prov;
     if (d.topology == 3) { raw[0] = 3 * p; raw[1] = 3 * p + 1; raw[2] = 3 * p + 2; prov = 3 * p; }
@@ -306,7 +301,7 @@ __global__ __launch_bounds__(256) void setup_kernel(SetupArgs a)
         ok = ok && s >= 0 && s < (int64_t)d.vout_count;
         slot[k] = d.vout_base + (uint32_t)s;
     }
-    if (!ok) { a.counts[gp] = 0; return; }   // vertex outside the bound buffer
+    if (!ok) return 0u;   // vertex outside the bound buffer
 
     uint32_t i0 = slot[0], i1 = slot[1], i2 = slot[2];
     if (d.front_face == 1) { const uint32_t t = i0; i0 = i2; i2 = t; }   // CLOCKWISE swaps p0, p2
@@ -349,7 +344,7 @@ __global__ __launch_bounds__(256) void setup_kernel(SetupArgs a)
         put_edge(r, 2, P[0], P[1]);
     }
     const bool culled = ((d.cull_mode & 2u) && !front) || ((d.cull_mode & 1u) && front);
-    if (culled || x0 >= x1 || y0 >= y1) { a.counts[gp] = 0; return; }
+    if (culled || x0 >= x1 || y0 >= y1) return 0u;
 
     r.area = area;
     r.z[0] = P[0][2]; r.z[1] = P[1][2]; r.z[2] = P[2][2];
@@ -365,22 +360,40 @@ __global__ __launch_bounds__(256) void setup_kernel(SetupArgs a)
         fast = fast && fabsf(P[k][0]) <= 0x1p20f && fabsf(P[k][1]) <= 0x1p20f && P[k][2] >= 0.0f && P[k][2] <= 0x1p20f;
     r.draw_flags = di | ((front ? kPrimFront : 0u) | (fast ? kPrimFast : 0u)) << kPrimFlagShift;
     depth_bounds(r, P, d);
-    uint4* dst = (uint4*)&a.recs[gp];
-    const uint4* src = (const uint4*)&r;
-#pragma unroll
-    for (int q = 0; q < 8; q++) dst[q] = src[q];
+    store_record(&a.recs[gp], r);
+    return tiles_of(x0, y0, x1, y1, a.tile_shift);
+}
 
-    const int sh = a.tile_shift;
-    const uint32_t tx0 = (uint32_t)x0 >> sh, tx1 = (uint32_t)(x1 - 1) >> sh;
-    const uint32_t ty0 = (uint32_t)y0 >> sh, ty1 = (uint32_t)(y1 - 1) >> sh;
-    a.counts[gp] = (tx1 - tx0 + 1) * (ty1 - ty0 + 1);
+// One thread per primitive.  A workgroup also adds up its primitives' tile
+// counts, so the pair offsets need one scan of a sum per 256 primitives
+// (scan_blocks_kernel) and no pass over the counts.
+__global__ __launch_bounds__(256) void setup_kernel(SetupArgs a)
+{
+    __shared__ uint32_t s_lo[4];
+    const uint32_t di = a.block_draw[blockIdx.x];
+    const DrawDesc& d = *uniform_ptr(&a.draws[di]);
+    const uint32_t p = (blockIdx.x - d.sblock_base) * 256u + threadIdx.x;
+    uint32_t c = 0;
+    if (p < d.prim_count) {
+        const uint32_t gp = d.prim_base + p;
+        if (d.topology == 0) c = setup_point(a, d, di, p, gp);
+        else if (d.topology <= 2) c = setup_line(a, d, di, p, gp);
+        else c = setup_triangle(a, d, di, p, gp);
+        a.counts[gp] = c;
+        // a dropped primitive's record keeps an empty pixel box, which
+        // bin_small_kernel reads
+        if (c == 0) *(int4*)&a.recs[gp].x0 = make_int4(0, 0, 0, 0);
+    }
+    // counts are at most 2^22 (a 16384^2 target in 8x8 tiles): sums of 256 fit
+    // 32 bits, so do the four waves'
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off, 64);
+    if ((threadIdx.x & 63u) == 0) s_lo[threadIdx.x >> 6] = c;
+    __syncthreads();
+    if (threadIdx.x == 0) a.sums[blockIdx.x] = (uint64_t)s_lo[0] + s_lo[1] + s_lo[2] + s_lo[3];
 }
 
 // ---------------------------------------------------------------- scans
-
-constexpr int kScanThreads = 256;
-constexpr int kScanItems = 16;
-constexpr int kScanTile = kScanThreads * kScanItems;
 
 __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* s_tmp, uint32_t& total)
 {
@@ -400,80 +413,74 @@ __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* s
     return wave_base + x - v;
 }
 
-__device__ __forceinline__ uint64_t block_exclusive_scan64(uint64_t v, uint64_t* s_tmp, uint64_t& total)
+constexpr int kScanThreads = 1024;
+constexpr int kScanItems = 4;
+
+struct ScanArgs {
+    uint64_t* sums;          // in: pairs of each setup workgroup; out: their exclusive scan
+    uint32_t blocks;
+    uint32_t cap;            // capacity of the pair arrays
+    uint64_t* total;         // the grand total, in 64 bits
+    uint32_t* kept;          // pairs kept for sorting: min(total, cap)
+    uint32_t* overflow;      // raised when total exceeds cap: then the emit kernels write only the pairs
+                             // below cap and the raster kernel draws nothing
+    uint32_t* big;           // emit_big_kernel's list, emptied
+    uint32_t* host;          // pinned host words: total (two), overflow (nullptr: not wanted)
+};
+
+// Exclusive scan of the setup workgroups' pair sums by one workgroup (4,096
+// a round: the million-triangle frame's 3,907 take one), and what follows
+// from the total.  It stands for the scan of the per-primitive counts (three
+// kernels), the clamp and a clear; the host reads the total from its own
+// memory as soon as this kernel is done, before the pairs are even emitted.
+__global__ __launch_bounds__(kScanThreads) void scan_blocks_kernel(ScanArgs a)
 {
+    __shared__ uint64_t s_tmp[kScanThreads / 64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    uint64_t x = v;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const uint64_t y = __shfl_up(x, off, 64);
-        if (lane >= off) x += y;
-    }
-    if (lane == 63) s_tmp[wave] = x;
-    __syncthreads();
-    uint64_t wave_base = 0;
-    for (int w = 0; w < wave; w++) wave_base += s_tmp[w];
-    total = s_tmp[0] + s_tmp[1] + s_tmp[2] + s_tmp[3];
-    __syncthreads();
-    return wave_base + x - v;
-}
-
-// Sum of each kScanTile-element slab, in 64 bits (a slab of large
-// primitives' tile counts can pass 2^32).
-__global__ __launch_bounds__(kScanThreads) void scan_reduce_kernel(const uint32_t* in, uint32_t n, uint64_t* sums)
-{
-    __shared__ uint64_t s_tmp[4];
-    const uint64_t base = (uint64_t)blockIdx.x * kScanTile + (uint64_t)threadIdx.x * kScanItems;
-    uint64_t s = 0;
-#pragma unroll
-    for (int i = 0; i < kScanItems; i++) s += (base + i < n) ? in[base + i] : 0u;
-    uint64_t total;
-    block_exclusive_scan64(s, s_tmp, total);
-    if (threadIdx.x == 0) sums[blockIdx.x] = total;
-}
-
-// Exclusive scan of the slab sums in place by one workgroup; the grand
-// total, in 64 bits, goes to *total64 (when given).
-__global__ __launch_bounds__(kScanThreads) void scan_sums_kernel(uint64_t* sums, uint32_t n, uint64_t* total64)
-{
-    __shared__ uint64_t s_tmp[4];
     uint64_t carry = 0;
-    for (uint32_t base = 0; base < n; base += kScanThreads) {
-        const uint32_t i = base + threadIdx.x;
-        const uint64_t v = i < n ? sums[i] : 0u;
-        uint64_t total;
-        const uint64_t ex = block_exclusive_scan64(v, s_tmp, total);
-        if (i < n) sums[i] = carry + ex;
+    for (uint32_t base = 0; base < a.blocks; base += kScanThreads * kScanItems) {
+        uint64_t v[kScanItems], s = 0;
+        const uint32_t i0 = base + threadIdx.x * kScanItems;
+#pragma unroll
+        for (int k = 0; k < kScanItems; k++) {
+            v[k] = i0 + k < a.blocks ? a.sums[i0 + k] : 0u;
+            s += v[k];
+        }
+        uint64_t x = s;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint64_t y = __shfl_up(x, off, 64);
+            if (lane >= off) x += y;
+        }
+        if (lane == 63) s_tmp[wave] = x;
+        __syncthreads();
+        uint64_t before = 0, total = 0;
+#pragma unroll
+        for (int w = 0; w < kScanThreads / 64; w++) {
+            const uint64_t t = s_tmp[w];
+            if (w < wave) before += t;
+            total += t;
+        }
+        __syncthreads();
+        uint64_t run = carry + before + x - s;
+#pragma unroll
+        for (int k = 0; k < kScanItems; k++) {
+            if (i0 + k < a.blocks) a.sums[i0 + k] = run;
+            run += v[k];
+        }
         carry += total;
     }
-    if (total64 && threadIdx.x == 0) *total64 = carry;
-}
-
-// Exclusive scan of every slab plus its slab offset; out[n] = grand total
-// when write_total is set.  The 32-bit outputs are exact when the grand
-// total is below 2^32 (the pair scan's is checked against that before its
-// offsets are used).
-__global__ __launch_bounds__(kScanThreads) void scan_down_kernel(const uint32_t* in, uint32_t n, const uint64_t* sums,
-                                                                 uint32_t* out, int write_total)
-{
-    __shared__ uint32_t s_tmp[4];
-    const uint64_t base = (uint64_t)blockIdx.x * kScanTile + (uint64_t)threadIdx.x * kScanItems;
-    uint32_t v[kScanItems];
-    uint32_t s = 0;
-#pragma unroll
-    for (int i = 0; i < kScanItems; i++) {
-        v[i] = (base + i < n) ? in[base + i] : 0u;
-        s += v[i];
+    if (threadIdx.x == 0) {
+        *a.total = carry;
+        *a.kept = carry < (uint64_t)a.cap ? (uint32_t)carry : a.cap;
+        if (carry > (uint64_t)a.cap) *a.overflow = 1u;
+        a.big[0] = 0u;
+        if (a.host) {
+            a.host[0] = (uint32_t)carry;
+            a.host[1] = (uint32_t)(carry >> 32);
+            a.host[2] = carry > (uint64_t)a.cap ? 1u : 0u;
+        }
     }
-    uint32_t total;
-    uint32_t run = (uint32_t)sums[blockIdx.x] + block_exclusive_scan(s, s_tmp, total);
-#pragma unroll
-    for (int i = 0; i < kScanItems; i++) {
-        if (base + i < n) out[base + i] = run;
-        run += v[i];
-    }
-    if (write_total && base < n && base + kScanItems >= n) out[n] = run;
-    if (write_total && n == 0 && blockIdx.x == 0 && threadIdx.x == 0) out[0] = 0;
 }
 
 // ---------------------------------------------------------------- emit
@@ -482,13 +489,13 @@ struct EmitArgs {
     const TriSetup* recs;
     const LineExt* ext;           // per-primitive line extension (launches with lines)
     const uint32_t* counts;
-    const uint32_t* offsets;
+    const uint64_t* sums;         // output offset of each setup workgroup's first pair
+    const uint32_t* block_draw;   // setup-grid block -> draw
     const DrawDesc* draws;
     const TargetParams* targets;
     uint32_t* keys;               // global tile index per pair
     uint32_t* vals;               // primitive index per pair
-    uint32_t* big;                // primitives left to emit_big_kernel; big[0] is the count
-    uint32_t prims;
+    uint32_t* big;                // primitives left to emit_big_kernel: big[0] of them, (primitive, offset) from big[1]
     int32_t tile_shift;
     uint32_t cap;                 // capacity of keys / vals; pairs at or beyond it are dropped
 };
@@ -632,16 +639,17 @@ __device__ __forceinline__ uint32_t pair_blocks_covered(int tile_shift, int4 box
     return keep << kPairBlockShift;
 }
 
-// Writes the (tile, primitive) pairs of every primitive at its scanned
-// offset, so the pair array is in primitive order.  A workgroup takes 256
-// consecutive primitives, whose pairs are one contiguous run of the output
-// (less the runs of primitives with more than kEmitBig pairs, queued for
-// emit_big_kernel): its threads stride over the run, so consecutive lanes
-// write consecutive pairs, and each finds its primitive by binary search of
-// the workgroup's scanned counts in LDS.  What a pair needs of its
-// primitive (tile rectangle, edges, viewport) is staged in LDS by the
-// primitive's thread, so the pair loop reads no record.  Tiles of a
-// primitive go in row-major order of its tile rectangle.
+// Writes the (tile, primitive) pairs of every primitive at its offset, so the
+// pair array is in primitive order.  A workgroup takes the 256 consecutive
+// primitives of one draw that the setup workgroup of its index took, whose
+// pairs are one contiguous run of the output (less the runs of primitives
+// with more than kEmitBig pairs, queued for emit_big_kernel): its threads
+// stride over the run, so consecutive lanes write consecutive pairs, and each
+// finds its primitive by binary search of the workgroup's scanned counts in
+// LDS.  What a pair needs of its primitive (tile rectangle, edges) is staged
+// in LDS by the primitive's thread, so the pair loop reads no record; what it
+// needs of the draw and target is the workgroup's, in scalar registers.
+// Tiles of a primitive go in row-major order of its tile rectangle.
 __global__ __launch_bounds__(256) void emit_kernel(EmitArgs a)
 {
     constexpr int kKindShift = 29;    // s_w: the primitive's kind (kPrimPoint, kPrimLine) above the columns
@@ -650,71 +658,70 @@ __global__ __launch_bounds__(256) void emit_kernel(EmitArgs a)
     __shared__ uint32_t s_dst[256];   // output offset of each primitive's first pair
     __shared__ uint32_t s_key[256];   // global tile index of each primitive's first tile
     __shared__ uint32_t s_w[256];     // tile columns of each primitive's rectangle, | kind << kKindShift
-    __shared__ uint32_t s_tx[256];    // tile columns of each primitive's target
     __shared__ int4 s_box[256];       // pixel box of each primitive, relative to its first tile
     __shared__ int2 s_org[256];       // pixel origin of each primitive's first tile
     __shared__ float4 s_edge[256][3]; // each primitive's edges (record bytes 0-47)
-    __shared__ float4 s_vp[256];      // its draw's vp_w, vp_h, half_x, half_y
-    const uint32_t nblk = (a.prims + 255u) / 256u;
-    for (uint32_t blk = blockIdx.x; blk < nblk; blk += gridDim.x) {
-        const uint32_t gp = blk * 256u + threadIdx.x;
-        uint32_t c = gp < a.prims ? a.counts[gp] : 0u;
-        if (c > kEmitBig) {
-            a.big[1 + atomicAdd(&a.big[0], 1u)] = gp;
-            c = 0;
-        }
-        if (c) {
-            const TriSetup& r = a.recs[gp];
-            const float4* e4 = (const float4*)&r;
-            const float4 e0 = e4[0], e1 = e4[1], e2 = e4[2];
-            const DrawDesc& dd = a.draws[r.draw_flags & kPrimDraw];
-            const TargetParams& t = a.targets[dd.target];
-            const int sh = a.tile_shift;
-            const uint32_t tx0 = (uint32_t)r.x0 >> sh, tx1 = (uint32_t)(r.x1 - 1) >> sh;
-            const uint32_t ty0 = (uint32_t)r.y0 >> sh;
-            s_dst[threadIdx.x] = a.offsets[gp];
-            s_key[threadIdx.x] = t.tile_base + ty0 * t.tiles_x + tx0;
-            s_w[threadIdx.x] = (tx1 - tx0 + 1) | (((r.draw_flags >> kPrimFlagShift) & (kPrimPoint | kPrimLine)) << kKindShift);
-            s_tx[threadIdx.x] = t.tiles_x;
-            const int ox = (int)(tx0 << sh), oy = (int)(ty0 << sh);
-            s_box[threadIdx.x] = make_int4(r.x0 - ox, r.y0 - oy, r.x1 - ox, r.y1 - oy);
-            s_org[threadIdx.x] = make_int2(ox, oy);
-            s_edge[threadIdx.x][0] = e0;
-            s_edge[threadIdx.x][1] = e1;
-            s_edge[threadIdx.x][2] = e2;
-            s_vp[threadIdx.x] = make_float4(dd.vp_w, dd.vp_h, dd.half_x, dd.half_y);
-        }
-        uint32_t total;
-        s_off[threadIdx.x] = block_exclusive_scan(c, s_tmp, total);
-        if (threadIdx.x == 0) s_off[256] = total;
-        __syncthreads();
-        for (uint32_t j = threadIdx.x; j < total; j += 256u) {
-            // lo: the last primitive whose run starts at or before j (s_off is
-            // non-decreasing and s_off[0] = 0), in eight unrolled halvings
-            uint32_t lo = 0;
+    const DrawDesc& dd = *uniform_ptr(&a.draws[a.block_draw[blockIdx.x]]);
+    const TargetParams& t = *uniform_ptr(&a.targets[dd.target]);
+    const uint32_t p = (blockIdx.x - dd.sblock_base) * 256u + threadIdx.x;
+    const uint32_t gp0 = dd.prim_base + (blockIdx.x - dd.sblock_base) * 256u, gp = gp0 + threadIdx.x;
+    const uint32_t tiles_x = t.tiles_x;
+    const float4 vp = make_float4(dd.vp_w, dd.vp_h, dd.half_x, dd.half_y);
+    uint32_t c = p < dd.prim_count ? a.counts[gp] : 0u;
+    uint32_t all;
+    const uint32_t dst = (uint32_t)uniform_ptr(a.sums)[blockIdx.x] + block_exclusive_scan(c, s_tmp, all);
+    if (all == 0) return;
+    if (c > kEmitBig) {
+        const uint32_t at = atomicAdd(&a.big[0], 1u);
+        a.big[1 + 2 * at] = gp;
+        a.big[2 + 2 * at] = dst;
+        c = 0;
+    }
+    if (c) {
+        const TriSetup& r = a.recs[gp];
+        const float4* e4 = (const float4*)&r;
+        const float4 e0 = e4[0], e1 = e4[1], e2 = e4[2];
+        const int sh = a.tile_shift;
+        const uint32_t tx0 = (uint32_t)r.x0 >> sh, tx1 = (uint32_t)(r.x1 - 1) >> sh;
+        const uint32_t ty0 = (uint32_t)r.y0 >> sh;
+        s_dst[threadIdx.x] = dst;
+        s_key[threadIdx.x] = t.tile_base + ty0 * tiles_x + tx0;
+        s_w[threadIdx.x] = (tx1 - tx0 + 1) | (((r.draw_flags >> kPrimFlagShift) & (kPrimPoint | kPrimLine)) << kKindShift);
+        const int ox = (int)(tx0 << sh), oy = (int)(ty0 << sh);
+        s_box[threadIdx.x] = make_int4(r.x0 - ox, r.y0 - oy, r.x1 - ox, r.y1 - oy);
+        s_org[threadIdx.x] = make_int2(ox, oy);
+        s_edge[threadIdx.x][0] = e0;
+        s_edge[threadIdx.x][1] = e1;
+        s_edge[threadIdx.x][2] = e2;
+    }
+    uint32_t total;
+    s_off[threadIdx.x] = block_exclusive_scan(c, s_tmp, total);
+    if (threadIdx.x == 0) s_off[256] = total;
+    __syncthreads();
+    for (uint32_t j = threadIdx.x; j < total; j += 256u) {
+        // lo: the last primitive whose run starts at or before j (s_off is
+        // non-decreasing and s_off[0] = 0), in eight unrolled halvings
+        uint32_t lo = 0;
 #pragma unroll
-            for (uint32_t step = 128; step >= 1; step >>= 1)
-                if (s_off[lo + step] <= j) lo += step;
-            const uint32_t k = j - s_off[lo];
-            const uint32_t wl = s_w[lo];
-            const uint32_t w = wl & ((1u << kKindShift) - 1u), kind = wl >> kKindShift;
-            // row = k / w: k < kEmitBig = 2048 and w <= 2048, so (k + 1/2) / w
-            // is at least 1/(2w) from an integer while the product with
-            // v_rcp_f32's reciprocal (1 ulp) errs by under 1.5 * 2^-23 * 2049 / w
-            const uint32_t row = (uint32_t)(((float)k + 0.5f) * __builtin_amdgcn_rcpf((float)w));
-            const uint32_t out = s_dst[lo] + k;
-            if (out < a.cap) {
-                const uint32_t col = k - row * w;
-                a.keys[out] = s_key[lo] + row * s_tx[lo] + col;
-                const int2 org = s_org[lo];
-                const float4 e[3] = {s_edge[lo][0], s_edge[lo][1], s_edge[lo][2]};
-                float4 l = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                if (kind & kPrimLine) l = *(const float4*)&a.ext[blk * 256u + lo];
-                a.vals[out] = (blk * 256u + lo) |
-                              pair_blocks_covered(a.tile_shift, s_box[lo], col, row, kind, e, l, s_vp[lo], org.x, org.y);
-            }
+        for (uint32_t step = 128; step >= 1; step >>= 1)
+            if (s_off[lo + step] <= j) lo += step;
+        const uint32_t k = j - s_off[lo];
+        const uint32_t wl = s_w[lo];
+        const uint32_t w = wl & ((1u << kKindShift) - 1u), kind = wl >> kKindShift;
+        // row = k / w: k < kEmitBig = 2048 and w <= 2048, so (k + 1/2) / w
+        // is at least 1/(2w) from an integer while the product with
+        // v_rcp_f32's reciprocal (1 ulp) errs by under 1.5 * 2^-23 * 2049 / w
+        const uint32_t row = (uint32_t)(((float)k + 0.5f) * __builtin_amdgcn_rcpf((float)w));
+        const uint32_t out = s_dst[lo] + k;
+        if (out < a.cap) {
+            const uint32_t col = k - row * w;
+            a.keys[out] = s_key[lo] + row * tiles_x + col;
+            const int2 org = s_org[lo];
+            const float4 e[3] = {s_edge[lo][0], s_edge[lo][1], s_edge[lo][2]};
+            float4 l = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (kind & kPrimLine) l = *(const float4*)&a.ext[gp0 + lo];
+            a.vals[out] = (gp0 + lo) | pair_blocks_covered(a.tile_shift, s_box[lo], col, row, kind, e, l, vp, org.x, org.y);
         }
-        __syncthreads();
     }
 }
 
@@ -725,17 +732,17 @@ __global__ __launch_bounds__(256) void emit_big_kernel(EmitArgs a)
 {
     const uint32_t n = a.big[0];
     for (uint32_t b = blockIdx.x; b < n; b += gridDim.x) {
-        const uint32_t gp = a.big[1 + b];
+        const uint32_t gp = a.big[1 + 2 * b], off = a.big[2 + 2 * b];
         const TriSetup& r = a.recs[gp];
-        const TargetParams& t = a.targets[a.draws[r.draw_flags & kPrimDraw].target];
+        const DrawDesc& dd = a.draws[r.draw_flags & kPrimDraw];
+        const TargetParams& t = a.targets[dd.target];
         const int sh = a.tile_shift;
         const uint32_t tx0 = (uint32_t)r.x0 >> sh, tx1 = (uint32_t)(r.x1 - 1) >> sh;
         const uint32_t ty0 = (uint32_t)r.y0 >> sh;
         const uint32_t w = tx1 - tx0 + 1;
-        const uint32_t c = a.counts[gp], off = a.offsets[gp];
+        const uint32_t c = a.counts[gp];
         const int4 box = make_int4(r.x0 - (int)(tx0 << sh), r.y0 - (int)(ty0 << sh), r.x1 - (int)(tx0 << sh),
                                    r.y1 - (int)(ty0 << sh));
-        const DrawDesc& dd = a.draws[r.draw_flags & kPrimDraw];
         const float4* e4 = (const float4*)&r;
         const float4 e[3] = {e4[0], e4[1], e4[2]};
         const float4 vp = make_float4(dd.vp_w, dd.vp_h, dd.half_x, dd.half_y);
@@ -749,58 +756,109 @@ __global__ __launch_bounds__(256) void emit_big_kernel(EmitArgs a)
     }
 }
 
-// Pair count kept for sorting: the 64-bit scanned total clamped to the
-// capacity of the pair arrays; a larger total raises the overflow word, and
-// then the emit kernels write only the pairs below the capacity and the
-// raster kernel draws nothing.
-__global__ void clamp_pairs_kernel(const uint64_t* total, uint32_t cap, uint32_t* kept, uint32_t* overflow)
-{
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    const uint64_t t = *total;
-    *kept = t < (uint64_t)cap ? (uint32_t)t : cap;
-    if (t > (uint64_t)cap) *overflow = 1u;
-}
+// ----------------------------------------------------- small launches' lists
 
-// First index in [lo, hi) of the ascending keys whose tile is not before
-// t; hi when there is none.
-__device__ __forceinline__ uint32_t lower_bound_key(const uint32_t* keys, uint32_t lo, uint32_t hi, uint32_t t)
+struct SmallBinArgs {
+    const TriSetup* recs;
+    const LineExt* ext;
+    const DrawDesc* draws;
+    const TargetParams* targets;
+    uint32_t* vals;               // lists, target by target: tile i's from list_base + i * prim_count
+    uint2* range;                 // (first, last) of each tile's list
+    uint32_t tiles;
+    uint32_t target_count;
+    int32_t tile_shift;
+};
+
+__device__ __forceinline__ uint32_t target_of(const TargetParams* t, uint32_t n, uint32_t tile)
 {
-    while (lo < hi) {
+    uint32_t lo = 0, hi = n;
+    while (hi - lo > 1) {
         const uint32_t mid = (lo + hi) >> 1;
-        if (keys[mid] < t) lo = mid + 1; else hi = mid;
+        if (t[mid].tile_base <= tile) lo = mid; else hi = mid;
     }
     return lo;
 }
 
-// Start of every tile's range in the tile-sorted pair array, start[t] =
-// the first pair whose tile is not before t (start[tiles] = pair count).
-// A workgroup takes 256 consecutive tiles: two searches over all pairs bound
-// its tiles' ranges, and each thread searches only between them (empty
-// tiles cost nothing, however many a sparse frame has).  The pair count is
-// read on the device.
-__global__ __launch_bounds__(256) void tile_ranges_kernel(const uint32_t* keys, const uint32_t* n_ptr, uint32_t tiles, uint32_t* start)
+// The tile lists of a small launch, without pairs, sorts or scans: WAVES
+// wavefronts per tile (four tiles or one per workgroup) test every primitive
+// of the tile's target, 64 * WAVES at a time in order, and append the ones
+// whose box meets the tile, with the quarters they may cover.  Every list has
+// room for all of its target's primitives, so nothing can overflow and no
+// total goes back to the host.
+template <int WAVES>
+__global__ __launch_bounds__(256) void bin_small_kernel(SmallBinArgs a)
 {
-    __shared__ uint32_t s_lim[2];
-    const uint32_t t0 = blockIdx.x * 256u;
-    const uint32_t n = *n_ptr;
-    if (threadIdx.x < 2) s_lim[threadIdx.x] = lower_bound_key(keys, 0u, n, min(t0 + threadIdx.x * 256u, tiles + 1u));
-    __syncthreads();
-    const uint32_t t = t0 + threadIdx.x;
-    if (t <= tiles) start[t] = lower_bound_key(keys, s_lim[0], s_lim[1], t);
+    __shared__ uint32_t s_n[2][4];
+    constexpr uint32_t kStep = 64u * WAVES;
+    const uint32_t tile = WAVES == 1 ? blockIdx.x * 4u + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : blockIdx.x;
+    if (tile >= a.tiles) return;   // whole waves, and with WAVES = 1 none meets a barrier
+    const uint32_t me = WAVES == 1 ? threadIdx.x & 63u : threadIdx.x;
+    const TargetParams& t = *uniform_ptr(&a.targets[target_of(uniform_ptr(a.targets), a.target_count, tile)]);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int sh = a.tile_shift;
+    const uint32_t local = tile - t.tile_base;
+    const int tx = (int)(local % t.tiles_x), ty = (int)(local / t.tiles_x);
+    const int X = tx << sh, Y = ty << sh, side = 1 << sh;
+    const uint32_t end = t.prim_base + t.prim_count;
+    const uint32_t list = t.list_base + local * t.prim_count;
+    uint32_t n = 0;
+    auto box_of = [&](uint32_t gp) { return gp < end ? *(const int4*)&a.recs[gp].x0 : make_int4(0, 0, 0, 0); };
+    int4 next = box_of(t.prim_base + me);
+    int flip = 0;
+    for (uint32_t base = t.prim_base; base < end; base += kStep, flip ^= 1) {
+        const uint32_t gp = base + me;
+        const int4 box = next;
+        next = box_of(gp + kStep);   // in flight while this round is worked on
+        const bool hit = box.x < box.z && box.y < box.w && box.x < X + side && box.z > X && box.y < Y + side && box.w > Y;
+        const uint64_t m = __builtin_amdgcn_ballot_w64(hit);
+        uint32_t at = n;
+        if (WAVES == 1) {
+            n += (uint32_t)__popcll(m);
+        } else {
+            if (lane == 0) s_n[flip][wave] = (uint32_t)__popcll(m);
+            __syncthreads();   // two buffers: the next round's writes meet no reader of this one's
+#pragma unroll
+            for (int w = 0; w < 4; w++) {
+                const uint32_t c = s_n[flip][w];
+                if (w < wave) at += c;
+                n += c;
+            }
+        }
+        if (hit) {
+            const TriSetup& r = a.recs[gp];
+            const DrawDesc& d = a.draws[r.draw_flags & kPrimDraw];
+            const uint32_t kind = (r.draw_flags >> kPrimFlagShift) & (kPrimPoint | kPrimLine);
+            const float4* e4 = (const float4*)&r;
+            const float4 e[3] = {e4[0], e4[1], e4[2]};
+            const float4 l = (kind & kPrimLine) ? *(const float4*)&a.ext[gp] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            const float4 vp = make_float4(d.vp_w, d.vp_h, d.half_x, d.half_y);
+            // the tile as the first of its own rectangle
+            const int4 rel = make_int4(box.x - X, box.y - Y, box.z - X, box.w - Y);
+            a.vals[list + at + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] =
+                gp | pair_blocks_covered(sh, rel, 0u, 0u, kind, e, l, vp, X, Y);
+        }
+    }
+    if (me == 0) a.range[tile] = make_uint2(list, list + n);
 }
 
 // ---------------------------------------------------------- radix sort
 
-// A pass sorts by an 8-bit digit.  The pair array is cut into kSortSegments
-// contiguous segments, one per workgroup; the histogram kernel counts each
-// segment's digits, a scan over (digit, segment) turns the counts into
-// output bases, and the scatter kernel walks its segment in order in tiles
-// of kSortTile items.  Each wave ranks its quarter of a tile (64-item
-// rounds, equal digits ranked with ballots), the workgroup orders the tile
-// by digit in LDS -- stable: by wave, then round, then lane, which is the
-// items' order -- and the sorted tile is written out with consecutive
-// threads on consecutive positions of each digit's run, so the stores of a
-// run coalesce instead of scattering one item per digit bucket.
+// A pass sorts by an 8-bit digit in three kernels.  The pair array is cut
+// into kSortSegments contiguous segments, one per workgroup; the histogram
+// kernel counts each segment's digits, the offsets kernel scans every digit's
+// counts over the segments (one workgroup per digit) and keeps the digit's
+// total, and the scatter kernel, which scans the 256 totals by itself, walks
+// its segment in order in tiles of kSortTile items.  Each wave ranks its
+// quarter of a tile (64-item rounds, equal digits ranked with ballots), the
+// workgroup orders the tile by digit in LDS -- stable: by wave, then round,
+// then lane, which is the items' order -- and the sorted tile is written out
+// with consecutive threads on consecutive positions of each digit's run, so
+// the stores of a run coalesce instead of scattering one item per digit
+// bucket.  The last pass over the tile keys leaves every tile's range too:
+// a digit's run holds a segment's items in key order (the earlier passes
+// sorted them), so a tile's items form runs whose ends it takes the minimum
+// and maximum of.
 constexpr int kSortSegments = 1024;
 constexpr int kSortThreads = 256;
 constexpr int kSortWaves = kSortThreads / 64;
@@ -814,9 +872,14 @@ __device__ __forceinline__ void segment_range(uint32_t n, uint32_t seg, uint32_t
     e = min(n, b + per);
 }
 
+// ranges, when given, are emptied (first = 2^32 - 1, last = 0) for the pass
+// that will fill them.
 __global__ __launch_bounds__(kSortThreads) void radix_hist_kernel(const uint32_t* keys, const uint32_t* n_ptr, int shift,
-                                                                 uint32_t* hist)
+                                                                 uint32_t* hist, uint2* ranges, uint32_t tiles)
 {
+    if (ranges)
+        for (uint32_t i = blockIdx.x * kSortThreads + threadIdx.x; i < tiles; i += kSortSegments * kSortThreads)
+            ranges[i] = make_uint2(0xFFFFFFFFu, 0u);
     __shared__ uint32_t s_cnt[kSortWaves][256];
     const int wave = threadIdx.x >> 6;
 #pragma unroll
@@ -843,21 +906,39 @@ __global__ __launch_bounds__(kSortThreads) void radix_hist_kernel(const uint32_t
     hist[threadIdx.x * kSortSegments + blockIdx.x] = c;
 }
 
+// Exclusive scan of one digit's counts over the segments, in place, and the
+// digit's total; one workgroup per digit.
+__global__ __launch_bounds__(kSortThreads) void radix_offsets_kernel(uint32_t* hist, uint32_t* totals)
+{
+    constexpr int kPer = kSortSegments / kSortThreads;
+    __shared__ uint32_t s_tmp[kSortWaves];
+    uint4* row = (uint4*)(hist + (uint64_t)blockIdx.x * kSortSegments) + threadIdx.x;
+    static_assert(kPer == 4, "a thread takes one uint4 of its digit's row");
+    const uint4 v = *row;
+    uint32_t total;
+    const uint32_t run = block_exclusive_scan(v.x + v.y + v.z + v.w, s_tmp, total);
+    *row = make_uint4(run, run + v.x, run + v.x + v.y, run + v.x + v.y + v.z);
+    if (threadIdx.x == 0) totals[blockIdx.x] = total;
+}
+
 __global__ __launch_bounds__(kSortThreads) void radix_scatter_kernel(const uint32_t* keys_in, const uint32_t* vals_in,
                                                                     uint32_t* keys_out, uint32_t* vals_out,
-                                                                    const uint32_t* n_ptr, int shift, const uint32_t* base)
+                                                                    const uint32_t* n_ptr, int shift, const uint32_t* base,
+                                                                    const uint32_t* totals, uint2* ranges, uint32_t tiles)
 {
     __shared__ uint32_t s_cnt[kSortWaves][256];   // a wave's items per digit, then the wave's offset in the digit's run
     __shared__ uint32_t s_start[256];             // where a digit's run starts in the sorted tile
     __shared__ uint32_t s_run[256];               // the segment's next output position per digit
     __shared__ uint32_t s_keys[kSortTile], s_vals[kSortTile];
-    __shared__ uint64_t s_tmp[kSortWaves];
+    __shared__ uint32_t s_tmp[kSortWaves];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const uint32_t d_me = threadIdx.x;            // the digit this thread keeps the books of
-    s_run[d_me] = base[d_me * kSortSegments + blockIdx.x];
     uint32_t b, e;
     const uint32_t n_total = *n_ptr;
     segment_range(n_total, blockIdx.x, b, e);
+    if (b >= e) return;   // the whole workgroup
+    uint32_t items;
+    s_run[d_me] = block_exclusive_scan(totals[d_me], s_tmp, items) + base[d_me * kSortSegments + blockIdx.x];
     const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
     for (uint32_t t0 = b; t0 < e; t0 += (uint32_t)kSortTile) {
 #pragma unroll
@@ -901,8 +982,8 @@ __global__ __launch_bounds__(kSortThreads) void radix_scatter_kernel(const uint3
             s_cnt[w][d_me] = total;
             total += c;
         }
-        uint64_t tile_n;
-        const uint32_t start = (uint32_t)block_exclusive_scan64(total, s_tmp, tile_n);
+        uint32_t tile_n;
+        const uint32_t start = block_exclusive_scan(total, s_tmp, tile_n);
         s_start[d_me] = start;
         __syncthreads();
         // the tile in digit order, in LDS
@@ -920,13 +1001,17 @@ __global__ __launch_bounds__(kSortThreads) void radix_scatter_kernel(const uint3
 #pragma unroll
         for (int r = 0; r < kSortRounds; r++) {
             const uint32_t p = (uint32_t)r * kSortThreads + threadIdx.x;
-            if (p < (uint32_t)tile_n) {
+            if (p < tile_n) {
                 const uint32_t key = s_keys[p];
                 const uint32_t dg = (key >> shift) & 255u;
                 const uint32_t dst = s_run[dg] + (p - s_start[dg]);
                 if (dst < n_total) {
-                    keys_out[dst] = key;
+                    if (keys_out) keys_out[dst] = key;
                     vals_out[dst] = s_vals[p];
+                    if (ranges && key < tiles) {
+                        if (p == 0 || s_keys[p - 1] != key) atomicMin(&ranges[key].x, dst);
+                        if (p + 1 == tile_n || s_keys[p + 1] != key) atomicMax(&ranges[key].y, dst + 1u);
+                    }
                 }
             }
         }

@@ -59,7 +59,7 @@ enum : uint32_t {
 // immediate render calls; a recorded batch owns its own so that replaying
 // it never reallocates.
 struct Buffers {
-    DevBuf vout, recs, counts, offsets, keys[2], vals[2], tile_start, hist, hist_base, sums, big;
+    DevBuf vout, recs, counts, keys[2], vals[2], tile_range, hist, digit_totals, sums, big;
     DevBuf arena, stats, traces, features, pred, okeys[2], ovals[2], line_ext;
     void release_all();
 };

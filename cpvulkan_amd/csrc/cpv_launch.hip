@@ -3,8 +3,9 @@
 // A render call becomes, per run of draws that share a shader program, one
 // launch of each stage on the context's stream:
 //   vertex kernel -> setup kernel -> scan -> emit -> radix sort by tile ->
-//   tile ranges -> [tile features -> cost prediction -> queue order] ->
-//   raster kernel
+//   [tile features -> cost prediction -> queue order] -> raster kernel
+// or, for small launches (LaunchPlan::small),
+//   vertex kernel -> setup kernel -> tile lists -> raster kernel
 // The raster kernel fuses the render pass clear (loadOp CLEAR) into its tile
 // initialisation, so a frame touches each framebuffer byte once on the way
 // in (LOAD only) and once on the way out.
@@ -72,8 +73,59 @@ struct LaunchPlan {
     int32_t hiz_op = -1, hiz_kind = 32;
     int32_t less_depth = 0;          // RasterArgs::less_depth
     int32_t uniform_fstate = -1;     // every draw's fragment state is fstates[0] (0), or not (-1)
+    // Small launches take bin_small_kernel in place of the scan, emit and sort
+    // kernels: the tiles' lists, each with room for every primitive of its
+    // target, then hold small_entries words.
+    bool small = false;
+    uint32_t small_entries = 0;
     size_t o_env = 0, o_dd = 0, o_fs = 0, o_tp = 0, o_vb = 0, o_sb = 0;   // offsets in the arena
 };
+
+// Whether a launch is small: each tile's workgroup can test every primitive
+// of the tile's target itself (bin_small_kernel), in the place of the nine
+// kernels that scan, emit and sort pairs, whose launches and latencies alone
+// are 40 to 60 us of a call.
+//
+// The line, by back-to-back calls with one path or the other on every size
+// (us, lists against pairs): at 640x480 64 against 88 for 500 triangles, 61
+// against 83 for 4,000, 86 against 87 for 8,000 and 145 against 97 for
+// 16,000; at 1920x1080 68 against 83 for 1,000, 98 against 86 for 2,000; at
+// 3840x2160 121 against 103 for 500.  The lists cost about 60 us per 2^24
+// (tile, primitive) tests.  With 8x8 tiles the two meet at 2^24 (91 against 88
+// for 500 triangles at 1920x1080, 60 against 87 for 250); their line is 2^22,
+// so that launches of viewport-sized triangles keep to pairs and their
+// capacity checks (the redraw tests draw 600 of them over 8,160 tiles).
+constexpr uint32_t kSmallEntries = 1u << 23;
+constexpr uint32_t kSmallEntries8 = 1u << 22;
+constexpr uint32_t kSmallPrims = 4096;
+constexpr uint32_t kSmallWavePrims = 256;   // up to this many per target, one wavefront per tile
+
+void plan_small(const cpv_config& cfg, LaunchPlan* P)
+{
+    P->small = false;
+    P->small_entries = 0;
+    for (TargetParams& t : P->targets) t.prim_base = t.prim_count = t.list_base = 0;
+    // a target's primitives: those of its draws, which are consecutive
+    bool runs = true;
+    for (size_t i = 0; i < P->dd.size(); i++) {
+        TargetParams& t = P->targets[P->dd[i].target];
+        if (t.prim_count == 0) t.prim_base = P->dd[i].prim_base;
+        else runs = runs && t.prim_base + t.prim_count == P->dd[i].prim_base;
+        t.prim_count += P->dd[i].prim_count;
+    }
+    uint64_t entries = 0;
+    uint32_t most = 0;
+    for (TargetParams& t : P->targets) {
+        t.list_base = (uint32_t)std::min<uint64_t>(entries, UINT32_MAX);
+        entries += (uint64_t)t.tiles_x * t.tiles_y * t.prim_count;
+        most = std::max(most, t.prim_count);
+    }
+    if (!runs || entries > (P->tile_shift == 3 ? kSmallEntries8 : kSmallEntries) || most > kSmallPrims) return;
+    // cost traces and the learned order read the general path's statistics
+    if (cfg.record_costs || cfg.scheduler == CPV_SCHED_PREDICTED) return;
+    P->small = true;
+    P->small_entries = (uint32_t)entries;
+}
 
 int plan_launch(const cpv_config& cfg, const Program& prog, const std::vector<TargetParams>& targets,
                 const std::vector<LaunchDraw>& lds, const std::vector<cpv_pass_desc>& passes,
@@ -219,6 +271,7 @@ int plan_launch(const cpv_config& cfg, const Program& prog, const std::vector<Ta
             P->less_depth = fs[0].depth_compare == CPV_COMPARE_LESS || fs[0].depth_compare == CPV_COMPARE_LESS_OR_EQUAL;
         }
     }
+    plan_small(cfg, P);
     P->uniform_fstate = P->fstates.empty() ? -1 : 0;
     for (const FragmentState& f : P->fstates)
         if (std::memcmp(&f, &P->fstates[0], sizeof(f)) != 0) P->uniform_fstate = -1;
@@ -259,42 +312,27 @@ struct Exec {
     uint32_t* overflow = nullptr; // overflow word shared by several launches (nullptr: the launch's own)
     unsigned long long* fragments = nullptr;   // covered-fragment counter (nullptr: the launch's own)
     const uint32_t* fixed_order = nullptr;     // learned tile order computed earlier (nullptr: computed here)
+    uint32_t* host_total = nullptr;            // pinned host words that receive the pair total and the overflow flag
 };
 
-// Exclusive scan of n counts into out (out[n] = the total when write_total);
-// total64, when given, receives the total in 64 bits.
-int scan_u32(Exec& x, const uint32_t* in, uint32_t n, uint32_t* out, bool write_total, uint64_t* total64 = nullptr)
-{
-    if (n == 0) {
-        if (write_total) fill_u32(x.s, out, 0u, 1);
-        if (total64) fill_u32(x.s, total64, 0u, 2);
-        return CPV_OK;
-    }
-    const uint32_t blocks = (n + kScanTile - 1) / kScanTile;
-    if (x.b->sums.ensure((size_t)blocks * 8, x.frozen)) return CPV_ERROR_OUT_OF_MEMORY;
-    uint64_t* sums = x.b->sums.as<uint64_t>();
-    hipLaunchKernelGGL(scan_reduce_kernel, dim3(blocks), dim3(kScanThreads), 0, x.s, in, n, sums);
-    hipLaunchKernelGGL(scan_sums_kernel, dim3(1), dim3(kScanThreads), 0, x.s, sums, blocks, total64);
-    hipLaunchKernelGGL(scan_down_kernel, dim3(blocks), dim3(kScanThreads), 0, x.s, in, n, (const uint64_t*)sums, out,
-                       write_total ? 1 : 0);
-    HIP_TRY(hipGetLastError());
-    return CPV_OK;
-}
-
-// Stable LSD radix sort of (key, value) pairs by the low `bits` key bits;
-// n is read on the device.  Returns the buffer index holding the result.
-int radix_sort(Exec& x, DevBuf* keys, DevBuf* vals, const uint32_t* d_n, int bits, int* result)
+// Stable LSD radix sort of (key, value) pairs by the low `bits` key bits
+// (one pass at least); n is read on the device.  ranges, when given, receive
+// every key's range of the sorted pairs (`keys_n` of them).  The sorted keys
+// themselves are not written.  Returns the buffer index of the sorted values.
+int radix_sort(Exec& x, DevBuf* keys, DevBuf* vals, const uint32_t* d_n, int bits, uint2* ranges, uint32_t keys_n, int* result)
 {
     Buffers& b = *x.b;
     int src = 0;
-    for (int shift = 0; shift < bits; shift += 8) {
-        hipLaunchKernelGGL(radix_hist_kernel, dim3(kSortSegments), dim3(kSortThreads), 0, x.s,
-                           (const uint32_t*)keys[src].p, d_n, shift, b.hist.as<uint32_t>());
-        int rc = scan_u32(x, b.hist.as<uint32_t>(), 256u * kSortSegments, b.hist_base.as<uint32_t>(), false);
-        if (rc) return rc;
+    for (int shift = 0; shift == 0 || shift < bits; shift += 8) {
+        const bool last = shift + 8 >= bits;
+        hipLaunchKernelGGL(radix_hist_kernel, dim3(kSortSegments), dim3(kSortThreads), 0, x.s, (const uint32_t*)keys[src].p, d_n,
+                           shift, b.hist.as<uint32_t>(), last ? ranges : nullptr, keys_n);
+        hipLaunchKernelGGL(radix_offsets_kernel, dim3(256), dim3(kSortThreads), 0, x.s, b.hist.as<uint32_t>(),
+                           b.digit_totals.as<uint32_t>());
         hipLaunchKernelGGL(radix_scatter_kernel, dim3(kSortSegments), dim3(kSortThreads), 0, x.s,
-                           (const uint32_t*)keys[src].p, (const uint32_t*)vals[src].p, keys[1 - src].as<uint32_t>(),
-                           vals[1 - src].as<uint32_t>(), d_n, shift, (const uint32_t*)b.hist_base.p);
+                           (const uint32_t*)keys[src].p, (const uint32_t*)vals[src].p, last ? nullptr : keys[1 - src].as<uint32_t>(),
+                           vals[1 - src].as<uint32_t>(), d_n, shift, (const uint32_t*)b.hist.p, (const uint32_t*)b.digit_totals.p,
+                           last ? ranges : nullptr, keys_n);
         HIP_TRY(hipGetLastError());
         src = 1 - src;
     }
@@ -329,14 +367,6 @@ int resident_workgroups(Exec& x, const KernelRef& k, int block)
     return per_cu * std::max(x.ctx->cu_count, 1);
 }
 
-// Slab sums of the scans of a launch: the primitive counts' and the radix
-// sorts' histogram scans (256 digits x kSortSegments segments).
-size_t scan_sums_bytes(uint32_t prims)
-{
-    const size_t most = std::max<size_t>(prims, (size_t)256 * kSortSegments);
-    return (most + kScanTile - 1) / kScanTile * 8;
-}
-
 // Buffers whose size depends only on the plan.
 int ensure_front(Exec& x, const LaunchPlan& P)
 {
@@ -344,8 +374,8 @@ int ensure_front(Exec& x, const LaunchPlan& P)
     const bool f = x.frozen;
     if (b.vout.ensure((size_t)std::max(P.vout_total, 1u) * P.stride * 4, f) ||
         b.recs.ensure((size_t)std::max(P.prim_total, 1u) * sizeof(TriSetup), f) ||
-        b.counts.ensure((size_t)std::max(P.prim_total, 1u) * 4, f) || b.offsets.ensure(((size_t)P.prim_total + 1) * 4, f) ||
-        b.stats.ensure(kStatAlloc * 4, f) || b.sums.ensure(scan_sums_bytes(P.prim_total), f))
+        b.counts.ensure((size_t)std::max(P.prim_total, 1u) * 4, f) || b.stats.ensure(kStatAlloc * 4, f) ||
+        b.sums.ensure(P.sblock.size() * 8, f) || b.big.ensure(((size_t)P.prim_total * 2 + 1) * 4, f))
         return CPV_ERROR_OUT_OF_MEMORY;
     if (P.lines && b.line_ext.ensure((size_t)std::max(P.prim_total, 1u) * sizeof(LineExt), f)) return CPV_ERROR_OUT_OF_MEMORY;
     return CPV_OK;
@@ -358,9 +388,10 @@ int ensure_back(Exec& x, const LaunchPlan& P, uint32_t pair_cap)
     const bool f = x.frozen;
     const size_t pairs = (size_t)std::max(pair_cap, 1u) * 4;
     const size_t tiles = (size_t)std::max(P.tiles, 1u);
+    if (b.tile_range.ensure(tiles * 8, f)) return CPV_ERROR_OUT_OF_MEMORY;
+    if (P.small) return b.vals[0].ensure((size_t)std::max(P.small_entries, 1u) * 4, f) ? CPV_ERROR_OUT_OF_MEMORY : CPV_OK;
     if (b.keys[0].ensure(pairs, f) || b.keys[1].ensure(pairs, f) || b.vals[0].ensure(pairs, f) || b.vals[1].ensure(pairs, f) ||
-        b.tile_start.ensure((tiles + 1) * 4, f) || b.hist.ensure((size_t)256 * kSortSegments * 4, f) ||
-        b.hist_base.ensure(((size_t)256 * kSortSegments + 1) * 4, f) || b.big.ensure(((size_t)P.prim_total + 1) * 4, f))
+        b.hist.ensure((size_t)256 * kSortSegments * 4, f) || b.digit_totals.ensure(256 * 4, f))
         return CPV_ERROR_OUT_OF_MEMORY;
     if (needs_features(x)) {
         if (b.features.ensure(tiles * kFeatureStride * 4, f) || b.pred.ensure(tiles * 4, f) || b.okeys[0].ensure(tiles * 4, f) ||
@@ -371,13 +402,15 @@ int ensure_back(Exec& x, const LaunchPlan& P, uint32_t pair_cap)
     return CPV_OK;
 }
 
-// Vertex stage, triangle setup and the pair-count scan; the pair total is
-// left at offsets[prim_total].
-int enqueue_front(Exec& x, const LaunchPlan& P, uint8_t* arena)
+// Vertex stage, triangle setup and, unless the launch is small, the scan of
+// the pair counts; the pair total, and what of it fits pair_cap, are left in
+// the control words.
+int enqueue_front(Exec& x, const LaunchPlan& P, uint8_t* arena, uint32_t pair_cap)
 {
     int rc = ensure_front(x, P);
     if (rc) return rc;
     Buffers& b = *x.b;
+    uint32_t* stats = b.stats.as<uint32_t>();
     const DrawDesc* d_dd = (const DrawDesc*)(arena + P.o_dd);
     const TargetParams* d_tp = (const TargetParams*)(arena + P.o_tp);
     if (P.vout_total > 0) {
@@ -386,12 +419,17 @@ int enqueue_front(Exec& x, const LaunchPlan& P, uint8_t* arena)
     }
     if (P.prim_total > 0) {
         SetupArgs sa{d_dd, (const uint32_t*)(arena + P.o_sb), d_tp, b.vout.as<float>(), b.recs.as<TriSetup>(),
-                     P.lines ? b.line_ext.as<LineExt>() : nullptr, b.counts.as<uint32_t>(), P.stride, P.tile_shift};
+                     P.lines ? b.line_ext.as<LineExt>() : nullptr, b.counts.as<uint32_t>(), b.sums.as<uint64_t>(), P.stride, P.tile_shift};
         hipLaunchKernelGGL(setup_kernel, dim3((uint32_t)P.sblock.size()), dim3(256), 0, x.s, sa);
         HIP_TRY(hipGetLastError());
     }
-    return scan_u32(x, b.counts.as<uint32_t>(), P.prim_total, b.offsets.as<uint32_t>(), true,
-                    (uint64_t*)(b.stats.as<uint32_t>() + kStatPairTotal));
+    if (P.small) return CPV_OK;
+    ScanArgs ca{b.sums.as<uint64_t>(), P.prim_total ? (uint32_t)P.sblock.size() : 0u, std::max(pair_cap, 1u),
+                (uint64_t*)(stats + kStatPairTotal), stats + kStatPairs, x.overflow ? x.overflow : stats + kStatOverflow,
+                b.big.as<uint32_t>(), x.host_total};
+    hipLaunchKernelGGL(scan_blocks_kernel, dim3(1), dim3(kScanThreads), 0, x.s, ca);
+    HIP_TRY(hipGetLastError());
+    return CPV_OK;
 }
 
 // Where the binning stage left its results for the raster kernel.
@@ -412,30 +450,37 @@ int enqueue_bin(Exec& x, const LaunchPlan& P, uint8_t* arena, uint32_t pair_cap,
     const DrawDesc* d_dd = (const DrawDesc*)(arena + P.o_dd);
     const FragmentState* d_fs = (const FragmentState*)(arena + P.o_fs);
     const TargetParams* d_tp = (const TargetParams*)(arena + P.o_tp);
+    uint2* ranges = b.tile_range.as<uint2>();
+    if (P.small) {
+        SmallBinArgs sb{b.recs.as<TriSetup>(), P.lines ? b.line_ext.as<LineExt>() : nullptr, d_dd, d_tp, b.vals[0].as<uint32_t>(),
+                        ranges, P.tiles, (uint32_t)P.targets.size(), P.tile_shift};
+        uint32_t most = 0;
+        for (const TargetParams& t : P.targets) most = std::max(most, t.prim_count);
+        if (P.tiles && most <= kSmallWavePrims)
+            hipLaunchKernelGGL(bin_small_kernel<1>, dim3((P.tiles + 3) / 4), dim3(256), 0, x.s, sb);
+        else if (P.tiles)
+            hipLaunchKernelGGL(bin_small_kernel<4>, dim3(P.tiles), dim3(256), 0, x.s, sb);
+        HIP_TRY(hipGetLastError());
+        out->src = 0;
+        out->order = nullptr;
+        return CPV_OK;
+    }
     const uint32_t cap = std::max(pair_cap, 1u);
-    hipLaunchKernelGGL(clamp_pairs_kernel, dim3(1), dim3(64), 0, x.s, (const uint64_t*)(stats + kStatPairTotal), cap,
-                       stats + kStatPairs, x.overflow ? x.overflow : stats + kStatOverflow);
     // emit pairs in primitive order
     if (P.prim_total) {
-        fill_u32(x.s, b.big.p, 0u, 1);
-        EmitArgs ea{b.recs.as<TriSetup>(), P.lines ? b.line_ext.as<LineExt>() : nullptr, b.counts.as<uint32_t>(), b.offsets.as<uint32_t>(), d_dd, d_tp, b.keys[0].as<uint32_t>(),
-                    b.vals[0].as<uint32_t>(), b.big.as<uint32_t>(), P.prim_total, P.tile_shift, cap};
-        const uint32_t blocks = std::min<uint32_t>((P.prim_total + 255) / 256, 8192);
-        hipLaunchKernelGGL(emit_kernel, dim3(blocks), dim3(256), 0, x.s, ea);
+        EmitArgs ea{b.recs.as<TriSetup>(), P.lines ? b.line_ext.as<LineExt>() : nullptr, b.counts.as<uint32_t>(), b.sums.as<uint64_t>(),
+                    (const uint32_t*)(arena + P.o_sb), d_dd, d_tp, b.keys[0].as<uint32_t>(), b.vals[0].as<uint32_t>(),
+                    b.big.as<uint32_t>(), P.tile_shift, cap};
+        hipLaunchKernelGGL(emit_kernel, dim3((uint32_t)P.sblock.size()), dim3(256), 0, x.s, ea);
         hipLaunchKernelGGL(emit_big_kernel, dim3(1024), dim3(256), 0, x.s, ea);
         HIP_TRY(hipGetLastError());
     }
-    // stable radix sort of the pairs by tile
+    // stable radix sort of the pairs by tile, which leaves the tiles' ranges
     int src = 0;
-    if (P.tiles > 1) {
-        int bits = 0;
-        while ((1u << bits) < P.tiles) bits++;
-        rc = radix_sort(x, b.keys, b.vals, stats + kStatPairs, bits, &src);
-        if (rc) return rc;
-    }
-    hipLaunchKernelGGL(tile_ranges_kernel, dim3(P.tiles / 256 + 1), dim3(256), 0, x.s, (const uint32_t*)b.keys[src].p,
-                       (const uint32_t*)(stats + kStatPairs), P.tiles, b.tile_start.as<uint32_t>());
-    HIP_TRY(hipGetLastError());
+    int bits = 0;
+    while ((1u << bits) < P.tiles) bits++;
+    rc = radix_sort(x, b.keys, b.vals, stats + kStatPairs, bits, ranges, P.tiles, &src);
+    if (rc) return rc;
 
     // scheduling (a recorded batch computes its learned order once, when it
     // is recorded, and its submits reuse it)
@@ -443,7 +488,7 @@ int enqueue_bin(Exec& x, const LaunchPlan& P, uint8_t* arena, uint32_t pair_cap,
     const uint32_t* order = nullptr;
     const bool reuse_order = sched == CPV_SCHED_PREDICTED && x.fixed_order;
     if (needs_features(x) && P.tiles && !(reuse_order && !x.cfg.record_costs)) {
-        FeatureArgs fa{b.recs.as<TriSetup>(), b.vals[src].as<uint32_t>(), b.tile_start.as<uint32_t>(), d_tp, d_dd, d_fs,
+        FeatureArgs fa{b.recs.as<TriSetup>(), b.vals[src].as<uint32_t>(), ranges, d_tp, d_dd, d_fs,
                        b.features.as<float>(), P.tiles, (uint32_t)P.targets.size(), (int32_t)x.cfg.tile_size,
                        (int32_t)x.cfg.waves_per_tile, P.hiz_op >= 0 ? 1 : 0, 0};
         hipLaunchKernelGGL(tile_features_kernel, dim3((P.tiles + 3) / 4), dim3(256), 0, x.s, fa);
@@ -464,7 +509,7 @@ int enqueue_bin(Exec& x, const LaunchPlan& P, uint8_t* arena, uint32_t pair_cap,
         HIP_TRY(hipGetLastError());
         fill_u32(x.s, stats + kStatTiles, P.tiles, 1);
         int osrc = 0;
-        rc = radix_sort(x, b.okeys, b.ovals, stats + kStatTiles, 16, &osrc);
+        rc = radix_sort(x, b.okeys, b.ovals, stats + kStatTiles, 16, nullptr, 0, &osrc);
         if (rc) return rc;
         order = b.ovals[osrc].as<uint32_t>();
     }
@@ -489,7 +534,7 @@ int enqueue_raster(Exec& x, const LaunchPlan& P, uint8_t* arena, const Binned& b
     RasterArgs ra{};
     ra.recs = b.recs.as<TriSetup>();
     ra.tile_prims = b.vals[src].as<uint32_t>();
-    ra.tile_start = b.tile_start.as<uint32_t>();
+    ra.tile_range = b.tile_range.as<uint2>();
     ra.targets = d_tp;
     ra.draws = d_dd;
     ra.fstates = d_fs;
@@ -569,11 +614,12 @@ namespace {
 
 // Enqueues an immediate launch in its buffer set with the context's pair
 // capacity (at least 16 pairs per primitive and 1M): the descriptors'
-// upload, the front half (vertex, setup, binning) and the read-back of the
-// 64-bit pair total and overflow word on front_stream, then the raster
-// kernel on the context's stream after it.  The next call on the context
-// checks the pair count (resolve_pending): no host round trip sits between
-// a launch's binning and its raster kernel.  The front half waits for the
+// upload and the front half (vertex, setup, binning) on front_stream, whose
+// scan writes the 64-bit pair total and the overflow flag into host memory,
+// then the raster kernel on the context's stream after it.  The next call on
+// the context checks the pair count (resolve_pending): no host round trip
+// sits between a launch's binning and its raster kernel.  A small launch has
+// no pair count to check.  The front half waits for the
 // raster kernel that last used the set and, unless the previous context
 // call was a launch too, for all work enqueued on the context's stream; so
 // back-to-back launches run one front half under the previous raster.
@@ -603,18 +649,18 @@ int enqueue_checked(cpv_context* c, PendingLaunch& L)
     x.cfg = L.cfg;
     x.s = fs;
     x.fragments = (unsigned long long*)(c->buf.stats.as<uint32_t>() + kStatFragments);
-    rc = enqueue_front(x, L.P, arena);
-    if (rc) return rc;
     const uint64_t want = std::max<uint64_t>(c->pair_cap, 16ull * L.P.prim_total + (1u << 20));
-    const uint32_t cap = (uint32_t)std::min<uint64_t>(want, UINT32_MAX);
+    const uint32_t cap = L.P.small ? 0u : (uint32_t)std::min<uint64_t>(want, UINT32_MAX);
+    // the scan hands the host the pair total; it can check the launch from
+    // there on, while the pairs are still emitted and sorted
+    x.host_total = c->readback + 32;
+    rc = enqueue_front(x, L.P, arena, cap);
+    if (rc) return rc;
+    if (!L.P.small) HIP_TRY(hipEventRecord(c->ev_check, fs));
     Binned bn;
     rc = enqueue_bin(x, L.P, arena, cap, &bn);
     if (rc) return rc;
     c->pair_cap = std::max<uint64_t>(c->pair_cap, cap);
-    uint32_t* stats = B.stats.as<uint32_t>();
-    HIP_TRY(hipMemcpyAsync(c->readback + 32, stats + kStatPairTotal, 8, hipMemcpyDeviceToHost, fs));
-    HIP_TRY(hipMemcpyAsync(c->readback + 34, stats + kStatOverflow, 4, hipMemcpyDeviceToHost, fs));
-    HIP_TRY(hipEventRecord(c->ev_check, fs));
     HIP_TRY(hipEventRecord(c->set_front_done[L.set], fs));
     HIP_TRY(hipStreamWaitEvent(c->stream, c->set_front_done[L.set], 0));
     x.s = c->stream;
@@ -641,7 +687,11 @@ int enqueue_checked(cpv_context* c, PendingLaunch& L)
 // created).  Every call on a GPU shares that GPU's array: calls that overlap
 // on one GPU, from two contexts or two threads, race.
 
-constexpr size_t kScratchBytes = 64ull << 20;
+// Room for the passes that the entry point's 64 MiB limit admits
+// (carve_scratch) with their tiles' ranges, two words for each of at most
+// 2^22 tiles where the limit counts one.
+constexpr size_t kScratchLimit = 64ull << 20;
+constexpr size_t kScratchBytes = kScratchLimit + (16ull << 20);
 
 static __device__ __align__(256) uint8_t scratch[kScratchBytes];
 
@@ -669,10 +719,40 @@ namespace {
 // Places every buffer of launch P in the scratch array at base, with the
 // sizes ensure_front and ensure_back ask for: the control words first (at
 // the same address for every launch), then the descriptors, vertex outputs,
-// records, scans and tile ranges; the four pair arrays share what is left
-// and *pair_cap receives their capacity.  Touches no memory.
+// records, scans and tile ranges, then the four pair arrays, of *pair_cap
+// entries each.  Touches no memory.
+//
+// What is refused, and the pair capacity, follow from the entry point's limit:
+// 64 MiB for the control words, descriptors, vertex outputs, records, four
+// words per primitive and line extension, a word per tile, 2 MiB of sort
+// tables, and the pairs (16 bytes each) in what is left.  The buffers placed
+// here never take more than that beside the ranges' second words.
 int carve_scratch(uint8_t* base, const LaunchPlan& P, size_t arena_bytes, Buffers* b, uint32_t* pair_cap)
 {
+    const size_t prims = std::max(P.prim_total, 1u), tiles = std::max(P.tiles, 1u);
+    const size_t vout = (size_t)std::max(P.vout_total, 1u) * P.stride * 4, arena = std::max<size_t>(arena_bytes, 256);
+    size_t limit = 0;
+    auto count = [&](size_t bytes) { limit = ((limit + 255) & ~(size_t)255) + bytes; };
+    count(kStatAlloc * 4);
+    count(arena);
+    count(vout);
+    count(prims * sizeof(TriSetup));
+    count(prims * 4);
+    count(((size_t)P.prim_total + 1) * 4);
+    const size_t scanned = std::max<size_t>(P.prim_total, (size_t)256 * kSortSegments);
+    count((scanned + 4095) / 4096 * 8);
+    if (P.lines) count(prims * sizeof(LineExt));
+    count((tiles + 1) * 4);
+    count((size_t)256 * kSortSegments * 4);
+    count(((size_t)256 * kSortSegments + 1) * 4);
+    count(((size_t)P.prim_total + 1) * 4);
+    // each pair array starts on a 256-byte boundary: at most 4 x 255 bytes of padding
+    const size_t left = limit + 1024 < kScratchLimit ? kScratchLimit - limit - 1024 : 0;
+    const uint64_t cap = std::min<uint64_t>(left / 16, UINT32_MAX);
+    if (cap == 0)
+        return fail(CPV_ERROR_UNSUPPORTED,
+                    "a launch of %u primitives over %u tiles needs more than the %zu MiB of the allocation-free entry point",
+                    P.prim_total, P.tiles, kScratchLimit >> 20);
     size_t at = 0;
     auto take = [&](DevBuf& d, size_t bytes) {
         at = (at + 255) & ~(size_t)255;
@@ -680,27 +760,19 @@ int carve_scratch(uint8_t* base, const LaunchPlan& P, size_t arena_bytes, Buffer
         d.cap = bytes;
         at += bytes;
     };
-    const size_t prims = std::max(P.prim_total, 1u), tiles = std::max(P.tiles, 1u);
     take(b->stats, kStatAlloc * 4);
-    take(b->arena, std::max<size_t>(arena_bytes, 256));
-    take(b->vout, (size_t)std::max(P.vout_total, 1u) * P.stride * 4);
+    take(b->arena, arena);
+    take(b->vout, vout);
     take(b->recs, prims * sizeof(TriSetup));
     take(b->counts, prims * 4);
-    take(b->offsets, ((size_t)P.prim_total + 1) * 4);
-    take(b->sums, scan_sums_bytes(P.prim_total));
+    take(b->sums, P.sblock.size() * 8);
+    take(b->big, ((size_t)P.prim_total * 2 + 1) * 4);
     if (P.lines) take(b->line_ext, prims * sizeof(LineExt));
-    take(b->tile_start, (tiles + 1) * 4);
+    take(b->tile_range, tiles * 8);
     take(b->hist, (size_t)256 * kSortSegments * 4);
-    take(b->hist_base, ((size_t)256 * kSortSegments + 1) * 4);
-    take(b->big, ((size_t)P.prim_total + 1) * 4);
-    // each pair array starts on a 256-byte boundary: at most 4 x 255 bytes of padding
-    const size_t left = at + 1024 < kScratchBytes ? kScratchBytes - at - 1024 : 0;
-    const uint64_t cap = std::min<uint64_t>(left / 16, UINT32_MAX);
-    if (cap == 0)
-        return fail(CPV_ERROR_UNSUPPORTED,
-                    "a launch of %u primitives over %u tiles needs more than the %zu MiB of the allocation-free entry point",
-                    P.prim_total, P.tiles, kScratchBytes >> 20);
+    take(b->digit_totals, 256 * 4);
     for (DevBuf* d : {&b->keys[0], &b->keys[1], &b->vals[0], &b->vals[1]}) take(*d, (size_t)cap * 4);
+    if (at > kScratchBytes) return fail(CPV_ERROR_UNSUPPORTED, "scratch layout of %zu bytes", at);
     *pair_cap = (uint32_t)cap;
     return CPV_OK;
 }
@@ -725,7 +797,8 @@ int enqueue_scratch(cpv_context* c, PendingLaunch& L)
     x.cfg.record_costs = 0;
     x.predictor = nullptr;   // the learned order needs the predictor's buffers: the counter queue runs instead
     x.frozen = true;         // a buffer that does not fit is an error, never an allocation
-    rc = enqueue_front(x, L.P, arena);
+    if (L.P.small && L.P.small_entries > cap) L.P.small = false;   // the lists' room: the pairs themselves may need less
+    rc = enqueue_front(x, L.P, arena, cap);
     if (rc) return rc;
     x.r0 = c->ev_raster0;
     x.r1 = c->ev_raster1;
@@ -898,7 +971,7 @@ int run_launch(cpv_context* c, const cpv_config& cfg, const Program& prog, const
     c->last_traces = cfg.record_costs != 0;
     c->last_target_base.clear();
     for (const TargetParams& t : P.targets) c->last_target_base.push_back(t.tile_base);
-    c->pending = L.release();
+    if (!L->P.small) c->pending = L.release();
     c->launches++;
     return CPV_OK;
 }
@@ -1459,7 +1532,7 @@ static int batch_front(cpv_context* c, cpv_batch* B, cpv_batch::Set& S, std::vec
         x.overflow = S.overflow();
         if (!B->order.empty() && B->order[g].p) x.fixed_order = B->order[g].as<uint32_t>();
         fill_u32(x.s, S.b[g].stats.p, 0u, 2);   // the fragment counter restarts
-        int r = enqueue_front(x, B->plans[g], arena);
+        int r = enqueue_front(x, B->plans[g], arena, B->caps[g]);
         if (r == CPV_OK) r = enqueue_bin(x, B->plans[g], arena, B->caps[g], &bins[g]);
         if (r) return r;
     }
@@ -1510,7 +1583,7 @@ static int batch_record(cpv_context* c, cpv_batch* B)
             Exec x = context_exec(c, &B->set[0].b[g]);
             x.cfg = B->cfg;
             Binned bn;
-            int rc = enqueue_front(x, B->plans[g], arena);
+            int rc = enqueue_front(x, B->plans[g], arena, B->caps[g]);
             if (rc == CPV_OK) rc = enqueue_bin(x, B->plans[g], arena, B->caps[g], &bn);
             if (rc) return rc;
             if (bn.order) {
@@ -1562,7 +1635,11 @@ static int batch_build(cpv_context* c, cpv_batch* B, std::vector<LaunchSpec>& sp
     for (size_t g = 0; g < G; g++) {
         Exec x = context_exec(c, &B->set[0].b[g]);
         x.cfg = B->cfg;
-        rc = enqueue_front(x, B->plans[g], arena);
+        if (resident_workgroups(x, B->plans[g].prog.raster[B->plans[g].raster_variant], 64 * (int)B->cfg.waves_per_tile) <= 0)
+            return CPV_ERROR_DEVICE;
+        B->caps[g] = 0;
+        if (B->plans[g].small) continue;   // its lists have room for everything
+        rc = enqueue_front(x, B->plans[g], arena, UINT32_MAX);
         if (rc) return rc;
         HIP_TRY(hipMemcpyAsync(c->readback, x.b->stats.as<uint32_t>() + kStatPairTotal, 8, hipMemcpyDeviceToHost, c->stream));
         HIP_TRY(hipStreamSynchronize(c->stream));
@@ -1573,8 +1650,6 @@ static int batch_build(cpv_context* c, cpv_batch* B, std::vector<LaunchSpec>& sp
                         (unsigned long long)pairs);
         // room for vertex data that moves a little between submits
         B->caps[g] = (uint32_t)std::min<uint64_t>(pairs + pairs / 8 + 4096, UINT32_MAX);
-        if (resident_workgroups(x, B->plans[g].prog.raster[B->plans[g].raster_variant], 64 * (int)B->cfg.waves_per_tile) <= 0)
-            return CPV_ERROR_DEVICE;
     }
     return batch_record(c, B);
 }

@@ -157,8 +157,8 @@ void DevBuf::release()
 
 void Buffers::release_all()
 {
-    DevBuf* bufs[] = {&vout, &recs, &counts, &offsets, &keys[0], &keys[1], &vals[0], &vals[1], &tile_start, &hist,
-                      &hist_base, &sums, &big, &arena, &stats, &traces, &features, &pred, &okeys[0], &okeys[1],
+    DevBuf* bufs[] = {&vout, &recs, &counts, &keys[0], &keys[1], &vals[0], &vals[1], &tile_range, &hist,
+                      &digit_totals, &sums, &big, &arena, &stats, &traces, &features, &pred, &okeys[0], &okeys[1],
                       &ovals[0], &ovals[1], &line_ext};
     for (DevBuf* b : bufs) b->release();
 }

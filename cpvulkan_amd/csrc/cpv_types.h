@@ -153,6 +153,8 @@ struct TargetParams {
     uint32_t width, height;        // attachment extent
     uint32_t tiles_x, tiles_y;
     uint32_t tile_base;            // first global tile index of this target
+    uint32_t prim_base, prim_count;   // the launch's primitives drawn into this target
+    uint32_t list_base;            // first entry of its tiles' lists (bin_small_kernel)
     int32_t color_load, ds_load;   // CPV_LOAD_OP_*
     int32_t has_color, has_ds;
     int32_t color_bytes, ds_bytes; // bytes per pixel

@@ -62,7 +62,8 @@ __global__ __launch_bounds__(256) void vertex_kernel(VertexArgs a)
 struct RasterArgs {
     const TriSetup* recs;
     const uint32_t* tile_prims;     // primitive ids grouped by tile, submission order within a tile
-    const uint32_t* tile_start;     // per global tile, size tiles + 1
+    const uint2* tile_range;        // per global tile: first entry of its primitives and the one past the last
+                                    // (none when first >= last)
     const TargetParams* targets;
     const DrawDesc* draws;
     const FragmentState* fstates;

@@ -366,7 +366,8 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
         };
 
         // ---- walk the tile's primitives in submission order
-        const uint32_t lbeg = uniform_ptr(a.tile_start)[tile], lend = uniform_ptr(a.tile_start)[tile + 1];
+        const uint2 range = uniform_ptr(a.tile_range)[tile];
+        const uint32_t lbeg = range.x, lend = range.y;
         uint32_t e_next = lbeg + (uint32_t)lane < lend ? a.tile_prims[lbeg + lane] : 0u;
         for (uint32_t base = lbeg; base < lend; base += 64) {
             const int n = (int)min(64u, lend - base);

@@ -12,7 +12,7 @@ namespace cpv {
 struct FeatureArgs {
     const TriSetup* recs;
     const uint32_t* tile_prims;
-    const uint32_t* tile_start;
+    const uint2* tile_range;
     const TargetParams* targets;
     const DrawDesc* draws;
     const FragmentState* fstates;
@@ -61,9 +61,10 @@ __global__ __launch_bounds__(256) void tile_features_kernel(FeatureArgs a)
     const int x0 = (int)(local % tp.tiles_x) * a.tile, y0 = (int)(local / tp.tiles_x) * a.tile;
     const int x1 = min(x0 + a.tile, (int)tp.width), y1 = min(y0 + a.tile, (int)tp.height);
     const float tile_px = (float)(a.tile * a.tile);
-    const uint32_t b = a.tile_start[tile], e = a.tile_start[tile + 1];
+    const uint2 range = a.tile_range[tile];
+    const uint32_t b = range.x, e = max(range.x, range.y);
     float s_box = 0.0f, s_full = 0.0f, s_tri = 0.0f, s_blend = 0.0f, s_span = 0.0f;
-    const uint32_t n_all = e - b;
+    const uint32_t n_all = e - b;   // 0 for an empty range
     const uint32_t m = min(n_all, 64u);
     if ((uint32_t)lane < m) {
         const uint32_t i = b + (uint32_t)(((uint64_t)lane * n_all) / m);

@@ -331,7 +331,7 @@ int cpv_render_jobs(cpv_context* ctx, const cpv_job_desc* jobs, uint32_t job_cou
  * it is for callers that cannot allocate device memory during a frame
  * (code under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc).  Same arguments, results and asynchrony as cpv_render_pass;
- * every working buffer lives in one 64 MiB device array per GPU, set up
+ * every working buffer lives in one device array per GPU (80 MiB), set up
  * when the context is created and kept until the process ends.  No
  * hipMalloc, hipFree, hipHostMalloc or other allocating call is made.
  * A pass whose buffers (vertex outputs, triangle records, scans, tile

@@ -152,15 +152,17 @@ __device__ __forceinline__ float wave_max(float f)
 }
 
 // LDS of a workgroup: the visit fields of a chunk's candidates, one region
-// per wave, used with several blocks per lane (see GATHER), and the lanes'
-// queues of shading work.
+// per wave, used with several blocks per lane (see GATHER), the lanes'
+// queues of shading work, and each wave's ring of candidate pairs.
 template <class FS, int TILE, int WAVES>
 struct RasterStage {
     static constexpr int kBlocksPerLane = (TILE / 8) * (TILE / 8) / WAVES;
     static constexpr bool kOn = !FS::kMayDiscard && kBlocksPerLane > 1;
     static constexpr int kQueue = FS::kMayDiscard ? 1 : 4;   // a power of two
+    static constexpr int kRing = TILE == 8 ? 1 : 512;        // a power of two, at least 63 + 256
     uint4 v[kOn ? WAVES : 1][kOn ? kVisitParts : 1][kOn ? 64 : 1];
     float4 q[FS::kMayDiscard ? 1 : WAVES][kQueue][64];
+    uint32_t ring[WAVES][kRing];
 };
 
 // True when a triangle's depth (weights q_i = e_i / area to within 2 ulps,
@@ -227,10 +229,11 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
     // soup frame's raster 9% slower, 0.85 -> 0.93 ms, and the 16x16 / one-wave
     // and 32x32 / four-wave ones 2-4% faster).  A shader that may discard
     // reads the whole record per fragment and keeps the scalar loads too.
-    // Every configuration loads the next chunk's pairs while it works on the
-    // current one.
     constexpr bool GATHER = RasterStage<FS, TILE, WAVES>::kOn;
     constexpr bool STAGE = GATHER;
+    // candidates between two depth tests of a chunk's remaining ones, and the
+    // fewest whose depths are bounded over the wave's block
+    constexpr int kCullLanes = 16, kCullVisits = 5, kRefineCandidates = 2;
     // block-local depth bounds of triangles, where a lane holds one pixel
     // of an 8x8 block (lane = row * 8 + column)
     constexpr bool BLOCK_DEPTH = !ANYPRIM && !GATHER && BPW == 1;
@@ -368,56 +371,93 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
         // ---- walk the tile's primitives in submission order
         const uint2 range = uniform_ptr(a.tile_range)[tile];
         const uint32_t lbeg = range.x, lend = range.y;
-        uint32_t e_next = lbeg + (uint32_t)lane < lend ? a.tile_prims[lbeg + lane] : 0u;
-        for (uint32_t base = lbeg; base < lend; base += 64) {
-            const int n = (int)min(64u, lend - base);
-            // Depth range stored in this wave's pixels, for hierarchical
-            // culling: a primitive whose depth interval fails the test
-            // against all of them cannot change any of them.
-            float bmin = __builtin_inff(), bmax = -__builtin_inff();
-            if (hiz_op >= 0) {
+        // The pairs that name one of this wave's blocks (the emit kernels pack
+        // a primitive's blocks, or for 32x32 tiles 16x16 quadrants, into the
+        // pair) are its candidates: fetch() gives the next up to 64 of them,
+        // a candidate per lane in order.  Lists of more than 64 pairs are
+        // read 256 at a time and their candidates packed through a ring in
+        // LDS, so that every chunk but the last is full: a wave's 8x8 block
+        // is named by about 40% of the 1M soup's pairs, and the clustered 4K
+        // frame's heaviest tile, a serial chain of 950 chunks of 64 pairs,
+        // is one of about 330.
+        uint32_t mine = 0u;
+        if (TILE == 16) {
 #pragma unroll
-                for (int k = 0; k < BPW; k++)
-                    if (inside[k]) bmax = fmaxf(bmax, cur_depth(k));
-                bmax = wave_max(bmax);
-                if (!less) {
+            for (int k = 0; k < BPW; k++) mine |= 1u << (kPairBlockShift + slot + k * WAVES);
+        } else if (TILE == 32) {
 #pragma unroll
-                    for (int k = 0; k < BPW; k++)
-                        if (inside[k]) bmin = fminf(bmin, cur_depth(k));
-                    bmin = -wave_max(-bmin);
-                }
+            for (int k = 0; k < BPW; k++) {
+                const int blk = slot + k * WAVES;
+                mine |= 1u << (kPairBlockShift + (blk / BW) / 2 * 2 + (blk % BW) / 2);
             }
-            // each lane tests one primitive of the chunk against the wave's area
-            const uint32_t e = e_next;
-            uint32_t gp_l = 0, blocks_l = 0;
-            bool ov = false;
-            if (lane < n) {
-                gp_l = e & kPairPrim;
-                blocks_l = e >> kPairBlockShift;
-                if (TILE == 8) {
-                    // one block per tile: a pair exists only where the box meets the tile
-                    ov = true;
-                } else if (TILE == 16) {
-                    // the pair carries the blocks the primitive may cover
-                    uint32_t mine = 0u;
+        }
+        const bool packed = TILE != 8 && lend > lbeg && lend - lbeg > 64u;   // wave-uniform
+        auto& ring = stage_area.ring[wave];
+        constexpr uint32_t R = RasterStage<FS, TILE, WAVES>::kRing;
+        uint32_t pos = packed ? lbeg & ~3u : lbeg, head = 0, tail = 0;
+        auto group = [&](uint32_t at) {   // pairs at + 4 * lane .. + 3 of the list (16-byte aligned)
+            const uint32_t i = at + 4u * (uint32_t)lane;
+            return i >= at && i < lend ? *(const uint4*)(a.tile_prims + i) : make_uint4(0u, 0u, 0u, 0u);
+        };
+        uint4 g_next = packed ? group(pos) : make_uint4(0u, 0u, 0u, 0u);   // loaded a step ahead
+        auto fetch = [&](uint32_t& e, bool& ok) {
+            if (packed) {
+                while (tail - head < 64u && pos < lend) {
+                    const uint32_t v[4] = {g_next.x, g_next.y, g_next.z, g_next.w};
+                    const uint32_t i = pos + 4u * (uint32_t)lane;
+                    pos += min(256u, lend - pos);
+                    g_next = group(pos);
+                    uint32_t at = tail;
+                    bool hit[4];
 #pragma unroll
-                    for (int k = 0; k < BPW; k++) mine |= 1u << (slot + k * WAVES);
-                    ov = (blocks_l & mine) != 0u;
-                } else {
-                    // the pair carries the 16x16 quadrants the primitive may
-                    // cover; a wave's blocks lie in the quadrants of mine
-                    uint32_t mine = 0u;
-#pragma unroll
-                    for (int k = 0; k < BPW; k++) {
-                        const int blk = slot + k * WAVES;
-                        mine |= 1u << ((blk / BW) / 2 * 2 + (blk % BW) / 2);
+                    for (int j = 0; j < 4; j++) {
+                        hit[j] = (v[j] & mine) != 0u && i + j >= lbeg && i + j < lend;
+                        const uint64_t m = lanes(hit[j]);
+                        at = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, at));
+                        tail += (uint32_t)__popcll(m);
                     }
-                    ov = (blocks_l & mine) != 0u;
+#pragma unroll
+                    for (int j = 0; j < 4; j++)
+                        if (hit[j]) { ring[at & (R - 1)] = v[j]; at++; }
                 }
+                wave_lds_fence();
+                const uint32_t n = min(64u, tail - head);
+                e = ring[(head + (uint32_t)lane) & (R - 1)];
+                ok = (uint32_t)lane < n;
+                head += n;
+                wave_lds_fence();
+            } else {
+                const uint32_t i = pos + (uint32_t)lane;
+                ok = i >= pos && i < lend;
+                e = ok ? a.tile_prims[i] : 0u;
+                if (TILE != 8) ok = ok && (e & mine) != 0u;
+                pos += min(64u, lend - min(pos, lend));
             }
+        };
+        auto more = [&]() { return packed ? tail != head || pos < lend : pos < lend; };
+        // The next chunk's candidates are fetched, and the lower end of their
+        // depth interval loaded, before this chunk is worked on; with it their
+        // records come into the XCD's L2.
+        uint32_t e_next = 0u;
+        bool ok_next = false;
+        float lo_next = 0.0f;
+        auto prefetch = [&]() {
+            ok_next = false;
+            if (more()) {
+                fetch(e_next, ok_next);
+                if (ok_next) lo_next = a.recs[e_next & kPairPrim].dt_lo;
+            }
+        };
+        bool chunk = more();
+        prefetch();
+        while (chunk) {
+            const uint32_t e = e_next, gp_l = e & kPairPrim, blocks_l = e >> kPairBlockShift;
+            float lo_l = lo_next;
+            bool ov = ok_next;
+            chunk = more();
+            prefetch();
             // the candidates' visit fields, all lanes at once, straight into
             // the wave's LDS region (global_load_lds: no registers)
-            float4 dz = make_float4(0.0f, 0.0f, 0.0f, 0.0f);   // dt_lo, dt_hi, area, draw
             if constexpr (GATHER) {
                 wave_lds_fence();   // the previous chunk's reads come first
                 if (ov) {
@@ -426,69 +466,96 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
                     for (int p = 0; p < kVisitParts; p++)
                         __builtin_amdgcn_global_load_lds((const void*)(src + p),
                                                          (__attribute__((address_space(3))) void*)&stage[wave][p][0], 16, 0, 0);
-                    dz = *(const float4*)&a.recs[gp_l].dt_lo;
                 }
             }
-            // the next chunk's pairs, loaded while this chunk is worked on
-            {
-                const uint32_t nb = base + 64u + (uint32_t)lane;
-                e_next = nb < lend ? a.tile_prims[nb] : 0u;
+            // Hierarchical culling: a primitive whose depth interval fails
+            // the test against every depth stored in the wave's pixels
+            // cannot change any of them.  With LESS and LESS_OR_EQUAL the
+            // interval's lower end decides: `lo_l` holds a candidate's, and
+            // the stored depths only fall, so it is tested again every few
+            // visits against their current maximum (a dozen vector
+            // instructions, a third of a visit).  Testing once per chunk left
+            // the soup 27 us slower once the chunks were full.
+            const bool culls = hiz_op >= 0 && less;
+            if (hiz_op >= 0 && !less) {
+                float bmin = __builtin_inff(), bmax = -__builtin_inff();
+#pragma unroll
+                for (int k = 0; k < BPW; k++) {
+                    if (!inside[k]) continue;
+                    bmin = fminf(bmin, cur_depth(k));
+                    bmax = fmaxf(bmax, cur_depth(k));
+                }
+                bmax = wave_max(bmax);
+                bmin = -wave_max(-bmin);
+                if (ov) {
+                    const float2 dz = *(const float2*)&a.recs[gp_l].dt_lo;
+                    ov = !hiz_rejects(hiz_op, dz.x, dz.y, bmin, bmax);
+                }
             }
-            if (hiz_op >= 0) {
-                if constexpr (BLOCK_DEPTH) {
-                    // A triangle's depth bounded over the pixels it may cover
-                    // in this wave's block (block_depth_range): its box
-                    // clipped to the block, far tighter than its bounds over
-                    // all its pixels.  Taken for the candidates of the draw
-                    // last visited, whose pixel centres the lanes hold, when
-                    // that draw's depth range is [0, 1] (the depth then is
-                    // the tested value).  The record's visit fields are
-                    // loaded with the depth interval, at once: one memory
-                    // latency per chunk; before the tile's first visit
-                    // (all of a short list) only the interval is loaded.
-                    const bool near = cur_draw != 0xFFFFFFFFu && vp_identity;   // wave-uniform
-                    uint4 p0 = make_uint4(0u, 0u, 0u, 0u), p1 = p0, p2 = p0, p3 = p0, p5 = p0;
-                    if (ov) {
-                        const uint4* src = (const uint4*)&a.recs[gp_l];
-                        if (near) {
-                            p0 = src[0]; p1 = src[1]; p2 = src[2]; p3 = src[3];
-                            p5 = src[5];
+            bool refined = !BLOCK_DEPTH || !packed;   // short lists: not worth the records' loads
+            auto cull = [&](uint64_t m) {
+                float bmax = -__builtin_inff();
+#pragma unroll
+                for (int k = 0; k < BPW; k++)
+                    if (inside[k]) bmax = fmaxf(bmax, cur_depth(k));
+                bmax = wave_max(bmax);
+                m &= ~lanes(lo_l > bmax);
+                if (BLOCK_DEPTH && !refined && __popcll(m) >= kRefineCandidates) {
+                    if (cur_draw != 0xFFFFFFFFu && vp_identity) {
+                        // A triangle's depth bounded over the pixels it may
+                        // cover in this wave's block (block_depth_range): its
+                        // box clipped to the block, far tighter than its
+                        // bounds over all its pixels.  For the candidates of
+                        // the draw last visited, whose pixel centres the lanes
+                        // hold, when that draw's depth range is [0, 1] (the
+                        // depth then is the tested value).
+                        refined = true;
+                        const bool mine_l = in_lanes(m);
+                        uint4 p0 = make_uint4(0u, 0u, 0u, 0u), p1 = p0, p2 = p0, p3 = p0, p4 = p0, p5 = p0;
+                        if (mine_l) {
+                            const uint4* src = (const uint4*)&a.recs[gp_l];
+                            p0 = src[0]; p1 = src[1]; p2 = src[2]; p3 = src[3]; p4 = src[4]; p5 = src[5];
                         }
-                        dz = *(const float4*)(src + 4);
-                        ov = less ? !(dz.x > bmax) : !hiz_rejects(hiz_op, dz.x, dz.y, bmin, bmax);
-                    }
-                    if (near) {
                         // lane c holds column bx0 + c, lane 8 r row by0 + r
                         const int bx0 = __builtin_amdgcn_readfirstlane(pxx[0]), by0 = __builtin_amdgcn_readfirstlane(pxy[0]);
                         const int cl = min(max((int)p3.x - bx0, 0), 7), ch = min(max((int)p3.z - 1 - bx0, 0), 7);
                         const int rl = min(max((int)p3.y - by0, 0), 7), rh = min(max((int)p3.w - 1 - by0, 0), 7);
                         const float xa = __shfl(xf[0], cl, 64), xb = __shfl(xf[0], ch, 64);
                         const float ya = __shfl(yf[0], rl * 8, 64), yb = __shfl(yf[0], rh * 8, 64);
-                        if (ov && (__float_as_uint(dz.w) & kPrimDraw) == cur_draw) {
+                        if (mine_l && (p4.w & kPrimDraw) == cur_draw) {
                             const float ax[3] = {__uint_as_float(p0.x), __uint_as_float(p0.y), __uint_as_float(p0.z)};
                             const float ay[3] = {__uint_as_float(p0.w), __uint_as_float(p1.x), __uint_as_float(p1.y)};
                             const float dy[3] = {__uint_as_float(p1.z), __uint_as_float(p1.w), __uint_as_float(p2.x)};
                             const float dx[3] = {__uint_as_float(p2.y), __uint_as_float(p2.z), __uint_as_float(p2.w)};
                             const float z[3] = {__uint_as_float(p5.x), __uint_as_float(p5.y), __uint_as_float(p5.z)};
                             float lo, hi;
-                            if (block_depth_range(ax, ay, dy, dx, dz.z, __uint_as_float(p5.w), z, fminf(xa, xb), fmaxf(xa, xb),
-                                                  fminf(ya, yb), fmaxf(ya, yb), lo, hi))
-                                ov = less ? !(lo > bmax) : !hiz_rejects(hiz_op, lo, hi, bmin, bmax);
+                            if (block_depth_range(ax, ay, dy, dx, __uint_as_float(p4.z), __uint_as_float(p5.w), z, fminf(xa, xb),
+                                                  fmaxf(xa, xb), fminf(ya, yb), fmaxf(ya, yb), lo, hi))
+                                lo_l = fmaxf(lo_l, lo);
                         }
+                        m &= ~lanes(lo_l > bmax);
                     }
-                } else if (ov) {
-                    if constexpr (!GATHER) dz = *(const float4*)&a.recs[gp_l].dt_lo;
-                    ov = less ? !(dz.x > bmax) : !hiz_rejects(hiz_op, dz.x, dz.y, bmin, bmax);
                 }
-            }
+                return m;
+            };
             uint64_t mask = lanes(ov);
             if constexpr (STAGE) {
                 __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): the LDS loads have landed
                 wave_lds_fence();
             }
-            while (mask) {
-                const int j = (int)__builtin_ctzll(mask);
-                mask &= mask - 1;
+            int since = kCullVisits;   // candidates visited since the last cull
+            const int step = packed ? kCullLanes : 64;
+            for (int first = 0; first < 64; first += step) {
+              uint64_t window = mask & ((~0ull >> (64 - step)) << first);
+              if (culls && window && since >= kCullVisits) {
+                  mask = cull(mask & (~0ull << first));
+                  window &= mask;
+                  since = 0;
+              }
+              since += __popcll(window);
+              while (window) {
+                const int j = (int)__builtin_ctzll(window);
+                window &= window - 1;
                 const uint32_t gprim = __builtin_amdgcn_readlane(gp_l, j);
                 const uint32_t blocks = (TILE >= 16 && BPW > 1) ? __builtin_amdgcn_readlane(blocks_l, j) : 0u;
                 TriSetup r;
@@ -664,6 +731,7 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
                         }
                     }
                 }
+              }
             }
         }
         if (!FS::kMayDiscard) {

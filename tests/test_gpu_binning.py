@@ -105,3 +105,16 @@ def test_more_setup_workgroups_than_a_scan_round(ctx):
     """4,200 workgroups of setup: the scan of their sums takes a second round."""
     s = S.soup(4200 * 256 - 5, 320, 200, seed=8, size_px=np.log(2.0))
     _check(ctx, s, "1.07M small triangles", count=False)
+
+
+@pytest.mark.parametrize("op", ["LESS", "LESS_OR_EQUAL", "GREATER"])
+@pytest.mark.parametrize("tile,waves", [(16, 4), (16, 1), (32, 4), (8, 1)])
+def test_list_lengths(ctx, tile, waves, op):
+    """Lists around the sizes at which the raster kernel packs their candidates (64) and reads them (256 at a time), and
+    chunks of candidates around 16 and 64, at list starts that are no multiple of four."""
+    for n in (1, 15, 17, 63, 64, 65, 66, 127, 200, 255, 257, 320, 519, 1025):
+        s = S.soup(n, 40, 33, seed=n, size_px=np.log(24.0))
+        s.pipeline["depth_compare"] = {"LESS": 1, "LESS_OR_EQUAL": 3, "GREATER": 4}[op]
+        s.clear_depth = 0.0 if op == "GREATER" else 1.0
+        _check(ctx, s, f"lists of up to {n} {op} {tile}x{waves}", tile, waves, count=False)
+    _check(ctx, s, f"lists of up to {n} {op} {tile}x{waves} counting", tile, waves)

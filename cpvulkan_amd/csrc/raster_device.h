@@ -49,6 +49,19 @@ CPV_DEV const T* uniform_ptr(uint64_t address)
 template <class T>
 CPV_DEV const T* uniform_ptr(const T* p) { return uniform_ptr<T>((uint64_t)p); }
 
+// A device address from a descriptor as a pointer that is known to be global
+// (an integer converts to a flat pointer, whose accesses test the address's
+// aperture and count against the LDS too).
+template <class T>
+CPV_DEV T* global_ptr(uint64_t address)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    return (T*)(__attribute__((address_space(1))) T*)address;
+#else
+    return (T*)address;
+#endif
+}
+
 // Byte extraction/insertion in a pixel held as 4 dwords (up to 16 bytes).
 CPV_DEV uint32_t pick_word(const uint32_t px[4], int w)
 {
@@ -261,7 +274,7 @@ CPV_DEV void texel(const TextureDesc& t, uint32_t level, int32_t x, int32_t y, f
         border_colour(t.sampler.border_color, out);
         return;
     }
-    const uint8_t* p = (const uint8_t*)t.address + t.level_offset[level] +
+    const uint8_t* p = global_ptr<const uint8_t>(t.address) + t.level_offset[level] +
                        ((uint64_t)y * w + (uint64_t)x) * (uint64_t)t.fmt.total;
     uint32_t px[4] = {0u, 0u, 0u, 0u};
     if (t.fmt.total == 4) {
@@ -287,17 +300,39 @@ CPV_DEV void lerp4(const float a[4], const float b[4], double t, float out[4])
     }
 }
 
+// A texture of four 8-bit UNORM channels in 4 bytes, no border mode and at most
+// 2^30 texels in the level: texels then come by 32-bit offsets, with no
+// bounds test (wrapped coordinates are inside) and no per-channel format
+// branches.  The tests are on scalars; the generic code takes about 40 of them
+// per bilinear sample.
+CPV_DEV bool plain_texture(const TextureDesc& t, uint32_t level)
+{
+    const FormatDesc& f = t.fmt;
+    return f.base == kBaseUNorm && f.element == 1 && f.total == 4 && (f.off[0] | f.off[1] | f.off[2] | f.off[3]) >= 0 &&
+           t.sampler.address_u != 3 && t.sampler.address_v != 3 &&
+           (uint64_t)t.level_w[level] * t.level_h[level] - 1ull < (1ull << 30);   // an empty level takes the bounds tests
+}
+CPV_DEV void plain_texel(const TextureDesc& t, const uint32_t* base, uint32_t at, float out[4])
+{
+    const uint32_t w = base[at];
+#pragma unroll
+    for (int i = 0; i < 4; i++) out[i] = unorm8_to_float((w >> (t.fmt.off[i] * 8)) & 255u);
+}
+
 // SampleImageOfLevel, 2D, weighted average (ImageSampler.cpp:461-579).
-CPV_DEV void sample_level(const TextureDesc& t, uint32_t level, float u, float v, int32_t filter, float out[4])
+template <bool PLAIN>
+CPV_DEV void sample_level_as(const TextureDesc& t, uint32_t level, float u, float v, int32_t filter, float out[4])
 {
     const float fw = (float)t.level_w[level], fh = (float)t.level_h[level];
     const int32_t iw = (int32_t)t.level_w[level], ih = (int32_t)t.level_h[level];
+    const uint32_t* base = global_ptr<const uint32_t>(t.address + t.level_offset[level]);
     if (filter == 0) {
         int32_t cx = (int32_t)floorf(u * fw + 0.0f);
         int32_t cy = (int32_t)floorf(v * fh + 0.0f);
         cx = wrap_coord(cx, iw, t.sampler.address_u);
         cy = wrap_coord(cy, ih, t.sampler.address_v);
-        texel(t, level, cx, cy, out);
+        if (PLAIN) plain_texel(t, base, (uint32_t)cy * (uint32_t)iw + (uint32_t)cx, out);
+        else texel(t, level, cx, cy, out);
         return;
     }
     int32_t x0 = (int32_t)floorf(u * fw - 0.5f);
@@ -309,13 +344,39 @@ CPV_DEV void sample_level(const TextureDesc& t, uint32_t level, float u, float v
     const float qx = u * fw - 0.5f, qy = v * fh - 0.5f;
     const float tx = qx - floorf(qx), ty = qy - floorf(qy);
     float p00[4], p01[4], p10[4], p11[4], a[4], b[4];
-    texel(t, level, x0, y0, p00);
-    texel(t, level, x0, y1, p01);
-    texel(t, level, x1, y0, p10);
-    texel(t, level, x1, y1, p11);
-    lerp4(p00, p10, (double)tx, a);
-    lerp4(p01, p11, (double)tx, b);
+    if (PLAIN) {
+        const uint32_t r0 = (uint32_t)y0 * (uint32_t)iw, r1 = (uint32_t)y1 * (uint32_t)iw;
+        plain_texel(t, base, r0 + (uint32_t)x0, p00);
+        plain_texel(t, base, r1 + (uint32_t)x0, p01);
+        plain_texel(t, base, r0 + (uint32_t)x1, p10);
+        plain_texel(t, base, r1 + (uint32_t)x1, p11);
+    } else {
+        texel(t, level, x0, y0, p00);
+        texel(t, level, x0, y1, p01);
+        texel(t, level, x1, y0, p10);
+        texel(t, level, x1, y1, p11);
+    }
+    // The lerps across x in single precision where that rounds alike: UNORM8
+    // values (and so their rounded differences) are multiples of 2^-31 of at
+    // most 1, and with |qx| >= 4 the fraction tx is a multiple of 2^-21, so
+    // the double sum a + d * tx has at most 52 bits, is exact, and its one
+    // rounding to float is the fma's (tests/test_unorm_forms.py).
+    if (PLAIN && fabsf(qx) >= 4.0f) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            a[i] = fmaf(p10[i] - p00[i], tx, p00[i]);
+            b[i] = fmaf(p11[i] - p01[i], tx, p01[i]);
+        }
+    } else {
+        lerp4(p00, p10, (double)tx, a);
+        lerp4(p01, p11, (double)tx, b);
+    }
     lerp4(a, b, (double)ty, out);
+}
+CPV_DEV void sample_level(const TextureDesc& t, uint32_t level, float u, float v, int32_t filter, float out[4])
+{
+    if (plain_texture(t, level)) sample_level_as<true>(t, level, u, v, filter, out);
+    else sample_level_as<false>(t, level, u, v, filter, out);
 }
 
 // ImageSampleExplicitLod (CPVulkan/GlslFunctions.cpp:598-654) and SampleImage
@@ -327,27 +388,26 @@ CPV_DEV void sample_explicit(const TextureDesc& t, float u, float v, float lod, 
     bias = bias < -32.0f ? -32.0f : (bias > 32.0f ? 32.0f : bias);
     float lambda = lod + bias;
     lambda = lambda < t.sampler.min_lod ? t.sampler.min_lod : (lambda > t.sampler.max_lod ? t.sampler.max_lod : lambda);
-    if (lambda <= 0) {
-        sample_level(t, 0, u, v, t.sampler.mag_filter, out);
-    } else {
+    // the first level's sample, and for a fraction between two levels the second's
+    uint32_t level = 0;
+    int32_t filter = t.sampler.mag_filter;
+    float delta = 0.0f;
+    if (!(lambda <= 0)) {
         const float maxl = (float)(t.level_count - 1);
         const float ml = lambda < 0.0f ? 0.0f : (lambda > maxl ? maxl : lambda);
+        filter = t.sampler.min_filter;
         if (t.sampler.mipmap_mode == 0) {
-            const uint32_t real = (uint32_t)ceilf(ml + 0.5f) - 1u;
-            sample_level(t, real, u, v, t.sampler.min_filter, out);
+            level = (uint32_t)ceilf(ml + 0.5f) - 1u;
         } else {
-            const uint32_t l1 = (uint32_t)floorf(ml);
-            const float delta = ml - (float)l1;
-            float p1[4];
-            sample_level(t, l1, u, v, t.sampler.min_filter, p1);
-            if (delta == 0) {
-                out[0] = p1[0]; out[1] = p1[1]; out[2] = p1[2]; out[3] = p1[3];
-            } else {
-                float p2[4];
-                sample_level(t, l1 + 1, u, v, t.sampler.min_filter, p2);
-                lerp4(p1, p2, (double)delta, out);
-            }
+            level = (uint32_t)floorf(ml);
+            delta = ml - (float)level;
         }
+    }
+    sample_level(t, level, u, v, filter, out);
+    if (!(delta == 0)) {
+        float p2[4];
+        sample_level(t, level + 1, u, v, filter, p2);
+        lerp4(out, p2, (double)delta, out);
     }
     if (t.fmt.off[0] < 0) out[0] = 0.0f;
     if (t.fmt.off[1] < 0) out[1] = 0.0f;

@@ -298,10 +298,10 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
             px[k].ds1 = tp.clear_ds[1];
             const uint64_t pix = (uint64_t)pxy[k] * tp.width + (uint64_t)pxx[k];
             if (inside[k] && has_color && tp.color_load != 1)
-                load_pixel((const uint8_t*)tp.color_addr + pix * color_bytes, color_bytes, px[k].color);
+                load_pixel(global_ptr<const uint8_t>(tp.color_addr) + pix * color_bytes, color_bytes, px[k].color);
             if (inside[k] && has_ds && tp.ds_load != 1) {
                 uint32_t w4[4];
-                load_pixel((const uint8_t*)tp.ds_addr + pix * ds_bytes, ds_bytes, w4);
+                load_pixel(global_ptr<const uint8_t>(tp.ds_addr) + pix * ds_bytes, ds_bytes, w4);
                 px[k].ds0 = w4[0];
                 px[k].ds1 = w4[1];
             } else if (inside[k] && has_ds && ds_bytes == 8) {
@@ -309,7 +309,7 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
                 // depth and the stencil byte and keeps the three padding bytes
                 // (ImageCompiler.cpp:895-945)
                 uint32_t w4[4];
-                load_pixel((const uint8_t*)tp.ds_addr + pix * ds_bytes, ds_bytes, w4);
+                load_pixel(global_ptr<const uint8_t>(tp.ds_addr) + pix * ds_bytes, ds_bytes, w4);
                 px[k].ds1 = (w4[1] & 0xFFFFFF00u) | (tp.clear_ds[1] & 0xFFu);
             }
             zc[k] = stored_depth(tile_depth, px[k].ds0);
@@ -744,10 +744,10 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
         for (int k = 0; k < BPW; k++) {
             if (!inside[k]) continue;
             const uint64_t pix = (uint64_t)pxy[k] * tp.width + (uint64_t)pxx[k];
-            if (has_color) store_pixel((uint8_t*)tp.color_addr + pix * color_bytes, color_bytes, px[k].color);
+            if (has_color) store_pixel(global_ptr<uint8_t>(tp.color_addr) + pix * color_bytes, color_bytes, px[k].color);
             if (has_ds) {
                 const uint32_t w4[4] = {px[k].ds0, px[k].ds1, 0u, 0u};
-                store_pixel((uint8_t*)tp.ds_addr + pix * ds_bytes, ds_bytes, w4);
+                store_pixel(global_ptr<uint8_t>(tp.ds_addr) + pix * ds_bytes, ds_bytes, w4);
             }
         }
 

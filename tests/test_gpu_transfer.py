@@ -200,6 +200,29 @@ def test_blit_colour(gpu_ctx, mem, fmt, filter_):
     assert np.array_equal(got, want), f"{fmt}: {np.count_nonzero(got != want)} bytes differ"
 
 
+@pytest.mark.parametrize("sfmt,dfmt", [("R8G8B8A8_UNORM", "B8G8R8A8_UNORM"), ("B8G8R8A8_UNORM", "B8G8R8A8_UNORM"),
+                                       ("R8G8B8A8_UNORM", "R16G16B16A16_UNORM")])
+def test_blit_unorm8_row_ends(gpu_ctx, mem, sfmt, dfmt):
+    """Destinations around the 64 x 4 pixels of a workgroup, sources around the
+    first texels (where the lerps stay in double precision), both filters."""
+    SW, SH, DW, DH = 130, 11, 260, 23
+    sc, dc = F[sfmt], F[dfmt]
+    src = rand_bytes(SW * SH * 4)
+    s = mem.alloc(src)
+    dsts = [(0, 0, 1, 1), (2, 0, 65, 3), (67, 0, 131, 4), (260, 0, 195, 5), (0, 5, 257, 22), (258, 22, 260, 6)]
+    srcs = [(0, 0, 130, 11), (129, 10, 130, 11), (3, 0, 4, 11), (0, 11, 130, 0), (65, 1, 130, 9), (5, 5, 6, 6)]
+    for filter_ in (0, 1):
+        dst = rand_bytes(DW * DH * abi.FORMAT_BYTES[dc])
+        d = mem.alloc(dst)
+        regions = [abi.BlitRegion((C.c_int32 * 4)(*a), (C.c_int32 * 4)(*b), 1, 0) for a, b in zip(srcs, dsts)]
+        want = dst.copy()
+        oracle_lib.blit_image(src.copy(), sc, SW, SH, want, dc, DW, DH, regions, filter_)
+        print(f"[transfer] blit {sfmt} to {dfmt} filter={filter_}", flush=True)
+        gpu_ctx.blit_image(abi.ImageLevel(s, sc, SW, SH, 0), abi.ImageLevel(d, dc, DW, DH, 0), regions, filter_)
+        got = mem.read(d, dst.nbytes)
+        assert np.array_equal(got, want), (filter_, np.count_nonzero(got != want))
+
+
 @pytest.mark.parametrize("fmt,aspect", [("D32_SFLOAT", 2), ("D16_UNORM", 2), ("D24_UNORM_S8_UINT", 6), ("D24_UNORM_S8_UINT", 2),
                                         ("D24_UNORM_S8_UINT", 4), ("D32_SFLOAT_S8_UINT", 6)])
 def test_blit_depth_stencil(gpu_ctx, mem, fmt, aspect):

@@ -426,10 +426,24 @@ int enqueue_front(Exec& x, const LaunchPlan& P, uint8_t* arena, uint32_t pair_ca
     if (P.small) return CPV_OK;
     ScanArgs ca{b.sums.as<uint64_t>(), P.prim_total ? (uint32_t)P.sblock.size() : 0u, std::max(pair_cap, 1u),
                 (uint64_t*)(stats + kStatPairTotal), stats + kStatPairs, x.overflow ? x.overflow : stats + kStatOverflow,
-                b.big.as<uint32_t>(), x.host_total};
+                b.big.as<uint32_t>(), x.host_total, stats + kStatLong};
     hipLaunchKernelGGL(scan_blocks_kernel, dim3(1), dim3(kScanThreads), 0, x.s, ca);
     HIP_TRY(hipGetLastError());
     return CPV_OK;
+}
+
+// Workgroups that raster the long tiles' blocks: eight for each of the CUs,
+// a multiple of kRasterQueues.
+constexpr uint32_t kLongGroups = 2048u;
+
+// The launch splits its long tiles: waves that hold kSplitBlocks or more, a
+// workgroup per tile (the counter-ordered queue balances by itself), and no
+// cycles recorded per tile.
+bool splits_long_tiles(const Exec& x, const LaunchPlan& P)
+{
+    const uint32_t blocks = x.cfg.tile_size / 8;
+    return !P.small && P.tiles && P.prim_total && blocks * blocks >= (uint32_t)kSplitBlocks * x.cfg.waves_per_tile && !x.cfg.record_costs &&
+           effective_scheduler(x) != CPV_SCHED_COUNTER;
 }
 
 // Where the binning stage left its results for the raster kernel.
@@ -481,6 +495,15 @@ int enqueue_bin(Exec& x, const LaunchPlan& P, uint8_t* arena, uint32_t pair_cap,
     while ((1u << bits) < P.tiles) bits++;
     rc = radix_sort(x, b.keys, b.vals, stats + kStatPairs, bits, ranges, P.tiles, &src);
     if (rc) return rc;
+
+    // where the raster kernel splits them, the long tiles' list, in the space
+    // of the sorted keys, which nothing reads any more (a long tile has
+    // many pairs, so the list always fits)
+    if (splits_long_tiles(x, P)) {
+        hipLaunchKernelGGL(long_tiles_kernel, dim3((P.tiles + 255) / 256), dim3(256), 0, x.s, ranges, P.tiles, stats + kStatLong,
+                           b.keys[0].as<uint32_t>());
+        HIP_TRY(hipGetLastError());
+    }
 
     // scheduling (a recorded batch computes its learned order once, when it
     // is recorded, and its submits reuse it)
@@ -562,6 +585,12 @@ int enqueue_raster(Exec& x, const LaunchPlan& P, uint8_t* arena, const Binned& b
     ra.uniform_fstate = P.uniform_fstate;
     ra.count = x.cfg.count_fragments ? 1u : 0u;
     uint32_t grid = P.tiles;
+    if (splits_long_tiles(x, P)) {
+        ra.long_groups = kLongGroups;
+        ra.long_tiles = b.keys[0].as<uint32_t>();
+        ra.longs = stats + kStatLong;
+        grid += kLongGroups;
+    }
     if (ra.persistent) {
         const int resident = resident_workgroups(x, rk, block);
         if (resident <= 0) return CPV_ERROR_DEVICE;

@@ -33,6 +33,10 @@ namespace cpv {
 constexpr uint32_t kRasterQueues = 8;
 constexpr uint32_t kRasterQueueStride = 32;
 
+// Raster waves that hold at least this many 8x8 blocks take the blocks of
+// long tiles one by one (RasterArgs::longs).
+constexpr int kSplitBlocks = 4;
+
 // Channel base types of FormatInformation (CPVulkanBase/Formats.h:30-103).
 enum BaseType : int32_t {
     kBaseNone = 0,
@@ -76,17 +80,15 @@ struct TriSetup {
     uint32_t draw_flags;      // 76: draw index within the launch (28 bits), the kPrim flags above it
     float z[3];               // 80-91: p_k.z / p_k.w
     float rinv;               // 92: 1 / area, correctly rounded
-    // Bytes 0-95 are everything a primitive's visit of a pixel block reads
-    // (kVisitParts 16-byte parts); the rest only the colour work reads.
+    // Bytes 0-95 are everything a primitive's visit of a pixel block reads;
+    // the rest only the colour work reads.
     float w[3];               // 96-107: clip-space w of p_k
     uint32_t v[3];            // 108-119: vertex-output indices of p0, p1, p2 (after the CW swap)
     uint32_t provoking;       // 120: vertex-output index of the provoking vertex
     uint32_t pad;
 };
 static_assert(sizeof(TriSetup) == 128, "TriSetup must be 128 bytes");
-constexpr int kVisitParts = 6;
-static_assert(__builtin_offsetof(TriSetup, rinv) == 92 && __builtin_offsetof(TriSetup, w) == 16 * kVisitParts,
-              "the visit fields fill the first kVisitParts parts");
+static_assert(__builtin_offsetof(TriSetup, rinv) == 92 && __builtin_offsetof(TriSetup, w) == 96, "the visit fields come first");
 
 // The primitive's flags: front facing; its kind; kPrimFast, set for
 // triangles whose coordinates lie within 2^20, whose area is in [2^-60, 2^60]

@@ -151,16 +151,12 @@ __device__ __forceinline__ float wave_max(float f)
 #endif
 }
 
-// LDS of a workgroup: the visit fields of a chunk's candidates, one region
-// per wave, used with several blocks per lane (see GATHER), the lanes'
-// queues of shading work, and each wave's ring of candidate pairs.
+// LDS of a workgroup: the lanes' queues of shading work and each wave's ring
+// of candidate pairs.
 template <class FS, int TILE, int WAVES>
 struct RasterStage {
-    static constexpr int kBlocksPerLane = (TILE / 8) * (TILE / 8) / WAVES;
-    static constexpr bool kOn = !FS::kMayDiscard && kBlocksPerLane > 1;
     static constexpr int kQueue = FS::kMayDiscard ? 1 : 4;   // a power of two
     static constexpr int kRing = TILE == 8 ? 1 : 512;        // a power of two, at least 63 + 256
-    uint4 v[kOn ? WAVES : 1][kOn ? kVisitParts : 1][kOn ? 64 : 1];
     float4 q[FS::kMayDiscard ? 1 : WAVES][kQueue][64];
     uint32_t ring[WAVES][kRing];
 };
@@ -218,33 +214,37 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
     // with larger arrays.
     if (*a.overflow) return;
 
-    // With several blocks per lane, a chunk's candidate primitives have the
-    // visit fields of their records (the first kVisitParts parts) loaded by
-    // all their lanes at once straight into the wave's LDS region
-    // (global_load_lds_dwordx4, which takes no registers), before the
-    // chunk's depth test, and the survivor loop reads them from there: the
-    // chunk pays one memory latency for the records of all its survivors.
-    // With one block per lane each survivor's record is read with scalar
-    // loads (measured on MI355X: the LDS staging made the 16x16 / four-wave
-    // soup frame's raster 9% slower, 0.85 -> 0.93 ms, and the 16x16 / one-wave
-    // and 32x32 / four-wave ones 2-4% faster).  A shader that may discard
-    // reads the whole record per fragment and keeps the scalar loads too.
-    constexpr bool GATHER = RasterStage<FS, TILE, WAVES>::kOn;
-    constexpr bool STAGE = GATHER;
+    // Each survivor's record is read with scalar loads.  Staging the visit
+    // fields of a chunk's candidates through LDS (global_load_lds) where a wave
+    // holds several blocks, as this kernel did, took 6 KB a wave, which with
+    // one block's ring and queue left a CU 13 waves: without it the 48-job
+    // batch went from 1,764 to 1,373 us a submit with 16x16 tiles and two
+    // waves, from 2,040 to 1,776 with one, and with 32x32 tiles and four waves
+    // from 2,359 to 1,873.
     // candidates between two depth tests of a chunk's remaining ones, and the
     // fewest whose depths are bounded over the wave's block
     constexpr int kCullLanes = 16, kCullVisits = 5, kRefineCandidates = 2;
     // block-local depth bounds of triangles, where a lane holds one pixel
     // of an 8x8 block (lane = row * 8 + column)
-    constexpr bool BLOCK_DEPTH = !ANYPRIM && !GATHER && BPW == 1;
-    auto& stage = stage_area.v;
+    constexpr bool BLOCK_DEPTH = !ANYPRIM && BPW == 1;
     // the hierarchical depth op (-1: no hierarchical culling)
     const int32_t hiz_op = a.hiz_op;
     const bool less = a.less_depth != 0;
     uint32_t tried = 0;   // queues found empty, starting at home
+    // A wave that holds many blocks walks a long tile's list once for all of
+    // them, one after the other: a serial chain that the launch may end up
+    // waiting for.  Long tiles are split, a unit of work per block (of each
+    // of the workgroup's waves), and start first.  The 48-job batch went from
+    // 2,125 to 1,776 us a submit with 16x16 tiles and one wave, with 32x32
+    // tiles from 2,337 to 1,873 (four waves) and from 7,295 to 3,568 (one).
+    // Two blocks per wave gain nothing from it (1,354 and 1,373 us).
+    constexpr bool SPLIT = BPW >= kSplitBlocks;
+    const bool units = SPLIT && blockIdx.x < a.long_groups;
+    uint32_t unit = blockIdx.x;
 
     for (;;) {
-        uint32_t item = blockIdx.x;
+        uint32_t item = SPLIT ? blockIdx.x - a.long_groups : blockIdx.x;
+        uint32_t kmask = ~0u;   // the blocks k of a lane that this pass takes
         int slot = wave;
         if (a.persistent) {
             // Unit u of queue q is wave slot u % WAVES of the queue's
@@ -264,8 +264,22 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
             }
             if (tried == kRasterQueues) break;
         }
-        if (item >= a.tiles) break;
-        const uint32_t tile = __builtin_amdgcn_readfirstlane(a.order ? a.order[item] : item);
+        if (units) {
+            // units u, u + 8, ... of eight tiles are the eight's blocks 0, 1, ...:
+            // a tile's are taken by workgroups of one XCD
+            const uint32_t t = unit / (kRasterQueues * BPW) * kRasterQueues + unit % kRasterQueues;
+            if (unit / (kRasterQueues * BPW) * kRasterQueues >= uniform_ptr(a.longs)[0]) break;
+            kmask = 1u << unit / kRasterQueues % BPW;
+            unit += a.long_groups;
+            if (t >= uniform_ptr(a.longs)[0]) continue;
+            item = uniform_ptr(a.long_tiles)[t];
+        } else if (item >= a.tiles) {
+            break;
+        }
+        const uint32_t tile = units ? item : __builtin_amdgcn_readfirstlane(a.order ? a.order[item] : item);
+        const uint2 range = uniform_ptr(a.tile_range)[tile];
+        const uint32_t lbeg = range.x, lend = range.y;
+        if (SPLIT && a.long_groups && !units && lend > lbeg && lend - lbeg >= uniform_ptr(a.longs)[1]) break;
         const uint64_t t_begin = clock64();
 
         const uint32_t ti = find_target(uniform_ptr(a.targets), a.target_count, tile);
@@ -291,7 +305,7 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
             const int bx0 = tile_x0 + (blk % BW) * 8, by0 = tile_y0 + (blk / BW) * 8;
             pxx[k] = bx0 + (lane & 7);
             pxy[k] = by0 + (lane >> 3);
-            inside[k] = pxx[k] < (int)tp.width && pxy[k] < (int)tp.height;
+            inside[k] = pxx[k] < (int)tp.width && pxy[k] < (int)tp.height && (!SPLIT || (kmask >> k & 1u));
 #pragma unroll
             for (int w = 0; w < 4; w++) px[k].color[w] = tp.clear_color[w];
             px[k].ds0 = tp.clear_ds[0];
@@ -369,8 +383,6 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
         };
 
         // ---- walk the tile's primitives in submission order
-        const uint2 range = uniform_ptr(a.tile_range)[tile];
-        const uint32_t lbeg = range.x, lend = range.y;
         // The pairs that name one of this wave's blocks (the emit kernels pack
         // a primitive's blocks, or for 32x32 tiles 16x16 quadrants, into the
         // pair) are its candidates: fetch() gives the next up to 64 of them,
@@ -383,12 +395,13 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
         uint32_t mine = 0u;
         if (TILE == 16) {
 #pragma unroll
-            for (int k = 0; k < BPW; k++) mine |= 1u << (kPairBlockShift + slot + k * WAVES);
+            for (int k = 0; k < BPW; k++)
+                if (!SPLIT || (kmask >> k & 1u)) mine |= 1u << (kPairBlockShift + slot + k * WAVES);
         } else if (TILE == 32) {
 #pragma unroll
             for (int k = 0; k < BPW; k++) {
                 const int blk = slot + k * WAVES;
-                mine |= 1u << (kPairBlockShift + (blk / BW) / 2 * 2 + (blk % BW) / 2);
+                if (!SPLIT || (kmask >> k & 1u)) mine |= 1u << (kPairBlockShift + (blk / BW) / 2 * 2 + (blk % BW) / 2);
             }
         }
         const bool packed = TILE != 8 && lend > lbeg && lend - lbeg > 64u;   // wave-uniform
@@ -456,18 +469,6 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
             bool ov = ok_next;
             chunk = more();
             prefetch();
-            // the candidates' visit fields, all lanes at once, straight into
-            // the wave's LDS region (global_load_lds: no registers)
-            if constexpr (GATHER) {
-                wave_lds_fence();   // the previous chunk's reads come first
-                if (ov) {
-                    const uint4* src = (const uint4*)&a.recs[gp_l];
-#pragma unroll
-                    for (int p = 0; p < kVisitParts; p++)
-                        __builtin_amdgcn_global_load_lds((const void*)(src + p),
-                                                         (__attribute__((address_space(3))) void*)&stage[wave][p][0], 16, 0, 0);
-                }
-            }
             // Hierarchical culling: a primitive whose depth interval fails
             // the test against every depth stored in the wave's pixels
             // cannot change any of them.  With LESS and LESS_OR_EQUAL the
@@ -539,10 +540,6 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
                 return m;
             };
             uint64_t mask = lanes(ov);
-            if constexpr (STAGE) {
-                __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): the LDS loads have landed
-                wave_lds_fence();
-            }
             int since = kCullVisits;   // candidates visited since the last cull
             const int step = packed ? kCullLanes : 64;
             for (int first = 0; first < 64; first += step) {
@@ -559,24 +556,11 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
                 const uint32_t gprim = __builtin_amdgcn_readlane(gp_l, j);
                 const uint32_t blocks = (TILE >= 16 && BPW > 1) ? __builtin_amdgcn_readlane(blocks_l, j) : 0u;
                 TriSetup r;
-                if constexpr (STAGE) {
-                    uint32_t* dst = (uint32_t*)&r;
-#pragma unroll
-                    for (int p = 0; p < kVisitParts; p++) {
-                        // uniform words: kept in scalar registers
-                        const uint4 v = stage[wave][p][j];
-                        dst[4 * p + 0] = __builtin_amdgcn_readfirstlane(v.x);
-                        dst[4 * p + 1] = __builtin_amdgcn_readfirstlane(v.y);
-                        dst[4 * p + 2] = __builtin_amdgcn_readfirstlane(v.z);
-                        dst[4 * p + 3] = __builtin_amdgcn_readfirstlane(v.w);
-                    }
-                } else {
-                    load_record_uniform(a.recs, gprim, r);
-                    // the loads of all visit fields issued before the first of
-                    // them is used: one memory latency per survivor, not one
-                    // for the draw index and another for the rest
-                    __asm__ volatile("" ::"s"(r.ax[0]), "s"(r.y1), "s"(r.dt_lo), "s"(r.draw_flags), "s"(r.z[0]), "s"(r.rinv));
-                }
+                load_record_uniform(a.recs, gprim, r);
+                // the loads of all visit fields issued before the first of
+                // them is used: one memory latency per survivor, not one
+                // for the draw index and another for the rest
+                __asm__ volatile("" ::"s"(r.ax[0]), "s"(r.y1), "s"(r.dt_lo), "s"(r.draw_flags), "s"(r.z[0]), "s"(r.rinv));
                 const uint32_t flags = r.draw_flags >> kPrimFlagShift;
                 if ((r.draw_flags & kPrimDraw) != cur_draw) {
                     cur_draw = r.draw_flags & kPrimDraw;
@@ -606,6 +590,7 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
                 for (int k = 0; k < BPW; k++) {
                     const int blk = slot + k * WAVES;
                     const int bx0 = tile_x0 + (blk % BW) * 8, by0 = tile_y0 + (blk / BW) * 8;
+                    if (SPLIT && !(kmask >> k & 1u)) continue;   // wave-uniform
                     if (TILE == 16 && BPW > 1) {
                         if (!((blocks >> blk) & 1u)) continue;   // wave-uniform
                     } else if (BPW > 1) {
@@ -755,7 +740,7 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
         if (a.count && lane == 0 && nfrag) atomicAdd(a.fragments, nfrag);
         if (a.trace_cycles && lane == 0) a.trace_cycles[(uint64_t)tile * WAVES + slot] = (float)(clock64() - t_begin);
 
-        if (!a.persistent) break;
+        if (!a.persistent && !units) break;
     }
 }
 

@@ -118,3 +118,29 @@ def test_list_lengths(ctx, tile, waves, op):
         s.clear_depth = 0.0 if op == "GREATER" else 1.0
         _check(ctx, s, f"lists of up to {n} {op} {tile}x{waves}", tile, waves, count=False)
     _check(ctx, s, f"lists of up to {n} {op} {tile}x{waves} counting", tile, waves)
+
+
+@pytest.mark.parametrize("tile,waves", [(16, 1), (32, 1), (32, 2), (32, 4)])
+@pytest.mark.parametrize("n,w,h,size", [(4200, 333, 211, 40.0), (4200, 40, 33, 16.0), (250_000, 640, 360, 6.0)])
+def test_long_tiles(ctx, tile, waves, n, w, h, size):
+    """Waves that hold four blocks or more take long tiles (256 pairs) block by block: tiles on both sides of the rule, all
+    tiles long, and more units of work than the 2,048 workgroups that take them; recorded batches and allocation-free
+    calls."""
+    s = S.soup(n, w, h, seed=n + w, size_px=np.log(size))
+    _check(ctx, s, f"{n} triangles {w}x{h} {tile}x{waves}", tile, waves)
+    ref = oracle_lib.render_scene(s, threads=oracle_lib.default_threads())
+    mem, ms, jobs = materialize_jobs(ctx, [s])
+    try:
+        with ctx.batch(jobs) as b:
+            for _ in range(3):
+                b.submit()
+            assert b.wait(count=True) == ref[2]
+        compare_jobs([s], ms, [ref], "batch")
+        if n < 10_000:
+            for m in ms:
+                m.reset_attachments()
+            ctx.render_pass_noalloc(ms[0].pass_desc, ms[0].pipelines, ms[0].draws)
+            ctx.synchronize()
+            compare_jobs([s], ms, [ref], "noalloc")
+    finally:
+        mem.release()

@@ -33,9 +33,9 @@ struct FillArgs {
 // Each thread takes 16-byte aligned chunks: a chunk inside its row is one
 // store, at a row's ends the pixels inside are stored one by one.  A pixel's
 // size divides 16 and its address, so every chunk holds the same pattern.
-// Bound by HBM writes: 64 MiB in 12.0 us (5.6 TB/s; as whole words 11.6), a
-// clear of 3840x2160 RGBA8 in 7.8 us (4.3 TB/s; one 4-byte store a thread,
-// with the packing on the device, took 28).
+// Bound by HBM writes: 64 MiB in 11.1 us (6.0 TB/s; as whole words 11.4),
+// 1 GiB in 154 us (7.0 TB/s; 203), a clear of 3840x2160 RGBA8 in 6.6 us (5.0
+// TB/s; one 4-byte store a thread, with the packing on the device, took 28).
 __global__ __launch_bounds__(256) void fill_rows_kernel(FillArgs a)
 {
     const uint4 v = make_uint4(a.pattern[0], a.pattern[1], a.pattern[2], a.pattern[3]);
@@ -273,6 +273,8 @@ uint32_t grid_for(uint64_t n)
     return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((n + 255) / 256, 16384));
 }
 
+constexpr uint64_t kFillCached = (128u << 20) / 16;   // 16-byte chunks
+
 // Enqueues rows of a repeated pixel of `size` bytes (dividing 16 and every
 // row's address).
 int fill_rows(cpv_context* c, uint64_t dst, uint64_t row_bytes, uint64_t pitch, uint32_t rows, uint32_t size, const uint32_t* pixel)
@@ -288,8 +290,11 @@ int fill_rows(cpv_context* c, uint64_t dst, uint64_t row_bytes, uint64_t pitch, 
     for (uint32_t o = 0; o < 16; o += size) std::memcpy((uint8_t*)a.pattern + o, pixel, size);
     void* args[] = {&a};
     const dim3 block = rows == 1 ? dim3(256, 1) : dim3(64, 4);
-    // about 4 chunks a thread once the chip is full
-    const uint64_t gx = std::min<uint64_t>((a.chunks + block.x - 1) / block.x, rows == 1 ? 4096 : 64);
+    // One run of up to 128 MiB by 1,024 workgroups (64 MiB in 11.1 us, with a
+    // chunk per thread 12.1), a longer one, past what the caches take, by a
+    // chunk per thread (1 GiB in 154 us, by 1,024 workgroups 224).
+    const uint64_t most = rows > 1 ? 64 : a.chunks > kFillCached ? 1u << 23 : 1024;
+    const uint64_t gx = std::min<uint64_t>((a.chunks + block.x - 1) / block.x, most);
     const uint32_t gy = std::min<uint32_t>((rows + block.y - 1) / block.y, 16384);
     HIP_TRY(hipLaunchKernel((const void*)fill_rows_kernel, dim3((uint32_t)gx, gy), block, args, 0, c->stream));
     return CPV_OK;

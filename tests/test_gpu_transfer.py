@@ -159,11 +159,13 @@ def test_clear_rows_of_every_pixel_size(gpu_ctx, mem, fmt):
         assert np.array_equal(mem.read(d, img.nbytes), want), (fmt, w, h)
 
 
-def test_fill_longer_than_the_grid(gpu_ctx, mem):
-    buf = rand_bytes((40 << 20) + 64)
+@pytest.mark.parametrize("mib", [40, 128, 130])
+def test_fill_longer_than_the_grid(gpu_ctx, mem, mib):
+    """Several chunks a thread, and a chunk per thread past 128 MiB."""
+    buf = rand_bytes((mib << 20) + 64)
     d = mem.alloc(buf)
     want = buf.copy()
-    size = (40 << 20) - 24
+    size = (mib << 20) - 24
     oracle_lib.fill_buffer(want, size, 0x01020304, 36)
     print("[transfer] long fill", flush=True)
     gpu_ctx.fill_buffer(d + 36, size, 0x01020304)

@@ -432,8 +432,10 @@ struct ScanArgs {
     uint32_t cap;            // capacity of the pair arrays
     uint64_t* total;         // the grand total, in 64 bits
     uint32_t* kept;          // pairs kept for sorting: min(total, cap)
-    uint32_t* overflow;      // raised when total exceeds cap: then the emit kernels write only the pairs
+    uint32_t* overflow;      // set when total exceeds cap: then the emit kernels write only the pairs
                              // below cap and the raster kernel draws nothing
+    uint32_t shared;         // 1: several launches share the overflow word, which their front half has cleared
+                             // and each may only raise; 0: the word is this launch's, and holds its answer alone
     uint32_t* big;           // emit_big_kernel's list, emptied
     uint32_t* host;          // pinned host words: total (two), overflow (nullptr: not wanted)
     uint32_t* longs;         // long_tiles_kernel's count, cleared, and the pairs from which a list is long
@@ -486,12 +488,13 @@ __global__ __launch_bounds__(kScanThreads) void scan_blocks_kernel(ScanArgs a)
         a.longs[0] = 0u;
         a.longs[1] = max(kLongPairs, (uint32_t)(min(carry, (uint64_t)a.cap) / kLongShare));
         *a.kept = carry < (uint64_t)a.cap ? (uint32_t)carry : a.cap;
-        if (carry > (uint64_t)a.cap) *a.overflow = 1u;
+        const uint32_t over = carry > (uint64_t)a.cap ? 1u : 0u;
+        if (over || !a.shared) *a.overflow = over;
         a.big[0] = 0u;
         if (a.host) {
             a.host[0] = (uint32_t)carry;
             a.host[1] = (uint32_t)(carry >> 32);
-            a.host[2] = carry > (uint64_t)a.cap ? 1u : 0u;
+            a.host[2] = over;
         }
     }
 }

@@ -426,7 +426,7 @@ int enqueue_front(Exec& x, const LaunchPlan& P, uint8_t* arena, uint32_t pair_ca
     if (P.small) return CPV_OK;
     ScanArgs ca{b.sums.as<uint64_t>(), P.prim_total ? (uint32_t)P.sblock.size() : 0u, std::max(pair_cap, 1u),
                 (uint64_t*)(stats + kStatPairTotal), stats + kStatPairs, x.overflow ? x.overflow : stats + kStatOverflow,
-                b.big.as<uint32_t>(), x.host_total, stats + kStatLong};
+                x.overflow ? 1u : 0u, b.big.as<uint32_t>(), x.host_total, stats + kStatLong};
     hipLaunchKernelGGL(scan_blocks_kernel, dim3(1), dim3(kScanThreads), 0, x.s, ca);
     HIP_TRY(hipGetLastError());
     return CPV_OK;
@@ -566,7 +566,9 @@ int enqueue_raster(Exec& x, const LaunchPlan& P, uint8_t* arena, const Binned& b
     ra.order = order;
     ra.queue = stats + kStatQueues;
     ra.fragments = x.fragments ? x.fragments : (unsigned long long*)(stats + kStatFragments);
-    ra.overflow = x.overflow ? x.overflow : stats + kStatOverflow;
+    // a small launch has no pairs to lose: only a word that other launches
+    // may have raised is its concern
+    ra.overflow = x.overflow ? x.overflow : P.small ? nullptr : stats + kStatOverflow;
     ra.trace_cycles = x.cfg.record_costs ? b.traces.as<float>() : nullptr;
     ra.vout_stride = P.stride;
     ra.tiles = P.tiles;
@@ -673,7 +675,7 @@ int enqueue_checked(cpv_context* c, PendingLaunch& L)
     if (rc) return rc;
     const bool fresh = B.stats.p == nullptr;
     if (B.stats.ensure(kStatAlloc * 4)) return CPV_ERROR_OUT_OF_MEMORY;
-    if (fresh) fill_u32(fs, B.stats.p, 0u, kStatAlloc);   // the overflow word starts clear
+    if (fresh) fill_u32(fs, B.stats.p, 0u, kStatAlloc);
     Exec x = context_exec(c, &B);
     x.cfg = L.cfg;
     x.s = fs;
@@ -896,8 +898,7 @@ int cpvrt::resolve_pending(cpv_context* c, bool may_allocate)
                   (unsigned long long)total, L->scratch_cap);
     else if (may_allocate) {
         c->pair_cap = std::min<uint64_t>(total + total / 8 + 4096, UINT32_MAX);
-        fill_u32(c->stream, c->lbuf[L->set].stats.as<uint32_t>() + kStatOverflow, 0u, 1);
-        c->chain_seq = ~0ull;   // the redraw's front half waits for the context stream (the fill, the skipped raster)
+        c->chain_seq = ~0ull;   // the redraw's front half waits for the context stream (the skipped raster kernel)
         rc = enqueue_checked(c, *L);
     } else {
         Buffers probe;

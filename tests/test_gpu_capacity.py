@@ -94,3 +94,63 @@ def test_more_than_2_32_pairs_refused(fresh_ctx):
         compare(small, (ms.read_color(), ms.read_ds(), fresh_ctx.fragment_count()), ref, "after the refusal")
     finally:
         mem.release()
+
+
+def _four_frames(ctx, mem, label):
+    """Two frames in each of the context's two buffer sets, of a launch whose tile lists one kernel writes and of one that
+    bins pairs, each equal to the oracle."""
+    for scene in (W.soup_scene(2000, 160, 120, seed=11), W.soup_scene(6000, 160, 120, seed=12)):
+        ref = oracle_lib.render_scene(scene)
+        m = materialize(scene, mem)
+        for k in range(4):
+            m.reset_attachments()
+            ctx.render_pass(m.pass_desc, m.pipelines, m.draws)
+            ctx.synchronize()
+            compare(scene, (m.read_color(), m.read_ds(), ctx.fragment_count()), ref, f"{label}, {scene.draws[0].count // 3} triangles, frame {k}")
+
+
+@pytest.mark.parametrize("small_first", [False, True])
+def test_frames_after_a_refusal(fresh_ctx, small_first):
+    """A launch refused for its 5.2e9 pairs leaves nothing behind: every later launch in its buffer set draws."""
+    scene = big_triangles(40_000, 3840, 2160, seed=5, load=True)
+    mem = DeviceMemory(fresh_ctx)
+    try:
+        if small_first:   # the refused launch then runs in the second buffer set
+            m = materialize(W.soup_scene(100, 64, 64, seed=3), mem)
+            fresh_ctx.render_pass(m.pass_desc, m.pipelines, m.draws)
+        fresh_ctx.set_config(tile_size=8, waves_per_tile=1)
+        m = materialize(scene, mem)
+        print("[capacity] refused launch", flush=True)
+        fresh_ctx.render_pass(m.pass_desc, m.pipelines, m.draws)
+        with pytest.raises(cpvulkan_amd.CpvError, match="more than 2\\^32 - 1"):
+            fresh_ctx.synchronize()
+        _four_frames(fresh_ctx, mem, "after the refusal")
+    finally:
+        mem.release()
+
+
+@pytest.mark.parametrize("side", [160, 320])   # 1.5M and 6M pairs: the allocation-free call's array holds the first only
+def test_frames_after_an_overflow_found_by_an_allocation_free_call(fresh_ctx, side):
+    """An overflowed launch that an allocation-free call finds is drawn again in that call's array, or given up: later
+    launches in the overflowed launch's buffer set draw all the same."""
+    scene = big_triangles(5000, side, side * 3 // 4, seed=7)
+    other = W.soup_scene(500, 96, 64, seed=2)
+    ref = oracle_lib.render_scene(other)
+    fresh_ctx.set_config(tile_size=8, waves_per_tile=1)
+    mem = DeviceMemory(fresh_ctx)
+    try:
+        m, o = materialize(scene, mem), materialize(other, mem)
+        print(f"[capacity] overflow, then noalloc, {side}", flush=True)
+        fresh_ctx.render_pass(m.pass_desc, m.pipelines, m.draws)
+        if side == 160:
+            fresh_ctx.render_pass_noalloc(o.pass_desc, o.pipelines, o.draws)
+            fresh_ctx.synchronize()
+            compare(other, (o.read_color(), o.read_ds(), fresh_ctx.fragment_count()), ref, "the allocation-free call")
+            want = oracle_lib.render_scene(scene, threads=oracle_lib.default_threads())
+            compare(scene, (m.read_color(), m.read_ds(), None), want, "drawn again in the array")
+        else:
+            with pytest.raises(cpvulkan_amd.CpvError, match="more than the allocation-free entry point holds"):
+                fresh_ctx.render_pass_noalloc(o.pass_desc, o.pipelines, o.draws)
+        _four_frames(fresh_ctx, mem, "after the overflow")
+    finally:
+        mem.release()

@@ -10,6 +10,7 @@
 #pragma once
 #pragma clang fp contract(off)
 
+#include "index_math.h"
 #include "raster_device.h"
 
 namespace cpv {
@@ -875,18 +876,10 @@ __global__ __launch_bounds__(256) void bin_small_kernel(SmallBinArgs a)
 // a digit's run holds a segment's items in key order (the earlier passes
 // sorted them), so a tile's items form runs whose ends it takes the minimum
 // and maximum of.
-constexpr int kSortSegments = 1024;
 constexpr int kSortThreads = 256;
 constexpr int kSortWaves = kSortThreads / 64;
 constexpr int kSortRounds = 8;                              // 64-item rounds per wave and tile
-constexpr int kSortTile = kSortThreads * kSortRounds;       // 2048 items
-
-__device__ __forceinline__ void segment_range(uint32_t n, uint32_t seg, uint32_t& b, uint32_t& e)
-{
-    const uint32_t per = ((n + kSortSegments - 1) / kSortSegments + 63u) & ~63u;
-    b = min(n, seg * per);
-    e = min(n, b + per);
-}
+static_assert(kSortTile == kSortThreads * kSortRounds, "a thread takes one item a round");
 
 // ranges, when given, are emptied (first = 2^32 - 1, last = 0) for the pass
 // that will fill them.
@@ -904,16 +897,17 @@ __global__ __launch_bounds__(kSortThreads) void radix_hist_kernel(const uint32_t
     uint32_t b, e;
     segment_range(*n_ptr, blockIdx.x, b, e);
     // kSortRounds keys per thread loaded before they are counted, so the loads overlap
-    for (uint32_t i0 = b; i0 < e; i0 += (uint32_t)kSortTile) {
+    for (uint32_t t0 = b; t0 < e; t0 += tile_items(t0, e)) {
+        const uint32_t n = tile_items(t0, e);
         uint32_t ks[kSortRounds];
 #pragma unroll
         for (int r = 0; r < kSortRounds; r++) {
-            const uint32_t i = i0 + (uint32_t)r * kSortThreads + threadIdx.x;
-            ks[r] = i < e ? keys[i] : 0u;
+            const uint32_t o = (uint32_t)r * kSortThreads + threadIdx.x;
+            ks[r] = o < n ? keys[t0 + o] : 0u;
         }
 #pragma unroll
         for (int r = 0; r < kSortRounds; r++)
-            if (i0 + (uint32_t)r * kSortThreads + threadIdx.x < e) atomicAdd(&s_cnt[wave][(ks[r] >> shift) & 255u], 1u);
+            if ((uint32_t)r * kSortThreads + threadIdx.x < n) atomicAdd(&s_cnt[wave][(ks[r] >> shift) & 255u], 1u);
     }
     __syncthreads();
     uint32_t c = 0;
@@ -956,22 +950,23 @@ __global__ __launch_bounds__(kSortThreads) void radix_scatter_kernel(const uint3
     uint32_t items;
     s_run[d_me] = block_exclusive_scan(totals[d_me], s_tmp, items) + base[d_me * kSortSegments + blockIdx.x];
     const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    for (uint32_t t0 = b; t0 < e; t0 += (uint32_t)kSortTile) {
+    for (uint32_t t0 = b; t0 < e; t0 += tile_items(t0, e)) {
+        const uint32_t n = tile_items(t0, e);
 #pragma unroll
         for (int w = 0; w < kSortWaves; w++) s_cnt[w][d_me] = 0;
         __syncthreads();
         // this wave's quarter of the tile: kSortRounds rounds of 64 consecutive items
-        const uint32_t w0 = t0 + (uint32_t)wave * (64u * kSortRounds);
+        const uint32_t w0 = (uint32_t)wave * (64u * kSortRounds);
         uint32_t ks[kSortRounds], vs[kSortRounds], rk[kSortRounds];
 #pragma unroll
         for (int r = 0; r < kSortRounds; r++) {
-            const uint32_t i = w0 + (uint32_t)r * 64u + (uint32_t)lane;
-            ks[r] = i < e ? keys_in[i] : 0u;
-            vs[r] = i < e ? vals_in[i] : 0u;
+            const uint32_t o = w0 + (uint32_t)r * 64u + (uint32_t)lane;
+            ks[r] = o < n ? (keys_in + t0)[o] : 0u;
+            vs[r] = o < n ? (vals_in + t0)[o] : 0u;
         }
 #pragma unroll
         for (int r = 0; r < kSortRounds; r++) {
-            const bool valid = w0 + (uint32_t)r * 64u + (uint32_t)lane < e;
+            const bool valid = w0 + (uint32_t)r * 64u + (uint32_t)lane < n;
             const uint32_t dg = (ks[r] >> shift) & 255u;
             // lanes of this round holding the same digit
             uint64_t match = __ballot(valid);
@@ -1005,7 +1000,7 @@ __global__ __launch_bounds__(kSortThreads) void radix_scatter_kernel(const uint3
         // the tile in digit order, in LDS
 #pragma unroll
         for (int r = 0; r < kSortRounds; r++) {
-            if (w0 + (uint32_t)r * 64u + (uint32_t)lane < e) {
+            if (w0 + (uint32_t)r * 64u + (uint32_t)lane < n) {
                 const uint32_t dg = (ks[r] >> shift) & 255u;
                 const uint32_t pos = s_start[dg] + s_cnt[wave][dg] + rk[r];
                 s_keys[pos] = ks[r];

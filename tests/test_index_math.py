@@ -1,0 +1,46 @@
+"""Index arithmetic of the kernels (csrc/index_math.h), compiled for the host, at the ends of its ranges."""
+import ctypes as C
+import subprocess
+from pathlib import Path
+
+import numpy as np
+import pytest
+
+CSRC = Path(__file__).resolve().parent.parent / "cpvulkan_amd" / "csrc"
+
+SOURCE = """
+#include "index_math.h"
+extern "C" void segment(unsigned n, unsigned seg, unsigned* be) { cpv::segment_range(n, seg, be[0], be[1]); }
+extern "C" unsigned items(unsigned t0, unsigned e) { return cpv::tile_items(t0, e); }
+"""
+
+
+@pytest.fixture(scope="module")
+def lib(tmp_path_factory):
+    d = tmp_path_factory.mktemp("index_math")
+    (d / "m.cpp").write_text(SOURCE)
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", f"-I{CSRC}", "-o", str(d / "m.so"), str(d / "m.cpp")], check=True)
+    return C.CDLL(str(d / "m.so"))
+
+
+@pytest.mark.parametrize("n", [0, 1, 63, 64, 65, 1023, 1024, 65535, 65536, 65537, 2**20, 2**31, 2**32 - 65537, 2**32 - 65536, 2**32 - 65535,
+                               2**32 - 4096, 2**32 - 1024, 2**32 - 1023, 2**32 - 2, 2**32 - 1])
+def test_sort_segments_cover_every_pair(lib, n):
+    """The segments follow each other from 0 to n, and a workgroup's walk takes every item of its own and ends."""
+    be, at = (C.c_uint32 * 2)(), 0
+    for seg in range(1024):
+        lib.segment(C.c_uint32(n), C.c_uint32(seg), be)
+        b, e = be
+        assert b == at and e >= b, (n, seg, b, e)
+        at = e
+    assert at == n
+    # the last segment that holds anything (the one nearest to 2^32), from two tiles before its end
+    t0, e = max(n - 5000, 0), n
+    steps = 0
+    while t0 < e:
+        k = int(np.uint32(lib.items(C.c_uint32(t0), C.c_uint32(e))))
+        assert 1 <= k <= 2048 and (k == 2048 or t0 + k == e)
+        t0 = (t0 + k) & 0xFFFFFFFF   # the kernels' 32-bit sum
+        steps += 1
+        assert steps <= 3
+    assert t0 == e

@@ -56,7 +56,7 @@ def _obj(src: Path, out_dir: Path, hip: bool, defines: tuple = (), tag: str = ""
 
 # Kernel headers a translated SPIR-V program is compiled against (hiprtc has
 # no file system access to the source tree, so the library carries them).
-RTC_HEADERS = ["cpv_types.h", "raster_device.h", "raster_kernels.h", "raster_tile.h"]
+RTC_HEADERS = ["cpv_types.h", "index_math.h", "raster_device.h", "raster_kernels.h", "raster_tile.h"]
 
 
 def write_embedded_headers(out: Path) -> Path:

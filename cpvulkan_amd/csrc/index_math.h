@@ -34,4 +34,33 @@ CPV_INDEX void segment_range(uint32_t n, uint32_t seg, uint32_t& b, uint32_t& e)
 // 2^32; items are told from what lies beyond by their offset in the tile.
 CPV_INDEX uint32_t tile_items(uint32_t t0, uint32_t e) { return e - t0 < (uint32_t)kSortTile ? e - t0 : (uint32_t)kSortTile; }
 
+// Whether a texture level's texels may be read without a bounds test: its
+// wrapped coordinates lie inside whatever the coordinate, and every texel's
+// offset fits 32 bits.  MIRRORED_REPEAT sums two remainders by twice the
+// extent, which pass 2^31 for extents above 2^29, so wider levels keep the
+// test; so does an empty one.
+CPV_INDEX bool plain_extent(uint32_t w, uint32_t h)
+{
+    return (uint64_t)w * h - 1ull < (1ull << 30) && w <= (1u << 29) && h <= (1u << 29);
+}
+
+// wrap (CPVulkan/ImageSampler.cpp:12-38)
+CPV_INDEX int32_t wrap_coord(int32_t v, int32_t size, int32_t mode)
+{
+    if (mode == 0) {                                                       // REPEAT: (v % size + size) % size
+        if ((size & (size - 1)) == 0) return v & (size - 1);               // no division for sizes 2^k
+        const int32_t m = v % size;
+        return m < 0 ? m + size : m;
+    }
+    if (mode == 1) {                                                       // MIRRORED_REPEAT
+        const int32_t two = 2 * size;
+        const int32_t n = (v % two + two) % two - size;
+        return size - 1 - (n >= 0 ? n : -(1 + n));
+    }
+    if (mode == 2) return v < 0 ? 0 : (v > size - 1 ? size - 1 : v);       // CLAMP_TO_EDGE
+    if (mode == 3) return v < -1 ? -1 : (v > size ? size : v);             // CLAMP_TO_BORDER
+    const int32_t m = v >= 0 ? v : -(1 + v);                               // MIRROR_CLAMP_TO_EDGE
+    return m < 0 ? 0 : (m > size - 1 ? size - 1 : m);
+}
+
 }  // namespace cpv

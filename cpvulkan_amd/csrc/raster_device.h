@@ -9,7 +9,7 @@
 #pragma once
 #pragma clang fp contract(off)
 
-#include "cpv_types.h"
+#include "index_math.h"
 
 namespace cpv {
 
@@ -240,25 +240,6 @@ struct TextureDesc {
     SamplerDesc sampler;
 };
 
-// wrap (CPVulkan/ImageSampler.cpp:12-38)
-CPV_DEV int32_t wrap_coord(int32_t v, int32_t size, int32_t mode)
-{
-    if (mode == 0) {                                                       // REPEAT: (v % size + size) % size
-        if ((size & (size - 1)) == 0) return v & (size - 1);               // no division for sizes 2^k
-        const int32_t m = v % size;
-        return m < 0 ? m + size : m;
-    }
-    if (mode == 1) {                                                       // MIRRORED_REPEAT
-        const int32_t two = 2 * size;
-        const int32_t n = (v % two + two) % two - size;
-        return size - 1 - (n >= 0 ? n : -(1 + n));
-    }
-    if (mode == 2) return v < 0 ? 0 : (v > size - 1 ? size - 1 : v);       // CLAMP_TO_EDGE
-    if (mode == 3) return v < -1 ? -1 : (v > size ? size : v);             // CLAMP_TO_BORDER
-    const int32_t m = v >= 0 ? v : -(1 + v);                               // MIRROR_CLAMP_TO_EDGE
-    return m < 0 ? 0 : (m > size - 1 ? size - 1 : m);
-}
-
 CPV_DEV void border_colour(int32_t b, float out[4])
 {
     const float rgb = (b >= 4) ? 1.0f : 0.0f;
@@ -300,8 +281,8 @@ CPV_DEV void lerp4(const float a[4], const float b[4], double t, float out[4])
     }
 }
 
-// A texture of four 8-bit UNORM channels in 4 bytes, no border mode and at most
-// 2^30 texels in the level: texels then come by 32-bit offsets, with no
+// A texture of four 8-bit UNORM channels in 4 bytes, no border mode and a
+// level that plain_extent admits: texels then come by 32-bit offsets, with no
 // bounds test (wrapped coordinates are inside) and no per-channel format
 // branches.  The tests are on scalars; the generic code takes about 40 of them
 // per bilinear sample.
@@ -310,7 +291,7 @@ CPV_DEV bool plain_texture(const TextureDesc& t, uint32_t level)
     const FormatDesc& f = t.fmt;
     return f.base == kBaseUNorm && f.element == 1 && f.total == 4 && (f.off[0] | f.off[1] | f.off[2] | f.off[3]) >= 0 &&
            t.sampler.address_u != 3 && t.sampler.address_v != 3 &&
-           (uint64_t)t.level_w[level] * t.level_h[level] - 1ull < (1ull << 30);   // an empty level takes the bounds tests
+           plain_extent(t.level_w[level], t.level_h[level]);
 }
 CPV_DEV void plain_texel(const TextureDesc& t, const uint32_t* base, uint32_t at, float out[4])
 {

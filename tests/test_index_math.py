@@ -11,6 +11,8 @@ CSRC = Path(__file__).resolve().parent.parent / "cpvulkan_amd" / "csrc"
 SOURCE = """
 #include "index_math.h"
 extern "C" void segment(unsigned n, unsigned seg, unsigned* be) { cpv::segment_range(n, seg, be[0], be[1]); }
+extern "C" int plain(unsigned w, unsigned h) { return cpv::plain_extent(w, h); }
+extern "C" int wrap(int v, int size, int mode) { return cpv::wrap_coord(v, size, mode); }
 extern "C" unsigned items(unsigned t0, unsigned e) { return cpv::tile_items(t0, e); }
 """
 
@@ -19,7 +21,7 @@ extern "C" unsigned items(unsigned t0, unsigned e) { return cpv::tile_items(t0, 
 def lib(tmp_path_factory):
     d = tmp_path_factory.mktemp("index_math")
     (d / "m.cpp").write_text(SOURCE)
-    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", f"-I{CSRC}", "-o", str(d / "m.so"), str(d / "m.cpp")], check=True)
+    subprocess.run(["g++", "-O1", "-fwrapv", "-std=c++17", "-shared", "-fPIC", f"-I{CSRC}", "-o", str(d / "m.so"), str(d / "m.cpp")], check=True)
     return C.CDLL(str(d / "m.so"))
 
 
@@ -44,3 +46,23 @@ def test_sort_segments_cover_every_pair(lib, n):
         steps += 1
         assert steps <= 3
     assert t0 == e
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2, 4])   # every address mode but CLAMP_TO_BORDER
+@pytest.mark.parametrize("size", [1, 2, 3, 5, 64, 1000, 16384, 2**29 - 1, 2**29, 2**29 + 1, 3 * 2**28, 2**30 - 1, 2**30])
+def test_texels_read_without_a_bounds_test_are_inside(lib, mode, size):
+    """Wherever the sampler leaves out the bounds test, the wrapped coordinate is a texel of the level."""
+    if not lib.plain(C.c_uint32(size), C.c_uint32(1)):
+        assert size > 16384   # no image that Vulkan's limits allow takes the slow path
+        return
+    rng = np.random.default_rng(size % 1000)
+    at = np.concatenate([np.arange(-5, 6), size * np.arange(-3, 4), size * np.arange(-3, 4) - 1, [-2**31, -2**31 + 1, 2**31 - 2, 2**31 - 1],
+                         rng.integers(-2**31, 2**31, 3000)])
+    for v in np.unique(at[(at >= -2**31) & (at < 2**31)]).tolist():
+        assert 0 <= lib.wrap(v, size, mode) < size, (v, size, mode)
+
+
+def test_plain_extents(lib):
+    for w, h, ok in [(0, 0, 0), (0, 7, 0), (7, 0, 0), (1, 1, 1), (16384, 16384, 1), (32768, 32768, 1), (32769, 32768, 0), (2**29, 2, 1),
+                     (2**29 + 1, 1, 0), (1, 2**30, 0), (2**32 - 1, 2**32 - 1, 0)]:
+        assert lib.plain(C.c_uint32(w), C.c_uint32(h)) == ok, (w, h)

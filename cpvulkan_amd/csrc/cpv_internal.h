@@ -44,8 +44,8 @@ enum : uint32_t {
     // waves add to the fragment counter at word 0 (sharing that line made
     // the raster kernel 30% slower)
     kStatOverflow = 32,
-    kStatLong = 33,       // tiles in the list of long ones
-    kStatLongFrom = 34,   // pairs from which a tile's list is long
+    kStatClear = 33,      // never written: what a launch reads in the place of an overflow word when it cannot overflow
+    kStatLong = 36,       // tiles in the list of long ones, then the pairs from which a tile's list is long
     kStatTiles = 11,      // tile count of the launch (length of the order sort)
     kStatPrio = 12,       // predicted log2 cost from which a tile is heavy and dispatched first (float bits)
     kStatPredMax = 13,    // the largest finite prediction, as an ordered integer

@@ -568,7 +568,7 @@ int enqueue_raster(Exec& x, const LaunchPlan& P, uint8_t* arena, const Binned& b
     ra.fragments = x.fragments ? x.fragments : (unsigned long long*)(stats + kStatFragments);
     // a small launch has no pairs to lose: only a word that other launches
     // may have raised is its concern
-    ra.overflow = x.overflow ? x.overflow : P.small ? nullptr : stats + kStatOverflow;
+    ra.overflow = x.overflow ? x.overflow : stats + (P.small ? kStatClear : kStatOverflow);
     ra.trace_cycles = x.cfg.record_costs ? b.traces.as<float>() : nullptr;
     ra.vout_stride = P.stride;
     ra.tiles = P.tiles;

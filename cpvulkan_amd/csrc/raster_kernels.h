@@ -74,7 +74,6 @@ struct RasterArgs {
     unsigned long long* fragments;  // covered (primitive, pixel) pairs
     float* trace_cycles;            // shader cycles per (tile, wave slot) (nullptr: not recorded)
     const uint32_t* overflow;       // set when the launch's pairs outgrew their arrays: then nothing is drawn
-                                    // (nullptr: they cannot)
     uint32_t vout_stride;
     uint32_t tiles;                 // total tiles over all targets
     uint32_t target_count;

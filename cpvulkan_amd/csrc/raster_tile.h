@@ -212,7 +212,7 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
     // Pairs that outgrew their arrays were dropped: the launch draws nothing
     // and leaves the attachments as they were, so that it can be run again
     // with larger arrays.
-    if (a.overflow && *a.overflow) return;
+    if (*a.overflow) return;
 
     // Each survivor's record is read with scalar loads.  Staging the visit
     // fields of a chunk's candidates through LDS (global_load_lds) where a wave

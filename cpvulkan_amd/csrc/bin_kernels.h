@@ -420,12 +420,9 @@ __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* s
 constexpr int kScanThreads = 256;
 constexpr int kScanItems = 16;
 
-// A tile is long, and its blocks are rastered by a wave each where a wave
-// holds several (RasterArgs::longs), from this many pairs on and from this
-// share of the launch's, about its even share among the resident waves.  The
-// 48-job batch with 16x16 tiles and one wave took 1,776 us a submit with 256
-// pairs, 1,771 with 128, 1,780 with 64, 2,238 with 32 and 2,125 unsplit.
-constexpr uint32_t kLongPairs = 256u, kLongShare = 8192u;
+// A tile may be long (LongTiles, below) from this many pairs on and from this
+// share of the launch's, about its even share among the resident waves.
+constexpr uint32_t kLongPairs = 256u, kLongShare = 4096u;
 
 struct ScanArgs {
     uint64_t* sums;          // in: pairs of each setup workgroup; out: their exclusive scan
@@ -439,7 +436,7 @@ struct ScanArgs {
                              // and each may only raise; 0: the word is this launch's, and holds its answer alone
     uint32_t* big;           // emit_big_kernel's list, emptied
     uint32_t* host;          // pinned host words: total (two), overflow (nullptr: not wanted)
-    uint32_t* longs;         // long_tiles_kernel's count, cleared, and the pairs from which a list is long
+    LongTiles* longs;        // emptied, with the least length of a long list and the pairs kept
 };
 
 // Exclusive scan of the setup workgroups' pair sums by one workgroup (4,096
@@ -486,9 +483,9 @@ __global__ __launch_bounds__(kScanThreads) void scan_blocks_kernel(ScanArgs a)
     }
     if (threadIdx.x == 0) {
         *a.total = carry;
-        a.longs[0] = 0u;
-        a.longs[1] = max(kLongPairs, (uint32_t)(min(carry, (uint64_t)a.cap) / kLongShare));
-        *a.kept = carry < (uint64_t)a.cap ? (uint32_t)carry : a.cap;
+        const uint32_t kept = carry < (uint64_t)a.cap ? (uint32_t)carry : a.cap;
+        *a.longs = LongTiles{0u, max(kLongPairs, kept / kLongShare), 0u, kept};
+        *a.kept = kept;
         const uint32_t over = carry > (uint64_t)a.cap ? 1u : 0u;
         if (over || !a.shared) *a.overflow = over;
         a.big[0] = 0u;
@@ -1031,13 +1028,16 @@ __global__ __launch_bounds__(kSortThreads) void radix_scatter_kernel(const uint3
     }
 }
 
-// The launch's long tiles, in any order.
-__global__ __launch_bounds__(256) void long_tiles_kernel(const uint2* ranges, uint32_t tiles, uint32_t* longs, uint32_t* list)
+// The tiles whose lists reach the least length, in any order, and the number
+// of tiles with any pairs.
+__global__ __launch_bounds__(256) void long_tiles_kernel(const uint2* ranges, uint32_t tiles, LongTiles* longs, uint32_t* list)
 {
     const uint32_t t = blockIdx.x * 256u + threadIdx.x;
-    if (t >= tiles) return;
-    const uint2 r = ranges[t];
-    if (r.y > r.x && r.y - r.x >= longs[1]) list[atomicAdd(longs, 1u)] = t;
+    const uint2 r = t < tiles ? ranges[t] : make_uint2(0u, 0u);
+    const uint32_t n = r.y > r.x ? r.y - r.x : 0u;
+    if (n && n >= longs->from) list[atomicAdd(&longs->count, 1u)] = t;
+    const uint32_t filled = (uint32_t)__syncthreads_count(n != 0u);
+    if (threadIdx.x == 0 && filled) atomicAdd(&longs->filled, filled);
 }
 
 }  // namespace cpv

@@ -45,7 +45,7 @@ enum : uint32_t {
     // the raster kernel 30% slower)
     kStatOverflow = 32,
     kStatClear = 33,      // never written: what a launch reads in the place of an overflow word when it cannot overflow
-    kStatLong = 36,       // tiles in the list of long ones, then the pairs from which a tile's list is long
+    kStatLong = 36,       // LongTiles, words 36-39
     kStatTiles = 11,      // tile count of the launch (length of the order sort)
     kStatPrio = 12,       // predicted log2 cost from which a tile is heavy and dispatched first (float bits)
     kStatPredMax = 13,    // the largest finite prediction, as an ordered integer

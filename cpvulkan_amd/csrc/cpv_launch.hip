@@ -426,15 +426,18 @@ int enqueue_front(Exec& x, const LaunchPlan& P, uint8_t* arena, uint32_t pair_ca
     if (P.small) return CPV_OK;
     ScanArgs ca{b.sums.as<uint64_t>(), P.prim_total ? (uint32_t)P.sblock.size() : 0u, std::max(pair_cap, 1u),
                 (uint64_t*)(stats + kStatPairTotal), stats + kStatPairs, x.overflow ? x.overflow : stats + kStatOverflow,
-                x.overflow ? 1u : 0u, b.big.as<uint32_t>(), x.host_total, stats + kStatLong};
+                x.overflow ? 1u : 0u, b.big.as<uint32_t>(), x.host_total, (LongTiles*)(stats + kStatLong)};
     hipLaunchKernelGGL(scan_blocks_kernel, dim3(1), dim3(kScanThreads), 0, x.s, ca);
     HIP_TRY(hipGetLastError());
     return CPV_OK;
 }
 
-// Workgroups that raster the long tiles' blocks: eight for each of the CUs,
-// a multiple of kRasterQueues.
-constexpr uint32_t kLongGroups = 2048u;
+// Workgroups that raster the split tiles' blocks, at most; a multiple of
+// kRasterQueues.  With 16x16 tiles and one wave, the clustered 1M soup took
+// 2,308 us a frame with 2,048, 1,944 with 4,096 and 1,830 with 8,192; a launch
+// that splits nothing pays for their dispatch (150k triangles at 1080p: 393
+// with 2,048, 405 with 8,192).
+constexpr uint32_t kLongGroups = 4096u;
 
 // The launch splits its long tiles: waves that hold kSplitBlocks or more, a
 // workgroup per tile (the counter-ordered queue balances by itself), and no
@@ -500,8 +503,8 @@ int enqueue_bin(Exec& x, const LaunchPlan& P, uint8_t* arena, uint32_t pair_cap,
     // of the sorted keys, which nothing reads any more (a long tile has
     // many pairs, so the list always fits)
     if (splits_long_tiles(x, P)) {
-        hipLaunchKernelGGL(long_tiles_kernel, dim3((P.tiles + 255) / 256), dim3(256), 0, x.s, ranges, P.tiles, stats + kStatLong,
-                           b.keys[0].as<uint32_t>());
+        hipLaunchKernelGGL(long_tiles_kernel, dim3((P.tiles + 255) / 256), dim3(256), 0, x.s, ranges, P.tiles,
+                           (LongTiles*)(stats + kStatLong), b.keys[0].as<uint32_t>());
         HIP_TRY(hipGetLastError());
     }
 
@@ -588,10 +591,13 @@ int enqueue_raster(Exec& x, const LaunchPlan& P, uint8_t* arena, const Binned& b
     ra.count = x.cfg.count_fragments ? 1u : 0u;
     uint32_t grid = P.tiles;
     if (splits_long_tiles(x, P)) {
-        ra.long_groups = kLongGroups;
+        // no more than there can be units: a tile's blocks over its waves, of the tiles in eights
+        const uint64_t units = (uint64_t)((P.tiles + kRasterQueues - 1) / kRasterQueues) * kRasterQueues * (x.cfg.tile_size / 8) *
+                               (x.cfg.tile_size / 8) / x.cfg.waves_per_tile;
+        ra.long_groups = (uint32_t)std::min<uint64_t>(kLongGroups, units);
         ra.long_tiles = b.keys[0].as<uint32_t>();
-        ra.longs = stats + kStatLong;
-        grid += kLongGroups;
+        ra.longs = (const LongTiles*)(stats + kStatLong);
+        grid += ra.long_groups;
     }
     if (ra.persistent) {
         const int resident = resident_workgroups(x, rk, block);

@@ -34,8 +34,16 @@ constexpr uint32_t kRasterQueues = 8;
 constexpr uint32_t kRasterQueueStride = 32;
 
 // Raster waves that hold at least this many 8x8 blocks take the blocks of
-// long tiles one by one (RasterArgs::longs).
+// long tiles one by one (LongTiles).
 constexpr int kSplitBlocks = 4;
+
+// What is known of a launch's tile lists when long ones are split.
+struct LongTiles {
+    uint32_t count;    // tiles whose list has `from` pairs or more (RasterArgs::long_tiles)
+    uint32_t from;     // the least length of a long list
+    uint32_t filled;   // tiles with any pairs
+    uint32_t pairs;    // the pairs of all tiles
+};
 
 // Channel base types of FormatInformation (CPVulkanBase/Formats.h:30-103).
 enum BaseType : int32_t {

@@ -85,11 +85,11 @@ struct RasterArgs {
     int32_t uniform_fstate;         // the fragment state every draw of the launch has, -1 when they differ
     uint32_t count;                 // covered fragments are counted
     // Kernels whose waves hold kSplitBlocks blocks or more: the first long_groups
-    // workgroups raster the launch's long tiles, a block of each wave's at a
+    // workgroups raster the launch's split tiles, a block of each wave's at a
     // time, and the tiles' own workgroups skip them (0: none is split)
     uint32_t long_groups;
     const uint32_t* long_tiles;
-    const uint32_t* longs;          // their count; the pairs from which a tile is long
+    const LongTiles* longs;         // what decides of each whether it is split (splits_tile)
 };
 
 // True when a depth in [lo, hi] fails `op` against every stored depth in

@@ -231,13 +231,9 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
     const int32_t hiz_op = a.hiz_op;
     const bool less = a.less_depth != 0;
     uint32_t tried = 0;   // queues found empty, starting at home
-    // A wave that holds many blocks walks a long tile's list once for all of
-    // them, one after the other: a serial chain that the launch may end up
-    // waiting for.  Long tiles are split, a unit of work per block (of each
-    // of the workgroup's waves), and start first.  The 48-job batch went from
-    // 2,125 to 1,776 us a submit with 16x16 tiles and one wave, with 32x32
-    // tiles from 2,337 to 1,873 (four waves) and from 7,295 to 3,568 (one).
-    // Two blocks per wave gain nothing from it (1,354 and 1,373 us).
+    // Split tiles (splits_tile) are units of work, one per block of each of the
+    // workgroup's waves, and start first.  Waves that hold two blocks gain
+    // nothing from it (48-job batch, 16x16 tiles: 1,354 us unsplit, 1,373).
     constexpr bool SPLIT = BPW >= kSplitBlocks;
     const bool units = SPLIT && blockIdx.x < a.long_groups;
     uint32_t unit = blockIdx.x;
@@ -268,10 +264,10 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
             // units u, u + 8, ... of eight tiles are the eight's blocks 0, 1, ...:
             // a tile's are taken by workgroups of one XCD
             const uint32_t t = unit / (kRasterQueues * BPW) * kRasterQueues + unit % kRasterQueues;
-            if (unit / (kRasterQueues * BPW) * kRasterQueues >= uniform_ptr(a.longs)[0]) break;
+            if (unit / (kRasterQueues * BPW) * kRasterQueues >= uniform_ptr(a.longs)->count) break;
             kmask = 1u << unit / kRasterQueues % BPW;
             unit += a.long_groups;
-            if (t >= uniform_ptr(a.longs)[0]) continue;
+            if (t >= uniform_ptr(a.longs)->count) continue;
             item = uniform_ptr(a.long_tiles)[t];
         } else if (item >= a.tiles) {
             break;
@@ -279,7 +275,11 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
         const uint32_t tile = units ? item : __builtin_amdgcn_readfirstlane(a.order ? a.order[item] : item);
         const uint2 range = uniform_ptr(a.tile_range)[tile];
         const uint32_t lbeg = range.x, lend = range.y;
-        if (SPLIT && a.long_groups && !units && lend > lbeg && lend - lbeg >= uniform_ptr(a.longs)[1]) break;
+        if (SPLIT && a.long_groups) {
+            const bool split = lend > lbeg && splits_tile(*uniform_ptr(a.longs), lend - lbeg, WAVES);
+            if (units && !split) continue;
+            if (!units && split) break;
+        }
         const uint64_t t_begin = clock64();
 
         const uint32_t ti = find_target(uniform_ptr(a.targets), a.target_count, tile);

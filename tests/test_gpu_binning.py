@@ -144,3 +144,18 @@ def test_long_tiles(ctx, tile, waves, n, w, h, size):
             compare_jobs([s], ms, [ref], "noalloc")
     finally:
         mem.release()
+
+
+@pytest.mark.parametrize("tile,waves,side", [(16, 1, 640), (32, 1, 1280), (32, 4, 640)])
+def test_some_tiles_split(ctx, tile, waves, side):
+    """A launch that fills the chip: of lists on both sides of the least length only those far beyond the mean are split."""
+    s = S.soup(250_000, side, side, seed=tile + waves, size_px=np.log(5.0))
+    rng = np.random.default_rng(9)
+    centres = rng.normal(0.3, 0.01, (20_000, 2))
+    v = W.soup_triangles(20_000, side, side, 5, centres=centres, mu_px=np.log(5.0))
+    s = copy.deepcopy(s)
+    d = copy.deepcopy(s.draws[0])
+    d.vertices = {0: v.view(np.uint8).reshape(-1)}
+    d.count = v.shape[0]
+    s.draws.append(d)
+    _check(ctx, s, f"{side}x{side} {tile}x{waves}", tile, waves)

@@ -66,3 +66,29 @@ def test_plain_extents(lib):
     for w, h, ok in [(0, 0, 0), (0, 7, 0), (7, 0, 0), (1, 1, 1), (16384, 16384, 1), (32768, 32768, 1), (32769, 32768, 0), (2**29, 2, 1),
                      (2**29 + 1, 1, 0), (1, 2**30, 0), (2**32 - 1, 2**32 - 1, 0)]:
         assert lib.plain(C.c_uint32(w), C.c_uint32(h)) == ok, (w, h)
+
+
+LONG = """
+#include "index_math.h"
+extern "C" int splits(unsigned from, unsigned filled, unsigned pairs, unsigned n, unsigned waves)
+{ return cpv::splits_tile(cpv::LongTiles{0, from, filled, pairs}, n, waves); }
+"""
+
+
+def test_which_tiles_are_split(tmp_path):
+    """Lists much alike are split only while their tiles leave the chip idle; lists far beyond the mean always."""
+    (tmp_path / "l.cpp").write_text(LONG)
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", f"-I{CSRC}", "-o", str(tmp_path / "l.so"), str(tmp_path / "l.cpp")],
+                   check=True)
+    splits = C.CDLL(str(tmp_path / "l.so")).splits
+    u = C.c_uint32
+    for waves in (1, 2, 4):
+        for filled, alike in ((1, 1), (300, 1), (1535 // waves, 1), (1536 // waves, 0), (8160, 0), (1 << 22, 0)):
+            n = 500
+            pairs = n * filled
+            at = max(256, pairs // 4096)
+            assert splits(u(at), u(filled), u(pairs), u(max(n, at)), u(waves)) == (alike or at >= 2 * n), (waves, filled)
+            assert not splits(u(at), u(filled), u(pairs), u(at - 1), u(waves))
+        # one tile in ten holds nine tenths of the pairs
+        assert splits(u(256), u(10_000), u(1_000_000), u(900), u(waves)) and not splits(u(256), u(10_000), u(9_000_000), u(900), u(waves))
+    assert splits(u(2**20), u(2**22), u(2**32 - 1), u(2**32 - 1), u(1))   # the products are taken in 64 bits

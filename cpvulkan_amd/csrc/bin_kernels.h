@@ -28,6 +28,7 @@ struct SetupArgs {
     uint64_t* sums;               // tiles overlapped by the primitives of each workgroup
     uint32_t stride;
     int32_t tile_shift;
+    uint32_t cull_mode;           // RasterArgs::cull_mode
 };
 
 // EdgeFunction(a, b, c) with c the pixel centre, stored as a, (b.y - a.y), (b.x - a.x).
@@ -361,6 +362,11 @@ __device__ uint32_t setup_triangle(const SetupArgs& a, const DrawDesc& d, uint32
         fast = fast && fabsf(P[k][0]) <= 0x1p20f && fabsf(P[k][1]) <= 0x1p20f && P[k][2] >= 0.0f && P[k][2] <= 0x1p20f;
     r.draw_flags = di | ((front ? kPrimFront : 0u) | (fast ? kPrimFast : 0u)) << kPrimFlagShift;
     depth_bounds(r, P, d);
+    if (a.cull_mode & kCullGreater) {
+        const float lo = r.dt_lo;
+        r.dt_lo = -r.dt_hi;
+        r.dt_hi = -lo;
+    }
     store_record(&a.recs[gp], r);
     return tiles_of(x0, y0, x1, y1, a.tile_shift);
 }

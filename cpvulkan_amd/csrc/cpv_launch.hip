@@ -70,7 +70,7 @@ struct LaunchPlan {
     int tile_shift = 4;
     int raster_variant = 3;          // index into Program::raster
     bool lines = false;              // some draw rasterises lines (LineExt records)
-    int32_t hiz_op = -1, hiz_kind = 32;
+    int32_t hiz_op = -1;
     int32_t less_depth = 0;          // RasterArgs::less_depth
     int32_t uniform_fstate = -1;     // every draw's fragment state is fstates[0] (0), or not (-1)
     // Small launches take bin_small_kernel in place of the scan, emit and sort
@@ -254,7 +254,6 @@ int plan_launch(const cpv_config& cfg, const Program& prog, const std::vector<Ta
     // raster kernel's short depth path takes launches whose every draw so
     // observes LESS or LESS_OR_EQUAL, counted or not.
     P->hiz_op = -1;
-    P->hiz_kind = 32;
     P->less_depth = 0;
     if (!P->fstates.empty()) {
         const std::vector<FragmentState>& fs = P->fstates;
@@ -267,7 +266,6 @@ int plan_launch(const cpv_config& cfg, const Program& prog, const std::vector<Ta
         for (const TargetParams& t : targets) ok = ok && t.has_ds && t.ds_fmt.depth_kind == fs[0].ds.depth_kind;
         if (ok) {
             if (!cfg.count_fragments) P->hiz_op = fs[0].depth_compare;
-            P->hiz_kind = fs[0].ds.depth_kind;
             P->less_depth = fs[0].depth_compare == CPV_COMPARE_LESS || fs[0].depth_compare == CPV_COMPARE_LESS_OR_EQUAL;
         }
     }
@@ -367,6 +365,20 @@ int resident_workgroups(Exec& x, const KernelRef& k, int block)
     return per_cu * std::max(x.ctx->cu_count, 1);
 }
 
+// RasterArgs::cull_mode of a launch.
+uint32_t cull_mode(const LaunchPlan& P)
+{
+    switch (P.hiz_op) {
+    case CPV_COMPARE_NEVER: return kCullAll;
+    case CPV_COMPARE_LESS:
+    case CPV_COMPARE_LESS_OR_EQUAL:
+    case CPV_COMPARE_EQUAL: return kCullOn;
+    case CPV_COMPARE_GREATER:
+    case CPV_COMPARE_GREATER_OR_EQUAL: return kCullOn | kCullGreater;
+    default: return 0u;   // no culling, or an op that fails against no interval
+    }
+}
+
 // Buffers whose size depends only on the plan.
 int ensure_front(Exec& x, const LaunchPlan& P)
 {
@@ -419,7 +431,8 @@ int enqueue_front(Exec& x, const LaunchPlan& P, uint8_t* arena, uint32_t pair_ca
     }
     if (P.prim_total > 0) {
         SetupArgs sa{d_dd, (const uint32_t*)(arena + P.o_sb), d_tp, b.vout.as<float>(), b.recs.as<TriSetup>(),
-                     P.lines ? b.line_ext.as<LineExt>() : nullptr, b.counts.as<uint32_t>(), b.sums.as<uint64_t>(), P.stride, P.tile_shift};
+                     P.lines ? b.line_ext.as<LineExt>() : nullptr, b.counts.as<uint32_t>(), b.sums.as<uint64_t>(), P.stride, P.tile_shift,
+                     cull_mode(P)};
         hipLaunchKernelGGL(setup_kernel, dim3((uint32_t)P.sblock.size()), dim3(256), 0, x.s, sa);
         HIP_TRY(hipGetLastError());
     }
@@ -585,7 +598,7 @@ int enqueue_raster(Exec& x, const LaunchPlan& P, uint8_t* arena, const Binned& b
     // tiles themselves no faster.)
     ra.persistent = sched == CPV_SCHED_COUNTER ? 1u : 0u;
     ra.hiz_op = P.hiz_op;
-    ra.hiz_depth_kind = P.hiz_kind;
+    ra.cull_mode = cull_mode(P);
     ra.less_depth = P.less_depth;
     ra.uniform_fstate = P.uniform_fstate;
     ra.count = x.cfg.count_fragments ? 1u : 0u;

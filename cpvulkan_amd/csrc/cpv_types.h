@@ -37,6 +37,11 @@ constexpr uint32_t kRasterQueueStride = 32;
 // long tiles one by one (LongTiles).
 constexpr int kSplitBlocks = 4;
 
+// How the raster kernel culls candidates by their depths: at all; all of them
+// (NEVER); against stored depths that rise (GREATER, GREATER_OR_EQUAL) rather
+// than fall.
+enum : uint32_t { kCullOn = 1u, kCullAll = 2u, kCullGreater = 0x80000000u };
+
 // What is known of a launch's tile lists when long ones are split.
 struct LongTiles {
     uint32_t count;    // tiles whose list has `from` pairs or more (RasterArgs::long_tiles)
@@ -83,7 +88,8 @@ struct TriSetup {
     float ax[3], ay[3];       // bytes 0-23
     float dy[3], dx[3];       // 24-47
     int32_t x0, y0, x1, y1;   // 48-63: pixel bounding box, [x0, x1) x [y0, y1)
-    float dt_lo, dt_hi;       // 64-71: bounds of the viewport-transformed depth of every covered pixel
+    float dt_lo, dt_hi;       // 64-71: bounds of the viewport-transformed depth of every covered pixel, or of its
+                              // negative (RasterArgs::cull_mode)
     float area;               // 72: |EdgeFunction(p0, p1, p2)|
     uint32_t draw_flags;      // 76: draw index within the launch (28 bits), the kPrim flags above it
     float z[3];               // 80-91: p_k.z / p_k.w

@@ -79,7 +79,7 @@ struct RasterArgs {
     uint32_t target_count;
     uint32_t persistent;            // 0: one workgroup per tile; 1: work queue
     int32_t hiz_op;                 // depth compare op shared by every draw when depth culling is exact, else -1
-    int32_t hiz_depth_kind;         // 16, 24 or 32
+    uint32_t cull_mode;             // how chunks are culled by depth (kCull flags)
     int32_t less_depth;             // 1: every draw has the depth test with LESS or LESS_OR_EQUAL (all the same
                                     // op) and no stencil or depth-bounds test, and all share one depth format
     int32_t uniform_fstate;         // the fragment state every draw of the launch has, -1 when they differ

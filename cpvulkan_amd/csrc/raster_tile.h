@@ -230,6 +230,15 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
     // the hierarchical depth op (-1: no hierarchical culling)
     const int32_t hiz_op = a.hiz_op;
     const bool less = a.less_depth != 0;
+    // Chunk culling compares the lower end of a candidate's depth interval with
+    // the largest stored depth.  Launches with GREATER or GREATER_OR_EQUAL hold
+    // the intervals of the negated depths in their records (setup_kernel), and
+    // the stored depths are compared negated: the op then fails in the same
+    // direction.  (Choosing the interval's end here made every frame 0.8%
+    // slower.)  For EQUAL the lower end alone is compared: the upper one's test
+    // in the walk raised the scalar spills from 67 to 92.
+    const uint32_t cull_mode = a.cull_mode;
+    auto toward = [&](float v) { return __uint_as_float(__float_as_uint(v) ^ (cull_mode & kCullGreater)); };
     uint32_t tried = 0;   // queues found empty, starting at home
     // Split tiles (splits_tile) are units of work, one per block of each of the
     // workgroup's waves, and start first.  Waves that hold two blocks gain
@@ -274,7 +283,7 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
         }
         const uint32_t tile = units ? item : __builtin_amdgcn_readfirstlane(a.order ? a.order[item] : item);
         const uint2 range = uniform_ptr(a.tile_range)[tile];
-        const uint32_t lbeg = range.x, lend = range.y;
+        const uint32_t lbeg = range.x, lend = (a.cull_mode & kCullAll) ? range.x : range.y;
         if (SPLIT && a.long_groups) {
             const bool split = lend > lbeg && splits_tile(*uniform_ptr(a.longs), lend - lbeg, WAVES);
             if (units && !split) continue;
@@ -404,7 +413,8 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
                 if (!SPLIT || (kmask >> k & 1u)) mine |= 1u << (kPairBlockShift + (blk / BW) / 2 * 2 + (blk % BW) / 2);
             }
         }
-        const bool packed = TILE != 8 && lend > lbeg && lend - lbeg > 64u;   // wave-uniform
+        const bool deep = lend > lbeg && lend - lbeg > 64u;   // wave-uniform
+        const bool packed = TILE != 8 && deep;   // every pair of an 8x8 tile names its block
         auto& ring = stage_area.ring[wave];
         constexpr uint32_t R = RasterStage<FS, TILE, WAVES>::kRing;
         uint32_t pos = packed ? lbeg & ~3u : lbeg, head = 0, tail = 0;
@@ -471,34 +481,18 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
             prefetch();
             // Hierarchical culling: a primitive whose depth interval fails
             // the test against every depth stored in the wave's pixels
-            // cannot change any of them.  With LESS and LESS_OR_EQUAL the
-            // interval's lower end decides: `lo_l` holds a candidate's, and
-            // the stored depths only fall, so it is tested again every few
-            // visits against their current maximum (a dozen vector
-            // instructions, a third of a visit).  Testing once per chunk left
-            // the soup 27 us slower once the chunks were full.
-            const bool culls = hiz_op >= 0 && less;
-            if (hiz_op >= 0 && !less) {
-                float bmin = __builtin_inff(), bmax = -__builtin_inff();
-#pragma unroll
-                for (int k = 0; k < BPW; k++) {
-                    if (!inside[k]) continue;
-                    bmin = fminf(bmin, cur_depth(k));
-                    bmax = fmaxf(bmax, cur_depth(k));
-                }
-                bmax = wave_max(bmax);
-                bmin = -wave_max(-bmin);
-                if (ov) {
-                    const float2 dz = *(const float2*)&a.recs[gp_l].dt_lo;
-                    ov = !hiz_rejects(hiz_op, dz.x, dz.y, bmin, bmax);
-                }
-            }
-            bool refined = !BLOCK_DEPTH || !packed;   // short lists: not worth the records' loads
+            // cannot change any of them.  `lo_l` holds the lower end of a
+            // candidate's interval, and the stored depths only fall (negated
+            // ones too), so it is tested again every few visits against their
+            // current maximum (a dozen vector instructions, a third of a
+            // visit).  Testing once per chunk left the soup 27 us
+            // slower once the chunks were full.
+            bool refined = !BLOCK_DEPTH || !deep;   // short lists: not worth the records' loads
             auto cull = [&](uint64_t m) {
                 float bmax = -__builtin_inff();
 #pragma unroll
                 for (int k = 0; k < BPW; k++)
-                    if (inside[k]) bmax = fmaxf(bmax, cur_depth(k));
+                    if (inside[k]) bmax = fmaxf(bmax, toward(cur_depth(k)));
                 bmax = wave_max(bmax);
                 m &= ~lanes(lo_l > bmax);
                 if (BLOCK_DEPTH && !refined && __popcll(m) >= kRefineCandidates) {
@@ -532,7 +526,7 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
                             float lo, hi;
                             if (block_depth_range(ax, ay, dy, dx, __uint_as_float(p4.z), __uint_as_float(p5.w), z, fminf(xa, xb),
                                                   fmaxf(xa, xb), fminf(ya, yb), fmaxf(ya, yb), lo, hi))
-                                lo_l = fmaxf(lo_l, lo);
+                                lo_l = fmaxf(lo_l, toward((cull_mode & kCullGreater) ? hi : lo));
                         }
                         m &= ~lanes(lo_l > bmax);
                     }
@@ -541,10 +535,10 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
             };
             uint64_t mask = lanes(ov);
             int since = kCullVisits;   // candidates visited since the last cull
-            const int step = packed ? kCullLanes : 64;
+            const int step = deep ? kCullLanes : 64;
             for (int first = 0; first < 64; first += step) {
               uint64_t window = mask & ((~0ull >> (64 - step)) << first);
-              if (culls && window && since >= kCullVisits) {
+              if ((cull_mode & kCullOn) && window && since >= kCullVisits) {
                   mask = cull(mask & (~0ull << first));
                   window &= mask;
                   since = 0;
@@ -607,6 +601,7 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
                     if (hiz_op >= 0) {
                         const float cd = cur_depth(k);
                         if (less) m &= ~lanes(r.dt_lo > cd);
+                        else if (cull_mode & kCullGreater) m &= ~lanes(r.dt_lo > -cd);
                         else m &= ~lanes(hiz_rejects(hiz_op, r.dt_lo, r.dt_hi, cd, cd));
                     }
                     if (!m) continue;

@@ -10,10 +10,11 @@ tighter than the triangle's depth range, so it drops many candidates),
 several draws of one launch under different viewports (offset and
 scaled, interleaved so the last visited draw keeps changing),
 depth ranges other than [0, 1] (the bound must stay off), and the compare
-ops that fold to a constant and those that do not.  Colour and depth must
-equal the oracle's bit for bit, with hierarchical culling on (fragment
-counting off), in every tile configuration with one pixel of a block per
-lane (16x16 tiles with four waves, 8x8 tiles) and one without."""
+ops: those whose stored depths fall, those whose depths rise (culled by the
+negated depths), EQUAL, and those that cull nothing or everything.  Colour and
+depth must equal the oracle's bit for bit, with hierarchical culling on
+(fragment counting off), in every tile configuration with one pixel of a block
+per lane (16x16 tiles with four waves, 8x8 tiles) and one without."""
 import copy
 import zlib
 
@@ -71,6 +72,29 @@ def test_block_depth_bound_matches_oracle(ctx, vps, op, tile, waves):
     if op == "GREATER":
         s.clear_depth = 0.0
     s.draws = _draws(zlib.crc32(label.encode()), VIEWPORT_SETS[vps])
+    cfg = ctx.config()
+    cfg.tile_size, cfg.waves_per_tile = tile, waves
+    ctx.apply_config(cfg)
+    ref = oracle_lib.render_scene(s)
+    compare(s, render_gpu(ctx, s, count=False), (ref[0], ref[1], None), label + " (culling on)")
+    compare(s, render_gpu(ctx, s), ref, label + " (counting)")
+
+
+@pytest.mark.parametrize("tile,waves", [(16, 4), (8, 1), (32, 4)])
+@pytest.mark.parametrize("ds", ["D32_SFLOAT", "D16_UNORM"])
+@pytest.mark.parametrize("op", ["NEVER", "EQUAL", "NOT_EQUAL", "GREATER", "GREATER_OR_EQUAL", "ALWAYS"])
+def test_every_other_op(ctx, op, ds, tile, waves):
+    """Lists of several chunks: steep depths, and depths of which many are equal to what is stored."""
+    label = f"block depth {op} {ds} {tile}x{waves}"
+    print(f"[block_depth] {label}", flush=True)
+    s = copy.deepcopy(W.soup_scene(10, WIDTH, HEIGHT, seed=1))
+    s.pipeline["depth_compare"] = abi.COMPARE[op]
+    s.ds_format = abi.FORMAT[ds]
+    s.clear_depth = 0.0 if op.startswith("GREATER") else 0.5
+    s.draws = _draws(zlib.crc32(label.encode()), VIEWPORT_SETS["three"], n=6000)
+    for d in s.draws[::2]:   # every other draw has one of three depths a triangle
+        v = d.vertices[0].view(np.float32).reshape(-1, 3, 8)
+        v[:, :, 2] = np.random.default_rng(3).choice([0.25, 0.5, 0.75], (v.shape[0], 1))
     cfg = ctx.config()
     cfg.tile_size, cfg.waves_per_tile = tile, waves
     ctx.apply_config(cfg)

@@ -27,6 +27,7 @@
 #include <thread>
 #include <cstring>
 #include <mutex>
+#include <unordered_map>
 #include <vector>
 
 #include "cpv_internal.h"
@@ -139,14 +140,33 @@ int plan_launch(const cpv_config& cfg, const Program& prog, const std::vector<Ta
     if (prog.fs_inputs > prog.vs_outputs) return fail(CPV_ERROR_INVALID, "fragment inputs exceed vertex outputs");
     P->dd.assign(lds.size(), DrawDesc{});
     P->envs.resize(lds.size());
-    P->fstates.resize(lds.size());
+    // the fragment states, each once: the raster kernel shades the fragments
+    // that share one together (shade_fragment), and a program's draws use few
+    std::unordered_multimap<uint64_t, uint32_t> state_of;
+    auto fragment_state = [&](const FragmentState& f) {
+        if (!P->fstates.empty() && std::memcmp(&P->fstates.back(), &f, sizeof(f)) == 0) return (uint32_t)P->fstates.size() - 1;
+        uint64_t h = 0xCBF29CE484222325ull;   // FNV-1a over the state's words
+        for (size_t i = 0; i + 4 <= sizeof(f); i += 4) {
+            uint32_t w;
+            std::memcpy(&w, (const uint8_t*)&f + i, 4);
+            h = (h ^ w) * 0x100000001B3ull;
+        }
+        const auto same = state_of.equal_range(h);
+        for (auto it = same.first; it != same.second; ++it)
+            if (std::memcmp(&P->fstates[it->second], &f, sizeof(f)) == 0) return it->second;
+        const uint32_t at = (uint32_t)P->fstates.size();
+        P->fstates.push_back(f);
+        state_of.emplace(h, at);
+        return at;
+    };
     uint32_t vout_total = 0, prim_total = 0;
     for (size_t i = 0; i < lds.size(); i++) {
         const cpv_pipeline_desc& p = *lds[i].pipe;
         const cpv_draw_desc& d = *lds[i].draw;
         int rc = build_env(p, d, &P->envs[i]);
         if (rc) return rc;
-        rc = build_fragment_state(p, passes[draw_target[i]], &P->fstates[i]);
+        FragmentState fs;
+        rc = build_fragment_state(p, passes[draw_target[i]], &fs);
         if (rc) return rc;
         if (p.topology > CPV_TOPOLOGY_TRIANGLE_FAN)
             return fail(CPV_ERROR_UNSUPPORTED, "topology %u (adjacency and patch lists)", p.topology);
@@ -167,7 +187,7 @@ int plan_launch(const cpv_config& cfg, const Program& prog, const std::vector<Ta
         DrawDesc& o = P->dd[i];
         std::memset(&o, 0, sizeof(o));
         o.target = draw_target[i];
-        o.fstate = (uint32_t)i;
+        o.fstate = fragment_state(fs);
         o.topology = p.topology;
         o.front_face = p.front_face;
         o.cull_mode = p.cull_mode;
@@ -270,9 +290,7 @@ int plan_launch(const cpv_config& cfg, const Program& prog, const std::vector<Ta
         }
     }
     plan_small(cfg, P);
-    P->uniform_fstate = P->fstates.empty() ? -1 : 0;
-    for (const FragmentState& f : P->fstates)
-        if (std::memcmp(&f, &P->fstates[0], sizeof(f)) != 0) P->uniform_fstate = -1;
+    P->uniform_fstate = P->fstates.size() == 1 ? 0 : -1;
     // the block tables are never empty
     if (P->vblock.empty()) P->vblock.push_back(0);
     if (P->sblock.empty()) P->sblock.push_back(0);
@@ -766,6 +784,10 @@ size_t cpvrt::scratch_bytes() { return kScratchBytes; }
 
 namespace {
 
+// What the draws' fragment states would take beyond the ones that are staged:
+// the allocation-free entry point's limits count one for each draw.
+size_t shared_state_bytes(const LaunchPlan& P) { return (P.dd.size() - P.fstates.size()) * sizeof(FragmentState); }
+
 // Places every buffer of launch P in the scratch array at base, with the
 // sizes ensure_front and ensure_back ask for: the control words first (at
 // the same address for every launch), then the descriptors, vertex outputs,
@@ -773,7 +795,8 @@ namespace {
 // entries each.  Touches no memory.
 //
 // What is refused, and the pair capacity, follow from the entry point's limit:
-// 64 MiB for the control words, descriptors, vertex outputs, records, four
+// 64 MiB for the control words, descriptors (a fragment state for every draw),
+// vertex outputs, records, four
 // words per primitive and line extension, a word per tile, 2 MiB of sort
 // tables, and the pairs (16 bytes each) in what is left.  The buffers placed
 // here never take more than that beside the ranges' second words.
@@ -784,7 +807,7 @@ int carve_scratch(uint8_t* base, const LaunchPlan& P, size_t arena_bytes, Buffer
     size_t limit = 0;
     auto count = [&](size_t bytes) { limit = ((limit + 255) & ~(size_t)255) + bytes; };
     count(kStatAlloc * 4);
-    count(arena);
+    count(arena + shared_state_bytes(P));
     count(vout);
     count(prims * sizeof(TriSetup));
     count(prims * 4);
@@ -1333,9 +1356,9 @@ extern "C" int cpv_render_pass_noalloc(cpv_context* c, const cpv_pass_desc* pass
         rc = plan_launch(cfg, S.prog, targets, S.lds, passes, S.dt, &L->P);
         if (rc) return rc;
         stage_plan(L->P, L->st);
-        if (L->st.bytes.size() > kStagingSlotBytes)
+        if (L->st.bytes.size() + shared_state_bytes(L->P) > kStagingSlotBytes)
             return fail(CPV_ERROR_UNSUPPORTED, "the pass's descriptors take %zu bytes; the allocation-free entry point stages at most %zu",
-                        L->st.bytes.size(), kStagingSlotBytes);
+                        L->st.bytes.size() + shared_state_bytes(L->P), kStagingSlotBytes);
         Buffers probe;
         uint32_t cap = 0;
         rc = carve_scratch(c->scratch, L->P, L->st.bytes.size(), &probe, &cap);

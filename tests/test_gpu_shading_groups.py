@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 import oracle_lib
+import scenes as S
 from gpu_util import compare, render_gpu
 from cpvulkan_amd import abi
 from cpvulkan_amd import workloads as W
@@ -51,3 +52,21 @@ def test_fragments_of_many_draws(gpu_ctx, op, ds, tile, waves):
         compare(s, render_gpu(gpu_ctx, s, count=False), (ref[0], ref[1], None), "culling on")
     finally:
         gpu_ctx.set_config()
+
+
+@pytest.mark.parametrize("blend", ["opaque", "both"])
+def test_small_draws_of_few_states(gpu_ctx, blend):
+    """Hundreds of draws of a few pixels under pipelines that differ in blend state, two of them equal: the fragments of one
+    shading pass are of many draws and few states.  Every other draw has a viewport of its own."""
+    s = S.soup(4, 96, 64, seed=2, size_px=np.log(6.0))
+    s.draws = [S.soup(4, 96, 64, seed=10 + k, size_px=np.log(6.0)).draws[0] for k in range(400)]
+    for k, d in enumerate(s.draws[::2]):
+        d.viewport = (float(k % 3), float(k % 5), 96.0 - k % 7, 64.0 - k % 4, 0.0, 1.0)
+    plain = dict(s.pipeline, blend=None)
+    s.pipelines = [plain, dict(plain), dict(plain, depth_write=0)] if blend == "opaque" else \
+        [plain, dict(plain), dict(plain, blend=W.ALPHA_BLEND), dict(plain, blend=W.ALPHA_BLEND, depth_write=0)]
+    s.draw_pipeline = [k % len(s.pipelines) for k in range(len(s.draws))]
+    ref = oracle_lib.render_scene(s)
+    print(f"[groups] {blend}", flush=True)
+    compare(s, render_gpu(gpu_ctx, s), ref, "counting")
+    compare(s, render_gpu(gpu_ctx, s, count=False), (ref[0], ref[1], None), "culling on")

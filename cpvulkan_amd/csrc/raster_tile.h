@@ -118,7 +118,16 @@ __device__ __forceinline__ uint64_t lanes(bool p)
 __device__ __forceinline__ bool in_lanes(uint64_t m)
 {
 #if defined(__HIP_DEVICE_COMPILE__)
+    // programs are also compiled at run time, by the hiprtc that the process
+    // has loaded: an older one (PyTorch's wheels bring ROCm 7.0's) does not
+    // know the builtin
+#if __has_builtin(__builtin_amdgcn_inverse_ballot_w64)
     return __builtin_amdgcn_inverse_ballot_w64(m);
+#else
+    uint32_t bit;
+    __asm__("v_cndmask_b32_e64 %0, 0, 1, %1" : "=v"(bit) : "s"(m));
+    return bit != 0u;
+#endif
 #else
     return m != 0;
 #endif

@@ -46,8 +46,18 @@ __global__ __launch_bounds__(256) void fill_rows_kernel(FillArgs a)
             if (p >= beg && p + 16 <= end) {
                 *global_ptr<uint4>(p) = v;
             } else {
-                for (uint32_t o = 0; o < 16u; o += a.size)
-                    if (p + o >= beg && p + o < end) store_pixel(global_ptr<uint8_t>(p + o), (int)a.size, a.pattern);
+                // words inside the row whole (pixels of 8 and 16 bytes are
+                // words inside it too), the rest by pixels of 1 and 2 bytes
+#pragma unroll
+                for (uint32_t w = 0; w < 4u; w++) {
+                    const uint64_t q = p + 4u * w;
+                    if (q >= beg && q + 4u <= end) {
+                        *global_ptr<uint32_t>(q) = a.pattern[w];
+                    } else if (q + 4u > beg && q < end) {
+                        for (uint32_t o = 0; o < 4u; o += a.size)
+                            if (q + o >= beg && q + o < end) store_pixel(global_ptr<uint8_t>(q + o), (int)a.size, a.pattern);
+                    }
+                }
             }
         }
     }
@@ -237,7 +247,8 @@ __global__ void blit_kernel(BlitArgs a)
 
 // A colour blit whose source and destination formats both hold four 8-bit
 // UNORM channels in 4 bytes (the common one: mip chains), the same arithmetic
-// with the formats and the wrapping folded; a wave takes 64 pixels of a row.
+// with the formats and the wrapping folded; a wave takes 64 pixels of a row
+// (or of several, when the region is narrower).
 // Bound by its vector instructions (two exact divisions, sixteen channels
 // unpacked and twelve lerps a pixel): 4096x4096 to 2048x2048 takes 26.4 us,
 // 3.2 TB/s (in blit_kernel, with a grid-strided pixel index, 40 us), and the
@@ -273,6 +284,15 @@ uint32_t grid_for(uint64_t n)
     return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((n + 255) / 256, 16384));
 }
 
+// Threads of a workgroup of 256 that lie along a row of n items: the power of
+// two that holds them, at most 64.
+uint32_t threads_across(uint64_t n)
+{
+    uint32_t t = 1;
+    while (t < 64u && t < n) t *= 2;
+    return t;
+}
+
 constexpr uint64_t kFillCached = (128u << 20) / 16;   // 16-byte chunks
 
 // Enqueues rows of a repeated pixel of `size` bytes (dividing 16 and every
@@ -289,7 +309,10 @@ int fill_rows(cpv_context* c, uint64_t dst, uint64_t row_bytes, uint64_t pitch, 
     a.chunks = rows == 1 ? ((dst & 15u) + row_bytes + 15) / 16 : (15 + row_bytes + 15) / 16;
     for (uint32_t o = 0; o < 16; o += size) std::memcpy((uint8_t*)a.pattern + o, pixel, size);
     void* args[] = {&a};
-    const dim3 block = rows == 1 ? dim3(256, 1) : dim3(64, 4);
+    // a row's chunks by one to 64 threads, so that narrow rows leave few idle
+    // (20 of 16,384 bytes: 16,384 rows in 20 us with 64)
+    const uint32_t across = rows == 1 ? 256u : threads_across(a.chunks);
+    const dim3 block(across, 256u / across);
     // One run of up to 128 MiB by 1,024 workgroups (64 MiB in 11.1 us, with a
     // chunk per thread 12.1), a longer one, past what the caches take, by a
     // chunk per thread (1 GiB in 154 us, by 1,024 workgroups 224).
@@ -452,9 +475,10 @@ extern "C" int cpv_blit_image(cpv_context* c, const cpv_image_level* src, const 
         a.aspect = r.aspect;
         void* args[] = {&a};
         if (plain) {
-            const dim3 block(64, 4);
-            const uint32_t gx = ((uint32_t)w + 63) / 64;
-            const uint32_t gy = std::min<uint32_t>(((uint32_t)h + 3) / 4, 65535);
+            const uint32_t across = threads_across((uint64_t)w);
+            const dim3 block(across, 256u / across);
+            const uint32_t gx = ((uint32_t)w + block.x - 1) / block.x;
+            const uint32_t gy = std::min<uint32_t>(((uint32_t)h + block.y - 1) / block.y, 65535);
             HIP_TRY(hipLaunchKernel(filter ? (const void*)blit_unorm8_kernel<1> : (const void*)blit_unorm8_kernel<0>, dim3(gx, gy), block,
                                     args, 0, c->stream));
             continue;

@@ -172,6 +172,29 @@ def test_fill_longer_than_the_grid(gpu_ctx, mem, mib):
     assert np.array_equal(mem.read(d, buf.nbytes), want)
 
 
+@pytest.mark.parametrize("width", [1, 2, 3, 5, 17, 33])
+def test_narrow_columns(gpu_ctx, mem, width):
+    """Blits and clears of columns, whose rows several share a wave: more rows than a workgroup takes, all ends of a chunk."""
+    print(f"[transfer] columns of {width}", flush=True)
+    code, W0, H = F["R8G8B8A8_UNORM"], 40, 700
+    src, dst = rand_bytes(W0 * H * 4), rand_bytes(W0 * H * 4)
+    s, d = mem.alloc(src), mem.alloc(dst)
+    for filter_ in (0, 1):
+        regions = [abi.BlitRegion((C.c_int32 * 4)(1, 0, 1 + width, H), (C.c_int32 * 4)(5, H, 5 + width, 1), 1, 0)]
+        oracle_lib.blit_image(src.copy(), code, W0, H, dst, code, W0, H, regions, filter_)
+        gpu_ctx.blit_image(abi.ImageLevel(s, code, W0, H, 0), abi.ImageLevel(d, code, W0, H, 0), regions, filter_)
+        assert np.array_equal(mem.read(d, dst.nbytes), dst), filter_
+    for fmt in ("R8_UNORM", "D16_UNORM", "R8G8B8A8_UNORM", "R16G16B16A16_UNORM", "R32G32B32A32_SFLOAT"):
+        code = F[fmt]
+        img = rand_bytes(61 * H * abi.FORMAT_BYTES[code])
+        d = mem.alloc(img)
+        value = f32words(0.7, 0.2, 0.9, 0.4) if fmt != "D16_UNORM" else f32words(0.7) + [0, 0, 0]
+        rects = [abi.Rect(3, 1, width, H - 2), abi.Rect(60 - width, 0, width, H)]
+        oracle_lib.clear_rects(img, code, 61, H, value, rects)
+        gpu_ctx.clear_rects(abi.ImageLevel(d, code, 61, H, 0), value, rects)
+        assert np.array_equal(mem.read(d, img.nbytes), img), fmt
+
+
 BLITS = [
     # (src rect, dst rect)
     ((0, 0, 37, 29), (0, 0, 37, 29)),        # same size

@@ -167,7 +167,9 @@ CPV_DEV void read_pixel(const uint8_t* p, int bytes, uint32_t w[4])
 // ImageSampler.cpp:676-681) and written with SetPixel; depth/stencil
 // formats read the texel at the truncated (u, v).
 // KIND is a.src_kind and FILTER a.filter, fixed per instantiation so each
-// carries only its own path.
+// carries only its own path; KIND 4 is a float source whose texels
+// sample_level_as<true> reads (with both in one kernel, 2048x2048 of R8 to half
+// the size took 24.1 us against 21.8).
 template <int KIND, int FILTER>
 __global__ void blit_kernel(BlitArgs a)
 {
@@ -210,9 +212,9 @@ __global__ void blit_kernel(BlitArgs a)
             pack_depth_stencil(a.dfmt, depth, stencil, d0, d1);
             px[0] = d0;
             px[1] = d1;
-        } else if (KIND == 0) {
+        } else if (KIND == 0 || KIND == 4) {
             float c[4];
-            sample_level(src, 0, u / (float)src.level_w[0], v / (float)src.level_h[0], FILTER, c);
+            sample_level_as<KIND == 4>(src, 0, u / (float)src.level_w[0], v / (float)src.level_h[0], FILTER, c);
             if (src.fmt.off[0] < 0) c[0] = 0.0f;
             if (src.fmt.off[1] < 0) c[1] = 0.0f;
             if (src.fmt.off[2] < 0) c[2] = 0.0f;
@@ -454,9 +456,9 @@ extern "C" int cpv_blit_image(cpv_context* c, const cpv_image_level* src, const 
         return f.base == kBaseUNorm && f.element == 1 && f.total == 4 && f.depth_off < 0 && f.stencil_off < 0 &&
                f.off[0] >= 0 && f.off[1] >= 0 && f.off[2] >= 0 && f.off[3] >= 0;
     };
-    // the texel offsets of sample_level_as<true> take 32 bits
-    const bool plain = a.src_kind == 0 && unorm8x4(sf) && unorm8x4(df) && src->width && src->height &&
-                       (uint64_t)src->width * src->height <= (1ull << 30) && dst->address % 4 == 0 && src->address % 4 == 0;
+    // sources that sample_level_as<true> reads, and of those to the same kind of format
+    const bool plain_src = a.src_kind == 0 && unorm8x4(sf) && plain_extent(src->width, src->height) && src->address % 4 == 0;
+    const bool plain = plain_src && unorm8x4(df) && dst->address % 4 == 0;
     for (uint32_t i = 0; i < count; i++) {
         const cpv_blit_region& r = regions[i];
         const int32_t w = std::abs(r.dst[2] - r.dst[0]), h = std::abs(r.dst[3] - r.dst[1]);
@@ -486,6 +488,7 @@ extern "C" int cpv_blit_image(cpv_context* c, const cpv_image_level* src, const 
         const void* fn = a.src_kind == 3 ? (const void*)blit_kernel<3, 0>
                          : a.src_kind == 2 ? (const void*)blit_kernel<2, 0>
                          : a.src_kind == 1 ? (const void*)blit_kernel<1, 0>
+                         : plain_src ? (filter ? (const void*)blit_kernel<4, 1> : (const void*)blit_kernel<4, 0>)
                          : filter ? (const void*)blit_kernel<0, 1> : (const void*)blit_kernel<0, 0>;
         HIP_TRY(hipLaunchKernel(fn, dim3(grid_for((uint64_t)w * h)), dim3(256), args, 0, c->stream));
     }

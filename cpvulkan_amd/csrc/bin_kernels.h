@@ -29,7 +29,19 @@ struct SetupArgs {
     uint32_t stride;
     int32_t tile_shift;
     uint32_t cull_mode;           // RasterArgs::cull_mode
+    uint32_t prims;
 };
+
+// The draw of primitive gp, which is one of draws [first, last]: the last of
+// them that begins at or before it.
+__device__ __forceinline__ uint32_t draw_of(const DrawDesc* draws, uint32_t first, uint32_t last, uint32_t gp)
+{
+    while (first < last) {
+        const uint32_t mid = (first + last + 1u) >> 1;
+        if (draws[mid].prim_base <= gp) first = mid; else last = mid - 1u;
+    }
+    return first;
+}
 
 // EdgeFunction(a, b, c) with c the pixel centre, stored as a, (b.y - a.y), (b.x - a.x).
 __device__ __forceinline__ void put_edge(TriSetup& r, int k, const float* a, const float* b)
@@ -371,21 +383,35 @@ __device__ uint32_t setup_triangle(const SetupArgs& a, const DrawDesc& d, uint32
     return tiles_of(x0, y0, x1, y1, a.tile_shift);
 }
 
-// One thread per primitive.  A workgroup also adds up its primitives' tile
-// counts, so the pair offsets need one scan of a sum per 256 primitives
-// (scan_blocks_kernel) and no pass over the counts.
+__device__ __forceinline__ uint32_t setup_primitive(const SetupArgs& a, const DrawDesc& d, uint32_t di, uint32_t gp)
+{
+    const uint32_t p = gp - d.prim_base;
+    if (d.topology == 0) return setup_point(a, d, di, p, gp);
+    if (d.topology <= 2) return setup_line(a, d, di, p, gp);
+    return setup_triangle(a, d, di, p, gp);
+}
+
+// One thread per primitive, 256 consecutive ones per workgroup.  Most
+// workgroups' primitives are of one draw, whose descriptor then comes by
+// scalar loads; where small draws share one, each thread finds its own.  (A
+// workgroup per 256 primitives of each draw cost a launch of 60,000 draws of
+// two triangles 138 us here, 130 in the emit kernel and 67 in the scan.)
+// A workgroup also adds up its primitives' tile counts, so the pair offsets
+// need one scan of a sum per 256 primitives (scan_blocks_kernel) and no pass
+// over the counts.
 __global__ __launch_bounds__(256) void setup_kernel(SetupArgs a)
 {
     __shared__ uint32_t s_lo[4];
-    const uint32_t di = a.block_draw[blockIdx.x];
-    const DrawDesc& d = *uniform_ptr(&a.draws[di]);
-    const uint32_t p = (blockIdx.x - d.sblock_base) * 256u + threadIdx.x;
+    const uint32_t first = a.block_draw[blockIdx.x], last = a.block_draw[blockIdx.x + 1];
+    const uint32_t gp = blockIdx.x * 256u + threadIdx.x;
     uint32_t c = 0;
-    if (p < d.prim_count) {
-        const uint32_t gp = d.prim_base + p;
-        if (d.topology == 0) c = setup_point(a, d, di, p, gp);
-        else if (d.topology <= 2) c = setup_line(a, d, di, p, gp);
-        else c = setup_triangle(a, d, di, p, gp);
+    if (gp < a.prims) {
+        if (first == last) {
+            c = setup_primitive(a, *uniform_ptr(&a.draws[first]), first, gp);
+        } else {
+            const uint32_t di = draw_of(a.draws, first, last, gp);
+            c = setup_primitive(a, a.draws[di], di, gp);
+        }
         a.counts[gp] = c;
         // a dropped primitive's record keeps an empty pixel box, which
         // bin_small_kernel reads
@@ -510,9 +536,10 @@ struct EmitArgs {
     const LineExt* ext;           // per-primitive line extension (launches with lines)
     const uint32_t* counts;
     const uint64_t* sums;         // output offset of each setup workgroup's first pair
-    const uint32_t* block_draw;   // setup-grid block -> draw
+    const uint32_t* block_draw;   // as setup_kernel's
     const DrawDesc* draws;
     const TargetParams* targets;
+    uint32_t prims;
     uint32_t* keys;               // global tile index per pair
     uint32_t* vals;               // primitive index per pair
     uint32_t* big;                // primitives left to emit_big_kernel: big[0] of them, (primitive, offset) from big[1]
@@ -661,14 +688,14 @@ __device__ __forceinline__ uint32_t pair_blocks_covered(int tile_shift, int4 box
 
 // Writes the (tile, primitive) pairs of every primitive at its offset, so the
 // pair array is in primitive order.  A workgroup takes the 256 consecutive
-// primitives of one draw that the setup workgroup of its index took, whose
-// pairs are one contiguous run of the output (less the runs of primitives
+// primitives that the setup workgroup of its index took, whose pairs are one contiguous run of the output (less the runs of primitives
 // with more than kEmitBig pairs, queued for emit_big_kernel): its threads
 // stride over the run, so consecutive lanes write consecutive pairs, and each
 // finds its primitive by binary search of the workgroup's scanned counts in
 // LDS.  What a pair needs of its primitive (tile rectangle, edges) is staged
 // in LDS by the primitive's thread, so the pair loop reads no record; what it
-// needs of the draw and target is the workgroup's, in scalar registers.
+// needs of the draw and target is the workgroup's, in scalar registers, or
+// where several draws share one the pair's own.
 // Tiles of a primitive go in row-major order of its tile rectangle.
 __global__ __launch_bounds__(256) void emit_kernel(EmitArgs a)
 {
@@ -681,13 +708,14 @@ __global__ __launch_bounds__(256) void emit_kernel(EmitArgs a)
     __shared__ int4 s_box[256];       // pixel box of each primitive, relative to its first tile
     __shared__ int2 s_org[256];       // pixel origin of each primitive's first tile
     __shared__ float4 s_edge[256][3]; // each primitive's edges (record bytes 0-47)
-    const DrawDesc& dd = *uniform_ptr(&a.draws[a.block_draw[blockIdx.x]]);
+    const uint32_t first = a.block_draw[blockIdx.x];
+    const bool one = first == a.block_draw[blockIdx.x + 1];   // one draw's primitives
+    const DrawDesc& dd = *uniform_ptr(&a.draws[first]);
     const TargetParams& t = *uniform_ptr(&a.targets[dd.target]);
-    const uint32_t p = (blockIdx.x - dd.sblock_base) * 256u + threadIdx.x;
-    const uint32_t gp0 = dd.prim_base + (blockIdx.x - dd.sblock_base) * 256u, gp = gp0 + threadIdx.x;
+    const uint32_t gp0 = blockIdx.x * 256u, gp = gp0 + threadIdx.x;
     const uint32_t tiles_x = t.tiles_x;
     const float4 vp = make_float4(dd.vp_w, dd.vp_h, dd.half_x, dd.half_y);
-    uint32_t c = p < dd.prim_count ? a.counts[gp] : 0u;
+    uint32_t c = gp < a.prims ? a.counts[gp] : 0u;
     uint32_t all;
     const uint32_t dst = (uint32_t)uniform_ptr(a.sums)[blockIdx.x] + block_exclusive_scan(c, s_tmp, all);
     if (all == 0) return;
@@ -705,7 +733,12 @@ __global__ __launch_bounds__(256) void emit_kernel(EmitArgs a)
         const uint32_t tx0 = (uint32_t)r.x0 >> sh, tx1 = (uint32_t)(r.x1 - 1) >> sh;
         const uint32_t ty0 = (uint32_t)r.y0 >> sh;
         s_dst[threadIdx.x] = dst;
-        s_key[threadIdx.x] = t.tile_base + ty0 * tiles_x + tx0;
+        if (one) {
+            s_key[threadIdx.x] = t.tile_base + ty0 * tiles_x + tx0;
+        } else {
+            const TargetParams& own = a.targets[a.draws[r.draw_flags & kPrimDraw].target];
+            s_key[threadIdx.x] = own.tile_base + ty0 * own.tiles_x + tx0;
+        }
         s_w[threadIdx.x] = (tx1 - tx0 + 1) | (((r.draw_flags >> kPrimFlagShift) & (kPrimPoint | kPrimLine)) << kKindShift);
         const int ox = (int)(tx0 << sh), oy = (int)(ty0 << sh);
         s_box[threadIdx.x] = make_int4(r.x0 - ox, r.y0 - oy, r.x1 - ox, r.y1 - oy);
@@ -735,12 +768,19 @@ __global__ __launch_bounds__(256) void emit_kernel(EmitArgs a)
         const uint32_t out = s_dst[lo] + k;
         if (out < a.cap) {
             const uint32_t col = k - row * w;
-            a.keys[out] = s_key[lo] + row * tiles_x + col;
+            uint32_t across = tiles_x;
+            float4 view = vp;
+            if (!one) {
+                const DrawDesc& own = a.draws[a.recs[gp0 + lo].draw_flags & kPrimDraw];
+                across = a.targets[own.target].tiles_x;
+                view = make_float4(own.vp_w, own.vp_h, own.half_x, own.half_y);
+            }
+            a.keys[out] = s_key[lo] + row * across + col;
             const int2 org = s_org[lo];
             const float4 e[3] = {s_edge[lo][0], s_edge[lo][1], s_edge[lo][2]};
             float4 l = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             if (kind & kPrimLine) l = *(const float4*)&a.ext[gp0 + lo];
-            a.vals[out] = (gp0 + lo) | pair_blocks_covered(a.tile_shift, s_box[lo], col, row, kind, e, l, vp, org.x, org.y);
+            a.vals[out] = (gp0 + lo) | pair_blocks_covered(a.tile_shift, s_box[lo], col, row, kind, e, l, view, org.x, org.y);
         }
     }
 }

@@ -66,7 +66,9 @@ struct LaunchPlan {
     std::vector<DrawEnv> envs;
     std::vector<FragmentState> fstates;
     std::vector<TargetParams> targets;
-    std::vector<uint32_t> vblock, sblock;
+    std::vector<uint32_t> vblock;    // vertex grid: the draw of each block
+    std::vector<uint32_t> sblock;    // setup grid: the draw of each block's first primitive, and the last draw
+    uint64_t own_blocks = 0;         // setup blocks if every draw had its own
     uint32_t vout_total = 0, prim_total = 0, tiles = 0, stride = 0;
     int tile_shift = 4;
     int raster_variant = 3;          // index into Program::raster
@@ -236,9 +238,10 @@ int plan_launch(const cpv_config& cfg, const Program& prog, const std::vector<Ta
         o.prim_base = prim_total;
         o.prim_count = prim_count_of(p.topology, d.count);
         o.vblock_base = (uint32_t)P->vblock.size();
-        o.sblock_base = (uint32_t)P->sblock.size();
         for (uint32_t b = 0; b < (nverts + 255) / 256; b++) P->vblock.push_back((uint32_t)i);
-        for (uint32_t b = 0; b < (o.prim_count + 255) / 256; b++) P->sblock.push_back((uint32_t)i);
+        // the setup grid's blocks of 256 primitives that begin in this draw
+        while ((uint64_t)P->sblock.size() * 256 < (uint64_t)prim_total + o.prim_count) P->sblock.push_back((uint32_t)i);
+        P->own_blocks += (o.prim_count + 255) / 256;
         vout_total += nverts;
         prim_total += o.prim_count;
     }
@@ -291,9 +294,13 @@ int plan_launch(const cpv_config& cfg, const Program& prog, const std::vector<Ta
     }
     plan_small(cfg, P);
     P->uniform_fstate = P->fstates.size() == 1 ? 0 : -1;
-    // the block tables are never empty
+    // the block tables are never empty; a block's draws end at its successor's
     if (P->vblock.empty()) P->vblock.push_back(0);
     if (P->sblock.empty()) P->sblock.push_back(0);
+    uint32_t last = 0;
+    for (size_t i = 0; i < P->dd.size(); i++)
+        if (P->dd[i].prim_count) last = (uint32_t)i;
+    P->sblock.push_back(last);
     return CPV_OK;
 }
 
@@ -383,6 +390,9 @@ int resident_workgroups(Exec& x, const KernelRef& k, int block)
     return per_cu * std::max(x.ctx->cu_count, 1);
 }
 
+// Workgroups of the setup and emit kernels.
+uint32_t setup_blocks(const LaunchPlan& P) { return (uint32_t)P.sblock.size() - 1u; }
+
 // RasterArgs::cull_mode of a launch.
 uint32_t cull_mode(const LaunchPlan& P)
 {
@@ -405,7 +415,7 @@ int ensure_front(Exec& x, const LaunchPlan& P)
     if (b.vout.ensure((size_t)std::max(P.vout_total, 1u) * P.stride * 4, f) ||
         b.recs.ensure((size_t)std::max(P.prim_total, 1u) * sizeof(TriSetup), f) ||
         b.counts.ensure((size_t)std::max(P.prim_total, 1u) * 4, f) || b.stats.ensure(kStatAlloc * 4, f) ||
-        b.sums.ensure(P.sblock.size() * 8, f) || b.big.ensure(((size_t)P.prim_total * 2 + 1) * 4, f))
+        b.sums.ensure(setup_blocks(P) * 8, f) || b.big.ensure(((size_t)P.prim_total * 2 + 1) * 4, f))
         return CPV_ERROR_OUT_OF_MEMORY;
     if (P.lines && b.line_ext.ensure((size_t)std::max(P.prim_total, 1u) * sizeof(LineExt), f)) return CPV_ERROR_OUT_OF_MEMORY;
     return CPV_OK;
@@ -450,12 +460,12 @@ int enqueue_front(Exec& x, const LaunchPlan& P, uint8_t* arena, uint32_t pair_ca
     if (P.prim_total > 0) {
         SetupArgs sa{d_dd, (const uint32_t*)(arena + P.o_sb), d_tp, b.vout.as<float>(), b.recs.as<TriSetup>(),
                      P.lines ? b.line_ext.as<LineExt>() : nullptr, b.counts.as<uint32_t>(), b.sums.as<uint64_t>(), P.stride, P.tile_shift,
-                     cull_mode(P)};
-        hipLaunchKernelGGL(setup_kernel, dim3((uint32_t)P.sblock.size()), dim3(256), 0, x.s, sa);
+                     cull_mode(P), P.prim_total};
+        hipLaunchKernelGGL(setup_kernel, dim3(setup_blocks(P)), dim3(256), 0, x.s, sa);
         HIP_TRY(hipGetLastError());
     }
     if (P.small) return CPV_OK;
-    ScanArgs ca{b.sums.as<uint64_t>(), P.prim_total ? (uint32_t)P.sblock.size() : 0u, std::max(pair_cap, 1u),
+    ScanArgs ca{b.sums.as<uint64_t>(), P.prim_total ? setup_blocks(P) : 0u, std::max(pair_cap, 1u),
                 (uint64_t*)(stats + kStatPairTotal), stats + kStatPairs, x.overflow ? x.overflow : stats + kStatOverflow,
                 x.overflow ? 1u : 0u, b.big.as<uint32_t>(), x.host_total, (LongTiles*)(stats + kStatLong)};
     hipLaunchKernelGGL(scan_blocks_kernel, dim3(1), dim3(kScanThreads), 0, x.s, ca);
@@ -517,9 +527,9 @@ int enqueue_bin(Exec& x, const LaunchPlan& P, uint8_t* arena, uint32_t pair_cap,
     // emit pairs in primitive order
     if (P.prim_total) {
         EmitArgs ea{b.recs.as<TriSetup>(), P.lines ? b.line_ext.as<LineExt>() : nullptr, b.counts.as<uint32_t>(), b.sums.as<uint64_t>(),
-                    (const uint32_t*)(arena + P.o_sb), d_dd, d_tp, b.keys[0].as<uint32_t>(), b.vals[0].as<uint32_t>(),
+                    (const uint32_t*)(arena + P.o_sb), d_dd, d_tp, P.prim_total, b.keys[0].as<uint32_t>(), b.vals[0].as<uint32_t>(),
                     b.big.as<uint32_t>(), P.tile_shift, cap};
-        hipLaunchKernelGGL(emit_kernel, dim3((uint32_t)P.sblock.size()), dim3(256), 0, x.s, ea);
+        hipLaunchKernelGGL(emit_kernel, dim3(setup_blocks(P)), dim3(256), 0, x.s, ea);
         hipLaunchKernelGGL(emit_big_kernel, dim3(1024), dim3(256), 0, x.s, ea);
         HIP_TRY(hipGetLastError());
     }
@@ -784,9 +794,14 @@ size_t cpvrt::scratch_bytes() { return kScratchBytes; }
 
 namespace {
 
-// What the draws' fragment states would take beyond the ones that are staged:
-// the allocation-free entry point's limits count one for each draw.
-size_t shared_state_bytes(const LaunchPlan& P) { return (P.dd.size() - P.fstates.size()) * sizeof(FragmentState); }
+// What the descriptors would take beyond the ones that are staged if every
+// draw had a fragment state and setup blocks of its own: the allocation-free
+// entry point's limits count them so.
+size_t shared_state_bytes(const LaunchPlan& P)
+{
+    const uint64_t blocks = std::max<uint64_t>(P.own_blocks, setup_blocks(P)) - setup_blocks(P);
+    return (P.dd.size() - P.fstates.size()) * sizeof(FragmentState) + (size_t)blocks * 4;
+}
 
 // Places every buffer of launch P in the scratch array at base, with the
 // sizes ensure_front and ensure_back ask for: the control words first (at
@@ -838,7 +853,7 @@ int carve_scratch(uint8_t* base, const LaunchPlan& P, size_t arena_bytes, Buffer
     take(b->vout, vout);
     take(b->recs, prims * sizeof(TriSetup));
     take(b->counts, prims * 4);
-    take(b->sums, P.sblock.size() * 8);
+    take(b->sums, (size_t)setup_blocks(P) * 8);
     take(b->big, ((size_t)P.prim_total * 2 + 1) * 4);
     if (P.lines) take(b->line_ext, prims * sizeof(LineExt));
     take(b->tile_range, tiles * 8);

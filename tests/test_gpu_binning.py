@@ -159,3 +159,37 @@ def test_some_tiles_split(ctx, tile, waves, side):
     d.count = v.shape[0]
     s.draws.append(d)
     _check(ctx, s, f"{side}x{side} {tile}x{waves}", tile, waves)
+
+
+@pytest.mark.parametrize("sizes", [(255, 1, 256, 257), (0, 3, 0, 600, 0), (2,) * 2600, (1, 0, 5000, 0, 0, 1, 300, 2)])
+@pytest.mark.parametrize("tile,waves", [(16, 4), (8, 1)])
+def test_draws_that_share_setup_workgroups(ctx, sizes, tile, waves):
+    """Workgroups of 256 primitives over draws that begin anywhere in them, empty ones and several viewports among them; small
+    launches and, by a fourth of the draws again, ones that bin pairs."""
+    s = S.soup(4, 150, 101, seed=1)
+    full = S.soup(max(sum(sizes), 1), 150, 101, seed=5, size_px=np.log(6.0)).draws[0].vertices[0].view(np.float32).reshape(-1, 3, 8)
+    s.draws, at = [], 0
+    for k, n in enumerate(sizes):
+        d = copy.deepcopy(S.soup(1, 150, 101, seed=1).draws[0])
+        d.vertices = {0: np.ascontiguousarray(full[at:at + max(n, 1)]).view(np.uint8).reshape(-1)}
+        d.count, at = 3 * n, min(at + n, full.shape[0] - 1)
+        if k % 3 == 1:
+            d.viewport = (3.0, 2.0, 120.0, 90.0, 0.0, 1.0)
+        s.draws.append(d)
+    _check(ctx, s, f"{len(sizes)} draws {tile}x{waves}", tile, waves)
+
+
+def test_targets_that_share_setup_workgroups(ctx):
+    """Jobs of a few triangles to targets of different widths: a workgroup's primitives are of many targets."""
+    scenes = [W.soup_scene(1 + k % 7, 40 + 16 * (k % 5), 30 + 8 * (k % 3), seed=100 + k) for k in range(300)]
+    scenes.append(W.soup_scene(5000, 320, 200, seed=99))   # beyond what the small launches' lists take
+    refs = oracle_jobs(scenes)
+    mem, ms, jobs = materialize_jobs(ctx, scenes)
+    try:
+        print("[binning] 301 jobs", flush=True)
+        ctx.render_jobs(jobs)
+        ctx.synchronize()
+        assert ctx.fragment_count() == sum(r[2] for r in refs)
+        compare_jobs(scenes, ms, refs, "jobs")
+    finally:
+        mem.release()

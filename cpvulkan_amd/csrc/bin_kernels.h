@@ -697,6 +697,11 @@ __device__ __forceinline__ uint32_t pair_blocks_covered(int tile_shift, int4 box
 // needs of the draw and target is the workgroup's, in scalar registers, or
 // where several draws share one the pair's own.
 // Tiles of a primitive go in row-major order of its tile rectangle.
+template <bool V>
+struct Uniform {
+    static constexpr bool value = V;
+};
+
 __global__ __launch_bounds__(256) void emit_kernel(EmitArgs a)
 {
     constexpr int kKindShift = 29;    // s_w: the primitive's kind (kPrimPoint, kPrimLine) above the columns
@@ -751,38 +756,46 @@ __global__ __launch_bounds__(256) void emit_kernel(EmitArgs a)
     s_off[threadIdx.x] = block_exclusive_scan(c, s_tmp, total);
     if (threadIdx.x == 0) s_off[256] = total;
     __syncthreads();
-    for (uint32_t j = threadIdx.x; j < total; j += 256u) {
-        // lo: the last primitive whose run starts at or before j (s_off is
-        // non-decreasing and s_off[0] = 0), in eight unrolled halvings
-        uint32_t lo = 0;
+    // a loop for each, so that one draw's holds nothing of the other (the 1M
+    // soup's pairs, beside its raster kernel, took 117 us with the branch
+    // inside and take 115)
+    auto pairs = [&](auto own) {
+        using Own = decltype(own);
+        for (uint32_t j = threadIdx.x; j < total; j += 256u) {
+            // lo: the last primitive whose run starts at or before j (s_off is
+            // non-decreasing and s_off[0] = 0), in eight unrolled halvings
+            uint32_t lo = 0;
 #pragma unroll
-        for (uint32_t step = 128; step >= 1; step >>= 1)
-            if (s_off[lo + step] <= j) lo += step;
-        const uint32_t k = j - s_off[lo];
-        const uint32_t wl = s_w[lo];
-        const uint32_t w = wl & ((1u << kKindShift) - 1u), kind = wl >> kKindShift;
-        // row = k / w: k < kEmitBig = 2048 and w <= 2048, so (k + 1/2) / w
-        // is at least 1/(2w) from an integer while the product with
-        // v_rcp_f32's reciprocal (1 ulp) errs by under 1.5 * 2^-23 * 2049 / w
-        const uint32_t row = (uint32_t)(((float)k + 0.5f) * __builtin_amdgcn_rcpf((float)w));
-        const uint32_t out = s_dst[lo] + k;
-        if (out < a.cap) {
-            const uint32_t col = k - row * w;
-            uint32_t across = tiles_x;
-            float4 view = vp;
-            if (!one) {
-                const DrawDesc& own = a.draws[a.recs[gp0 + lo].draw_flags & kPrimDraw];
-                across = a.targets[own.target].tiles_x;
-                view = make_float4(own.vp_w, own.vp_h, own.half_x, own.half_y);
+            for (uint32_t step = 128; step >= 1; step >>= 1)
+                if (s_off[lo + step] <= j) lo += step;
+            const uint32_t k = j - s_off[lo];
+            const uint32_t wl = s_w[lo];
+            const uint32_t w = wl & ((1u << kKindShift) - 1u), kind = wl >> kKindShift;
+            // row = k / w: k < kEmitBig = 2048 and w <= 2048, so (k + 1/2) / w
+            // is at least 1/(2w) from an integer while the product with
+            // v_rcp_f32's reciprocal (1 ulp) errs by under 1.5 * 2^-23 * 2049 / w
+            const uint32_t row = (uint32_t)(((float)k + 0.5f) * __builtin_amdgcn_rcpf((float)w));
+            const uint32_t out = s_dst[lo] + k;
+            if (out < a.cap) {
+                const uint32_t col = k - row * w;
+                uint32_t across = tiles_x;
+                float4 view = vp;
+                if (!Own::value) {
+                    const DrawDesc& own = a.draws[a.recs[gp0 + lo].draw_flags & kPrimDraw];
+                    across = a.targets[own.target].tiles_x;
+                    view = make_float4(own.vp_w, own.vp_h, own.half_x, own.half_y);
+                }
+                a.keys[out] = s_key[lo] + row * across + col;
+                const int2 org = s_org[lo];
+                const float4 e[3] = {s_edge[lo][0], s_edge[lo][1], s_edge[lo][2]};
+                float4 l = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                if (kind & kPrimLine) l = *(const float4*)&a.ext[gp0 + lo];
+                a.vals[out] = (gp0 + lo) | pair_blocks_covered(a.tile_shift, s_box[lo], col, row, kind, e, l, view, org.x, org.y);
             }
-            a.keys[out] = s_key[lo] + row * across + col;
-            const int2 org = s_org[lo];
-            const float4 e[3] = {s_edge[lo][0], s_edge[lo][1], s_edge[lo][2]};
-            float4 l = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            if (kind & kPrimLine) l = *(const float4*)&a.ext[gp0 + lo];
-            a.vals[out] = (gp0 + lo) | pair_blocks_covered(a.tile_shift, s_box[lo], col, row, kind, e, l, view, org.x, org.y);
         }
-    }
+    };
+    if (one) pairs(Uniform<true>{});
+    else pairs(Uniform<false>{});
 }
 
 // Pairs of the large primitives: one workgroup per primitive at a time,

@@ -548,6 +548,11 @@ int build_texture(const cpv_texture_desc& t, TextureDesc* o)
     o->sampler.min_lod = s.min_lod;
     o->sampler.max_lod = s.max_lod;
     o->sampler.border_color = (int32_t)s.border_color;
+    const FormatDesc& f = o->fmt;
+    if (f.base == kBaseUNorm && f.element == 1 && f.total == 4 && (f.off[0] | f.off[1] | f.off[2] | f.off[3]) >= 0 && s.address_u != 3 &&
+        s.address_v != 3)
+        for (uint32_t j = 0; j < t.level_count; j++)
+            if (plain_extent(o->level_w[j], o->level_h[j])) o->plain |= 1u << j;
     return CPV_OK;
 }
 

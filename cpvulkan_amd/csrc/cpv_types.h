@@ -231,7 +231,7 @@ struct DrawDesc {
     uint32_t fstate;           // FragmentState index
     uint32_t vout_base, vout_count;
     uint32_t prim_base, prim_count;
-    uint32_t vblock_base, sblock_base;   // first block of this draw in the vertex / setup grids
+    uint32_t vblock_base;          // first block of this draw in the vertex grid
     uint32_t topology, front_face, cull_mode;
     uint32_t vmode;            // vertex slot mode, see VertexSlotMode
     uint32_t first;            // firstVertex or firstIndex

@@ -379,6 +379,10 @@ __device__ uint32_t setup_triangle(const SetupArgs& a, const DrawDesc& d, uint32
         r.dt_lo = -r.dt_hi;
         r.dt_hi = -lo;
     }
+    if (a.cull_mode & kCullAll) {   // beyond every stored depth
+        r.dt_lo = __builtin_inff();
+        r.dt_hi = -__builtin_inff();
+    }
     store_record(&a.recs[gp], r);
     return tiles_of(x0, y0, x1, y1, a.tile_shift);
 }

@@ -397,7 +397,7 @@ uint32_t setup_blocks(const LaunchPlan& P) { return (uint32_t)P.sblock.size() - 
 uint32_t cull_mode(const LaunchPlan& P)
 {
     switch (P.hiz_op) {
-    case CPV_COMPARE_NEVER: return kCullAll;
+    case CPV_COMPARE_NEVER: return kCullOn | kCullAll;
     case CPV_COMPARE_LESS:
     case CPV_COMPARE_LESS_OR_EQUAL:
     case CPV_COMPARE_EQUAL: return kCullOn;

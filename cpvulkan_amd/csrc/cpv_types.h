@@ -37,9 +37,10 @@ constexpr uint32_t kRasterQueueStride = 32;
 // long tiles one by one (LongTiles).
 constexpr int kSplitBlocks = 4;
 
-// How the raster kernel culls candidates by their depths: at all; all of them
-// (NEVER); against stored depths that rise (GREATER, GREATER_OR_EQUAL) rather
-// than fall.
+// How candidates are culled by their depths: at all; against stored depths
+// that rise (GREATER, GREATER_OR_EQUAL) rather than fall; all of them (NEVER).
+// The raster kernel knows the first two, and setup writes the intervals that
+// the others need.
 enum : uint32_t { kCullOn = 1u, kCullAll = 2u, kCullGreater = 0x80000000u };
 
 // What is known of a launch's tile lists when long ones are split.

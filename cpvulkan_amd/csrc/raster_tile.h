@@ -292,7 +292,7 @@ __device__ __forceinline__ void raster_body(const RasterArgs& a, RasterStage<FS,
         }
         const uint32_t tile = units ? item : __builtin_amdgcn_readfirstlane(a.order ? a.order[item] : item);
         const uint2 range = uniform_ptr(a.tile_range)[tile];
-        const uint32_t lbeg = range.x, lend = (a.cull_mode & kCullAll) ? range.x : range.y;
+        const uint32_t lbeg = range.x, lend = range.y;
         if (SPLIT && a.long_groups) {
             const bool split = lend > lbeg && splits_tile(*uniform_ptr(a.longs), lend - lbeg, WAVES);
             if (units && !split) continue;

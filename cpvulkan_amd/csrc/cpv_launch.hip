@@ -544,7 +544,7 @@ int enqueue_bin(Exec& x, const LaunchPlan& P, uint8_t* arena, uint32_t pair_cap,
     // of the sorted keys, which nothing reads any more (a long tile has
     // many pairs, so the list always fits)
     if (splits_long_tiles(x, P)) {
-        hipLaunchKernelGGL(long_tiles_kernel, dim3((P.tiles + 255) / 256), dim3(256), 0, x.s, ranges, P.tiles,
+        hipLaunchKernelGGL(long_tiles_kernel, dim3(std::min<uint32_t>((P.tiles + 255) / 256, 256)), dim3(256), 0, x.s, ranges, P.tiles,
                            (LongTiles*)(stats + kStatLong), b.keys[0].as<uint32_t>());
         HIP_TRY(hipGetLastError());
     }

@@ -184,8 +184,8 @@ def test_image_layout_closed_form():
 
 @pytest.mark.parametrize("maxv", [255, 65535, 16777215])
 def test_unorm_double_multiply_identity(maxv):
-    """The device reads UNORM codes as (float)((double)u * (1.0 / max)); that
-    equals the reference's fp32 division u / (float)max for every code."""
+    """(float)((double)u * (1.0 / max)) equals the reference's fp32 division
+    u / (float)max for every code (the device's form of it: test_unorm_forms)."""
     u = np.arange(maxv + 1, dtype=np.uint64)
     a = u.astype(np.float32) / np.float32(maxv)
     b = (u.astype(np.float64) * (1.0 / maxv)).astype(np.float32)

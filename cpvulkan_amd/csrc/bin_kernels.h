@@ -456,9 +456,13 @@ __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* s
 constexpr int kScanThreads = 256;
 constexpr int kScanItems = 16;
 
-// A tile may be long (LongTiles, below) from this many pairs on and from this
-// share of the launch's, about its even share among the resident waves.
-constexpr uint32_t kLongPairs = 256u, kLongShare = 4096u;
+// A tile may be long (LongTiles) from this many pairs on and from this share of
+// the launch's, about its even share among the resident waves.  With 16x16
+// tiles and one wave a batch of 48 jobs took 1,776 us a submit from 256 pairs
+// on, 1,771 from 128, 1,780 from 64 and 2,238 from 32, another 2,374 from 1/8192
+// of the pairs and 2,475 from 1/4096 (a clustered soup, the other way, 1,942 and
+// 1,807, with 4,096 workgroups).
+constexpr uint32_t kLongPairs = 256u, kLongShare = 8192u;
 
 struct ScanArgs {
     uint64_t* sums;          // in: pairs of each setup workgroup; out: their exclusive scan

@@ -473,12 +473,12 @@ int enqueue_front(Exec& x, const LaunchPlan& P, uint8_t* arena, uint32_t pair_ca
     return CPV_OK;
 }
 
-// Workgroups that raster the split tiles' blocks, at most; a multiple of
-// kRasterQueues.  With 16x16 tiles and one wave, the clustered 1M soup took
-// 2,308 us a frame with 2,048, 1,944 with 4,096 and 1,830 with 8,192; a launch
-// that splits nothing pays for their dispatch (150k triangles at 1080p: 393
-// with 2,048, 405 with 8,192).
-constexpr uint32_t kLongGroups = 4096u;
+// Workgroups that raster the split tiles' blocks, at most: eight for each of
+// the CUs, a multiple of kRasterQueues.  With 16x16 tiles and one wave, 100k
+// triangles at 640x480 took 329 us a frame with 2,048 and 363 with 4,096, 150k
+// at 1080p, which splits next to nothing, 397 and 408, and the clustered 1M soup
+// 2,260 and 1,942.
+constexpr uint32_t kLongGroups = 2048u;
 
 // The launch splits its long tiles: waves that hold kSplitBlocks or more, a
 // workgroup per tile (the counter-ordered queue balances by itself), and no

@@ -73,14 +73,14 @@ CPV_INDEX int32_t wrap_coord(int32_t v, int32_t size, int32_t mode)
 // (none beyond twice the mean of the tiles that have any) a launch of enough
 // waves to fill the chip (kEvenWaves, one and a half for each SIMD) splits
 // none, and one of fewer waves every tile that is long at all.
-// us a frame, all split against none, for the soups of about 37 triangles a
-// 16x16 tile: one wave for 16x16 tiles 371 against 386 with 1,200 waves
-// (640x480), 615 against 481 with 3,600 (1280x720); one wave for 32x32 tiles
-// 574 against 1,771 with 300 waves, 1,363 against 1,861 with 920, 3,897
-// against 2,862 with 2,040 (1920x1080); four waves for 32x32 tiles 277 against
-// 472 with 1,200, 1,498 against 1,465 with 8,160.  Clustered soups, whose lists
-// differ: 1M triangles at 1080p 1,775 against 4,189 (16x16, one wave) and 4,176
-// against 17,331 (32x32, one wave).
+// us a frame, all split against none, for soups of 80 to 120 triangles a 16x16
+// tile: one wave for 16x16 tiles 329 against 385 with 1,200 waves (640x480),
+// 727 against 478 with 3,600 (1280x720); one wave for 32x32 tiles 631 against
+// 1,806 with 300 waves, 1,485 against 1,923 with 920, 4,160 against 2,869 with
+// 2,040 (1920x1080); four waves for 32x32 tiles 276 against 471 with 1,200,
+// 1,598 against 1,460 with 8,160.  Clustered soups, whose lists differ: 1M
+// triangles at 1080p 2,260 against 4,189 (16x16, one wave) and 4,836 against
+// 17,331 (32x32, one wave).
 constexpr uint32_t kEvenWaves = 1536u;
 CPV_INDEX bool splits_tile(const LongTiles& l, uint32_t n, uint32_t waves)
 {

@@ -86,7 +86,7 @@ def test_which_tiles_are_split(tmp_path):
         for filled, alike in ((1, 1), (300, 1), (1535 // waves, 1), (1536 // waves, 0), (8160, 0), (1 << 22, 0)):
             n = 500
             pairs = n * filled
-            at = max(256, pairs // 4096)
+            at = max(256, pairs // 8192)
             assert splits(u(at), u(filled), u(pairs), u(max(n, at)), u(waves)) == (alike or at >= 2 * n), (waves, filled)
             assert not splits(u(at), u(filled), u(pairs), u(at - 1), u(waves))
         # one tile in ten holds nine tenths of the pairs

@@ -1,5 +1,6 @@
-"""A translated SPIR-V program compiles with every hiprtc that a process may have loaded: the toolkit's and, once torch is
-imported, the one its wheel brings, which may be older.  One raster kernel and the vertex kernel, no GPU."""
+"""A translated SPIR-V program compiles with the hiprtc that torch's wheel brings, which a process that has imported torch
+has loaded and which may be older than the toolkit's (with that one the build compiles programs).  One raster kernel and
+the vertex kernel, no GPU."""
 import subprocess
 import sys
 from pathlib import Path
@@ -32,19 +33,11 @@ assert rc == 0, log.value.decode()[:2000]
 """
 
 
-def _libraries():
-    found = [p for p in (Path("/opt/rocm/lib/libhiprtc.so"),) if p.exists()]
-    try:
-        import torch
-        p = Path(torch.__file__).parent / "lib" / "libhiprtc.so"
-        found += [p] if p.exists() else []
-    except ImportError:
-        pass
-    return found
-
-
-@pytest.mark.parametrize("lib", _libraries(), ids=lambda p: "torch" if "torch" in p.parts else "toolkit")
-def test_program_compiles(lib):
-    # a process for each: a loaded hiprtc stays loaded
+def test_program_compiles_with_the_wheels_hiprtc():
+    torch = pytest.importorskip("torch")
+    lib = Path(torch.__file__).parent / "lib" / "libhiprtc.so"
+    if not lib.exists():
+        pytest.skip("this torch brings no hiprtc")
+    # a process of its own: a loaded hiprtc stays loaded
     r = subprocess.run([sys.executable, "-c", CODE.format(root=str(ROOT), lib=str(lib))], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, r.stdout + r.stderr
